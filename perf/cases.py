@@ -219,7 +219,7 @@ class Handle:
         self.h = h
 
     def __del__(self):
-        if getattr(self, "h", None):
+        if getattr(self, "h", None) and lib is not None:  # (None while the interpreter ends)
             lib().olv_graph_destroy(self.h)
             self.h = None
 
