@@ -1,332 +1,496 @@
-// Host construction of the source-segmented pull plan (blocked.hpp).
+// Device construction of the source-segmented pull plan (blocked.hpp).
+//
+// The entries are sorted by the segment of their source (one or two radix
+// passes; rows stay ascending inside a segment), cut into pieces, and the
+// pieces are sorted twice: by row, which gives the combine its term lists,
+// and by (segment, class), which gives the segment pass its layout.  Only
+// the per-segment and per-(segment, class) counts come to the host, which
+// deals the tasks out to the workgroups.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstring>
-#include <thread>
 #include <vector>
 
 #include "blocked.hpp"
+#include "radix.hpp"
 
 namespace olv {
 
 namespace {
 
-// Host threads for a pass over `work` items: one per 2^20 items, at most 16
-// and at most the machine's.
-unsigned host_threads(size_t work) {
-  const unsigned hc = std::max(1u, std::thread::hardware_concurrency());
-  return (unsigned)std::min<size_t>({(size_t)16, (size_t)hc, work / (1u << 20) + 1});
+unsigned pgrid(size_t items) {
+  const size_t b = (items + 255) / 256;
+  return (unsigned)std::max<size_t>(1, std::min(b, (size_t)cu_count() * 16));
 }
 
-// f(t) for t < T, on T - 1 new host threads and the caller (t = 0); a thread
-// that cannot be started runs its share on the caller.
-template <class F>
-void host_parallel(unsigned T, const F &f) {
-  std::vector<std::thread> th;
-  th.reserve(T);
-  for (unsigned t = 1; t < T; ++t) {
-    try {
-      th.emplace_back(f, t);
-    } catch (...) {
-      f(t);
+constexpr uint32_t kDirectKeyBits = 4;  // class field of a piece's layout key
+
+// Device binary search: first i in [0, m) with a[i] >= key (a ascending in
+// `at`), m if none.
+template <class At>
+__device__ __forceinline__ uint32_t first_ge(uint32_t m, uint32_t key, At at) {
+  uint32_t lo = 0, hi = m;
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo) / 2;
+    if (at(mid) < key) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ uint32_t row_of(const uint32_t *v, uint32_t i) { return v[i]; }
+__device__ __forceinline__ uint32_t row_of(const uint2 *v, uint32_t i) { return v[i].x; }
+__device__ __forceinline__ uint32_t slot_of(const uint32_t *, uint32_t) { return 0u; }
+__device__ __forceinline__ uint32_t slot_of(const uint2 *v, uint32_t i) { return v[i].y; }
+
+// flag[i] = 1 where entry i (sorted by segment, then row) starts a new
+// (segment, row).
+template <class V>
+__global__ void piece_head_kernel(const uint32_t *__restrict__ key, const V *__restrict__ val, uint32_t m,
+                                  uint32_t *__restrict__ flag) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (size_t)gridDim.x * blockDim.x)
+    flag[i] = i == 0 || (key[i - 1] >> kSegBits) != (key[i] >> kSegBits) ||
+              row_of(val, (uint32_t)i - 1) != row_of(val, (uint32_t)i);
+}
+
+// Cuts inside the (segment, row) groups that start at the flags of `scan`:
+// every kPieceMax entries, and the tail at half its capacity when it would
+// leave a quarter or more of that unused.
+__global__ void piece_cut_kernel(const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
+                                 uint32_t *__restrict__ flag) {
+  const uint32_t groups = *count;
+  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < groups; p += gridDim.x * blockDim.x) {
+    uint32_t a = start[p];
+    const uint32_t end = start[p + 1];
+    for (; end - a > kPieceMax; a += kPieceMax) flag[a + kPieceMax] = 1u;
+    const uint32_t len = end - a;
+    if (len <= kCutCap / 2) continue;
+    const uint32_t cap = 1u << (32 - __clz(len - 1));
+    if (len <= cap / 4 * 3) flag[a + cap / 2] = 1u;
+  }
+}
+
+// out[0] = pieces, out[1] = rows up to the last one with entries, out[2 + s]
+// = entries of segment s.
+__global__ void seg_stat_kernel(const uint32_t *__restrict__ key, const uint32_t *__restrict__ scan, uint32_t m,
+                                const uint32_t *__restrict__ rp, uint32_t n, uint32_t nseg,
+                                uint32_t *__restrict__ out) {
+  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < nseg; s += gridDim.x * blockDim.x) {
+    const uint32_t a = first_ge(m, s, [&](uint32_t i) { return key[i] >> kSegBits; });
+    const uint32_t b = first_ge(m, s + 1, [&](uint32_t i) { return key[i] >> kSegBits; });
+    out[2 + s] = b - a;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    out[0] = scan[m];
+    out[1] = first_ge(n, m, [&](uint32_t v) { return rp[v]; });
+  }
+}
+
+__global__ void live_rows_kernel(const uint32_t *__restrict__ rp, uint32_t n, uint32_t m, uint32_t *__restrict__ out) {
+  out[0] = first_ge(n, m, [&](uint32_t v) { return rp[v]; });
+}
+
+// pstart[p] = first entry of piece p (a flag of the scan); pstart[pieces] = m.
+__global__ void piece_start_kernel(const uint32_t *__restrict__ scan, uint32_t m, uint32_t *__restrict__ pstart) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (size_t)gridDim.x * blockDim.x) {
+    const uint32_t p = scan[i];
+    if (scan[i + 1] != p) pstart[p] = (uint32_t)i;
+    if (i + 1 == m) pstart[scan[m]] = m;
+  }
+}
+
+template <class V>
+__global__ void piece_row_kernel(const V *__restrict__ val, const uint32_t *__restrict__ pstart, uint32_t pieces,
+                                 uint32_t *__restrict__ prow) {
+  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < pieces; p += gridDim.x * blockDim.x)
+    prow[p] = row_of(val, pstart[p]);
+}
+
+// The layout key of every piece: (segment, class), or nseg << 4 for a piece
+// whose entries the combine reads directly.
+__global__ void piece_key_kernel(const uint32_t *__restrict__ key, const uint32_t *__restrict__ pstart,
+                                 uint32_t pieces, const uint32_t *__restrict__ entries, uint32_t nseg, uint32_t *__restrict__ lkey) {
+  for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < pieces; p += gridDim.x * blockDim.x) {
+    const uint32_t a = pstart[p], len = pstart[p + 1] - a, s = key[a] >> kSegBits;
+    uint32_t k = nseg << kDirectKeyBits;
+    if (entries[s] >= kSegMinEntries) k = (s << kDirectKeyBits) | (len <= 1 ? 0u : 32u - __clz(len - 1));
+    lkey[p] = k;
+  }
+}
+
+// terms[j] = combine terms of the j-th piece in row order.
+__global__ void piece_terms_kernel(const uint32_t *__restrict__ by_row, const uint32_t *__restrict__ pstart,
+                                   const uint32_t *__restrict__ lkey, uint32_t pieces, uint32_t nseg,
+                                   uint32_t *__restrict__ terms) {
+  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < pieces; j += gridDim.x * blockDim.x) {
+    const uint32_t p = by_row[j];
+    terms[j] = lkey[p] == nseg << kDirectKeyBits ? pstart[p + 1] - pstart[p] : 1u;
+  }
+}
+
+// cofs[p] = the piece's first combine term; cmb_rp[v] = row v's first term.
+__global__ void combine_rows_kernel(const uint32_t *__restrict__ by_row, const uint32_t *__restrict__ row_sorted,
+                                    const uint32_t *__restrict__ term_scan, uint32_t pieces, uint32_t n,
+                                    uint32_t *__restrict__ cofs, uint32_t *__restrict__ cmb_rp) {
+  const uint32_t stride = gridDim.x * blockDim.x, t = blockIdx.x * blockDim.x + threadIdx.x;
+  for (uint32_t j = t; j < pieces; j += stride) cofs[by_row[j]] = term_scan[j];
+  for (size_t v = t; v <= n; v += stride)
+    cmb_rp[v] = term_scan[first_ge(pieces, (uint32_t)v, [&](uint32_t i) { return row_sorted[i]; })];
+}
+
+__device__ __forceinline__ uint32_t tier_of(uint32_t terms) {
+  return terms > kCmbBig ? 3u : (terms > kCmbMid ? 2u : (terms > kCmbLight ? 1u : 0u));
+}
+
+__global__ void tier_kernel(const uint32_t *__restrict__ cmb_rp, uint32_t n, uint32_t *__restrict__ tier) {
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+    tier[v] = tier_of(cmb_rp[v + 1] - cmb_rp[v]);
+}
+
+// out[g] = first position of key g in the sorted keys, g < count.
+__global__ void group_start_kernel(const uint32_t *__restrict__ sorted, uint32_t items, uint32_t count,
+                                   uint32_t *__restrict__ out) {
+  for (uint32_t g = blockIdx.x * blockDim.x + threadIdx.x; g < count; g += gridDim.x * blockDim.x)
+    out[g] = first_ge(items, g, [&](uint32_t i) { return sorted[i]; });
+}
+
+// The j-th piece in layout order: its partial or direct terms go to the
+// combine list, epos[p] = its first entry's position (~0: direct).
+template <class V>
+__global__ void piece_place_kernel(const uint32_t *__restrict__ by_key, const uint32_t *__restrict__ key_sorted,
+                                   const uint32_t *__restrict__ gstart, const uint32_t *__restrict__ gtask,
+                                   const uint32_t *__restrict__ gpart, const uint32_t *__restrict__ pstart,
+                                   const uint32_t *__restrict__ cofs, const uint32_t *__restrict__ key,
+                                   const V *__restrict__ val, const uint32_t *__restrict__ eid, uint32_t pieces,
+                                   uint32_t nseg, uint32_t *__restrict__ cmb_pos, uint32_t *__restrict__ wcmb_eid,
+                                   size_t *__restrict__ epos) {
+  for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < pieces; j += gridDim.x * blockDim.x) {
+    const uint32_t p = by_key[j], g = key_sorted[j], c = cofs[p];
+    if (g == nseg << kDirectKeyBits) {
+      const uint32_t a = pstart[p], len = pstart[p + 1] - a;
+      for (uint32_t e = 0; e < len; ++e) {
+        cmb_pos[c + e] = key[a + e];
+        if (wcmb_eid) wcmb_eid[c + e] = eid[slot_of(val, a + e)];
+      }
+      epos[p] = ~(size_t)0;
+    } else {
+      const uint32_t r = j - gstart[g], cls = g & ((1u << kDirectKeyBits) - 1);
+      cmb_pos[c] = kIsPartial | (gpart[g] + r);
+      if (wcmb_eid) wcmb_eid[c] = kEidOne;
+      epos[p] = (size_t)gtask[g] * kTask + (r << cls);
     }
   }
-  f(0);
-  for (auto &x : th) x.join();
 }
 
-template <class T>
-int upload_vec(T **dst, const std::vector<T> &src) {
-  const size_t bytes = std::max<size_t>(src.size(), 1) * sizeof(T);
-  OLV_HIP(hipMalloc(reinterpret_cast<void **>(dst), bytes));
-  if (!src.empty()) OLV_HIP(hipMemcpy(*dst, src.data(), src.size() * sizeof(T), hipMemcpyHostToDevice));
+// Every entry of a staged piece into its place.
+template <class V>
+__global__ void entry_place_kernel(const uint32_t *__restrict__ key, const V *__restrict__ val,
+                                   const uint32_t *__restrict__ scan, uint32_t m, const uint32_t *__restrict__ pstart,
+                                   const size_t *__restrict__ epos, const uint32_t *__restrict__ eid,
+                                   uint16_t *__restrict__ lidx, uint32_t *__restrict__ went_eid) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (size_t)gridDim.x * blockDim.x) {
+    const uint32_t p = scan[i + 1] - 1;
+    const size_t ep = epos[p];
+    if (ep == ~(size_t)0) continue;
+    const size_t pos = ep + ((uint32_t)i - pstart[p]);
+    lidx[pos] = (uint16_t)(key[i] & (kSegSize - 1));
+    if (went_eid) went_eid[pos / kTask * kTask + wpos((uint32_t)(pos % kTask))] = eid[slot_of(val, (uint32_t)i)];
+  }
+}
+
+// Descriptors of the tasks of every (segment, class) group; one workgroup a
+// group.
+__global__ void task_desc_kernel(const uint32_t *__restrict__ gtask, const uint32_t *__restrict__ gpart,
+                                 uint2 *__restrict__ desc) {
+  const uint32_t g = blockIdx.x, cls = g & ((1u << kDirectKeyBits) - 1);
+  const uint32_t a = gtask[g], b = gtask[g + 1];
+  for (uint32_t t = a + threadIdx.x; t < b; t += blockDim.x) desc[t] = make_uint2(cls, gpart[g] + (t - a) * (kTask >> cls));
+}
+
+// Time of a task by class and of a segment's slice, in 1/16 of a middling
+// task, fitted to per-workgroup clocks of RMAT-20 passes.
+constexpr uint32_t kSliceCost = 800;
+inline uint32_t task_cost(uint32_t g) {
+  constexpr uint32_t kCost[1u << kDirectKeyBits] = {22, 17, 16, 16, 16, 16, 16, 18, 18, 18};
+  return kCost[g & ((1u << kDirectKeyBits) - 1)];
+}
+
+// Device memory in one block, cut into 256-byte aligned arrays.
+struct Arena {
+  size_t size = 0;
+  size_t take(size_t bytes) {
+    const size_t at = size;
+    size += (bytes + 255) / 256 * 256;
+    return at;
+  }
+};
+
+int to_host(void *h, const void *d, size_t bytes) {
+  OLV_HIP(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, stream()));
+  OLV_HIP(hipStreamSynchronize(stream()));
   return OLV_OK;
 }
 
-// Lanes and reads per piece by length: one lane with 2, 4 or 8 reads up to
-// 2, 4, 8 entries, then 8 reads on 2, 4, ..., 32 lanes up to 16, 32, ...,
-// 256 entries, and a wave up to kPieceMax.
-constexpr uint32_t kBucketLanes[9] = {1, 1, 1, 2, 4, 8, 16, 32, 64};
-constexpr uint32_t kBucketReads[9] = {2, 4, 8, 8, 8, 8, 8, 8, 8};
-constexpr int kBuckets = 9;
-static_assert(kBuckets <= (1 << kBucketBits), "a unit's bucket fits its descriptor");
-static_assert(kPieceMax <= kBucketReads[kBuckets - 1] * kBucketLanes[kBuckets - 1], "the widest bucket covers a piece");
-// the first bucket whose lanes and reads cover the piece (the segment pass
-// sums every piece in one step): the fewest reads for short pieces, then the
-// fewest lanes
-inline uint32_t piece_bucket(uint32_t len) {
-  uint32_t b = 0;
-  while (b + 1 < kBuckets && len > kBucketReads[b] * kBucketLanes[b]) ++b;
-  return b;
+// Rows by tier (bp.cmb_rp built): the mid, big and huge rows, each ascending,
+// into `rows` (n words at least); counts to the host.
+int list_tiers(BlockedPlan &bp, uint32_t *rows) {
+  ScratchBuf tier, start;
+  OLV_TRY(tier.alloc((size_t)bp.n * 4));
+  OLV_TRY(start.alloc(5 * 4));
+  hipLaunchKernelGGL(tier_kernel, dim3(pgrid(bp.n)), dim3(256), 0, stream(), bp.cmb_rp, bp.n, tier.as<uint32_t>());
+  SortBufs b;
+  OLV_TRY(radix_sort<uint32_t>(tier.as<uint32_t>(), LoadIndex{}, bp.n, 2, b));
+  hipLaunchKernelGGL(group_start_kernel, dim3(1), dim3(64), 0, stream(), b.keys(), bp.n, 5u, start.as<uint32_t>());
+  OLV_HIP(hipGetLastError());
+  uint32_t h[5];
+  OLV_TRY(to_host(h, start.p, sizeof(h)));
+  bp.n_mid = h[2] - h[1];
+  bp.n_big = h[3] - h[2];
+  bp.n_huge = h[4] - h[3];
+  if (h[4] > h[1])
+    OLV_HIP(hipMemcpyAsync(rows, b.vals<uint32_t>() + h[1], (size_t)(h[4] - h[1]) * 4, hipMemcpyDeviceToDevice, stream()));
+  bp.cmb_rows = rows;
+  return OLV_OK;
+}
+
+// No segment pass: the rows' entries are the combine's terms.
+int build_solo(const uint32_t *rp, const uint32_t *col, const uint32_t *eid, BlockedPlan &bp) {
+  const uint32_t n = bp.n, m = bp.m;
+  Arena ar;
+  const size_t o_rp = ar.take(((size_t)n + 1) * 4), o_pos = ar.take((size_t)m * 4),
+               o_rows = ar.take((size_t)n * 4), o_w = ar.take(eid ? (size_t)m * 4 : 0);
+  OLV_HIP(hipMalloc(&bp.mem, std::max<size_t>(ar.size, 256)));
+  char *base = static_cast<char *>(bp.mem);
+  bp.cmb_rp = reinterpret_cast<uint32_t *>(base + o_rp);
+  bp.cmb_pos = reinterpret_cast<uint32_t *>(base + o_pos);
+  OLV_HIP(hipMemcpyAsync(bp.cmb_rp, rp, ((size_t)n + 1) * 4, hipMemcpyDeviceToDevice, stream()));
+  if (m) OLV_HIP(hipMemcpyAsync(bp.cmb_pos, col, (size_t)m * 4, hipMemcpyDeviceToDevice, stream()));
+  if (eid) {
+    bp.weid = reinterpret_cast<uint32_t *>(base + o_w);
+    if (m) OLV_HIP(hipMemcpyAsync(bp.weid, eid, (size_t)m * 4, hipMemcpyDeviceToDevice, stream()));
+  }
+  bp.ncmb = m;
+  bp.nweights = eid ? m : 0;
+  return list_tiers(bp, reinterpret_cast<uint32_t *>(base + o_rows));
+}
+
+template <class V>
+int build_segmented(const uint32_t *rp, const uint32_t *col, const uint32_t *eid, uint32_t groups, BlockedPlan &bp) {
+  const uint32_t n = bp.n, m = bp.m;
+  const uint32_t nseg = ((n - 1) >> kSegBits) + 1;
+  hipStream_t s = stream();
+  // 1. entries by segment, rows ascending inside
+  SortBufs ent;
+  {
+    ScratchBuf erow;
+    OLV_TRY(erow.alloc((size_t)m * 4));
+    OLV_TRY(slot_rows(rp, n, m, erow.as<uint32_t>()));
+    if constexpr (sizeof(V) == 8) OLV_TRY((radix_sort<V>(col, LoadAndIndex{erow.as<uint32_t>()}, m, bits_for(nseg), ent, kSegBits)));
+    else OLV_TRY((radix_sort<V>(col, LoadArr{erow.as<uint32_t>()}, m, bits_for(nseg), ent, kSegBits)));
+  }
+  const uint32_t *key = ent.keys();
+  const V *val = ent.vals<V>();
+  // 2. pieces
+  ScratchBuf scan, stat;
+  OLV_TRY(scan.alloc(((size_t)m + 1) * 4));
+  OLV_TRY(stat.alloc(((size_t)nseg + 2) * 4));
+  {
+    ScratchBuf flag, gstart;
+    OLV_TRY(flag.alloc((size_t)m * 4));
+    OLV_TRY(gstart.alloc(((size_t)m + 1) * 4));
+    hipLaunchKernelGGL(piece_head_kernel<V>, dim3(pgrid(m)), dim3(256), 0, s, key, val, m, flag.as<uint32_t>());
+    OLV_TRY(exclusive_scan(flag.as<uint32_t>(), scan.as<uint32_t>(), m));
+    hipLaunchKernelGGL(piece_start_kernel, dim3(pgrid(m)), dim3(256), 0, s, scan.as<uint32_t>(), m,
+                       gstart.as<uint32_t>());
+    hipLaunchKernelGGL(piece_cut_kernel, dim3(pgrid(m)), dim3(256), 0, s, gstart.as<uint32_t>(),
+                       scan.as<uint32_t>() + m, flag.as<uint32_t>());
+    OLV_TRY(exclusive_scan(flag.as<uint32_t>(), scan.as<uint32_t>(), m));
+  }
+  hipLaunchKernelGGL(seg_stat_kernel, dim3(pgrid(nseg)), dim3(256), 0, s, key, scan.as<uint32_t>(), m, rp, n, nseg,
+                     stat.as<uint32_t>());
+  OLV_HIP(hipGetLastError());
+  std::vector<uint32_t> h_stat((size_t)nseg + 2);
+  OLV_TRY(to_host(h_stat.data(), stat.p, h_stat.size() * 4));
+  const uint32_t pieces = h_stat[0];
+  bp.n_live = h_stat[1];
+  // 3. the combine's term lists: pieces by row
+  ScratchBuf pbuf;
+  Arena pa;
+  const size_t pw = ((size_t)pieces + 1) * 4;
+  const size_t o_start = pa.take(pw), o_row = pa.take(pw), o_key = pa.take(pw), o_terms = pa.take(pw),
+               o_cofs = pa.take(pw), o_epos = pa.take(2 * pw);
+  OLV_TRY(pbuf.alloc(pa.size));
+  auto parr = [&](size_t o) { return reinterpret_cast<uint32_t *>(pbuf.as<char>() + o); };
+  uint32_t *pstart = parr(o_start), *prow = parr(o_row), *lkey = parr(o_key), *terms = parr(o_terms),
+           *cofs = parr(o_cofs);
+  size_t *epos = reinterpret_cast<size_t *>(parr(o_epos));
+  hipLaunchKernelGGL(piece_start_kernel, dim3(pgrid(m)), dim3(256), 0, s, scan.as<uint32_t>(), m, pstart);
+  hipLaunchKernelGGL(piece_row_kernel<V>, dim3(pgrid(pieces)), dim3(256), 0, s, val, pstart, pieces, prow);
+  hipLaunchKernelGGL(piece_key_kernel, dim3(pgrid(pieces)), dim3(256), 0, s, key, pstart, pieces,
+                     stat.as<uint32_t>() + 2, nseg, lkey);
+  OLV_HIP(hipGetLastError());
+  ScratchBuf crp;
+  OLV_TRY(crp.alloc(((size_t)n + 1) * 4));
+  {
+    SortBufs by;
+    OLV_TRY(radix_sort<uint32_t>(prow, LoadIndex{}, pieces, bits_for(n), by));
+    hipLaunchKernelGGL(piece_terms_kernel, dim3(pgrid(pieces)), dim3(256), 0, s, by.vals<uint32_t>(), pstart, lkey,
+                       pieces, nseg, terms);
+    OLV_TRY(exclusive_scan(terms, terms, pieces));
+    hipLaunchKernelGGL(combine_rows_kernel, dim3(pgrid(std::max(n, pieces))), dim3(256), 0, s, by.vals<uint32_t>(),
+                       by.keys(), terms, pieces, n, cofs, crp.as<uint32_t>());
+    OLV_HIP(hipGetLastError());
+  }
+  // 4. the segment pass's layout: pieces by (segment, class)
+  const uint32_t ngr = nseg << kDirectKeyBits;  // groups; key ngr: direct pieces
+  SortBufs by;
+  OLV_TRY(radix_sort<uint32_t>(lkey, LoadIndex{}, pieces, bits_for(ngr + 1), by));
+  ScratchBuf gbuf;  // gstart (ngr + 2, the last the terms in all), gtask (ngr + 1), gpart (ngr + 1)
+  OLV_TRY(gbuf.alloc(((size_t)ngr * 3 + 4) * 4));
+  uint32_t *gstart = gbuf.as<uint32_t>(), *gtask = gstart + ngr + 2, *gpart = gtask + ngr + 1;
+  hipLaunchKernelGGL(group_start_kernel, dim3(pgrid(ngr + 1)), dim3(256), 0, s, by.keys(), pieces, ngr + 1, gstart);
+  OLV_HIP(hipGetLastError());
+  OLV_HIP(hipMemcpyAsync(gstart + ngr + 1, terms + pieces, 4, hipMemcpyDeviceToDevice, s));
+  std::vector<uint32_t> hg((size_t)ngr + 2), ht((size_t)ngr * 2 + 2);
+  OLV_TRY(to_host(hg.data(), gstart, hg.size() * 4));
+  bp.ncmb = hg[ngr + 1];
+  uint64_t task = 0, part = 0;
+  for (uint32_t g = 0; g < ngr; ++g) {
+    const uint32_t cls = g & ((1u << kDirectKeyBits) - 1);
+    if (cls == 0) part = (part + kTask - 1) / kTask * kTask;  // 16-byte stores in the first classes
+    ht[g] = (uint32_t)task;
+    ht[ngr + 1 + g] = (uint32_t)part;
+    if (cls >= kClasses) continue;
+    const uint64_t ppt = kTask >> cls, nt = (hg[g + 1] - hg[g] + ppt - 1) / ppt;
+    task += nt;
+    part += nt * ppt;
+  }
+  ht[ngr] = (uint32_t)task;
+  ht[2 * (size_t)ngr + 1] = (uint32_t)part;
+  if (part >= kIsPartial) return build_solo(rp, col, eid, bp);  // beyond a term's 31 bits
+  bp.ntasks = (uint32_t)task;
+  bp.nparts = (uint32_t)part;
+  // Tasks to workgroups: consecutive runs of about equal cost, a task
+  // kTaskCost (classes of short pieces store more) and a segment's slice
+  // kSliceCost (its 128 KB load between two barriers, and the ring's restart).
+  std::vector<uint4> first, items;
+  {
+    uint64_t total = 0;
+    for (uint32_t g = 0; g < ngr; ++g) total += (uint64_t)(ht[g + 1] - ht[g]) * task_cost(g);
+    for (uint32_t g = 0; g < nseg; ++g)
+      total += ht[(g + 1) << kDirectKeyBits] > ht[g << kDirectKeyBits] ? kSliceCost : 0;
+    uint64_t share = std::max<uint64_t>((total + (uint64_t)kSliceCost * groups + groups - 1) / groups,
+                                        kSliceCost + kBlkWaves * task_cost(kClasses - 1));
+    for (;; share += share / 64 + 1) {  // until no more than `groups` workgroups come out
+      first.clear();
+      items.clear();
+      uint64_t room = 0;                // what the current workgroup may still take
+      uint32_t cur = 0xffffffffu;       // its current item's segment
+      for (uint32_t g = 0; g < ngr; ++g) {
+        const uint32_t sg = g >> kDirectKeyBits, c = task_cost(g);
+        for (uint32_t t = ht[g]; t < ht[g + 1];) {
+          if (first.empty() || room < (cur == sg ? 0u : kSliceCost) + kBlkWaves * c / 2 ||
+              (first.back().w & 0xfffu) == 0xfffu) {
+            first.push_back(make_uint4(0, 0, 0, (uint32_t)items.size() << 12));
+            room = share;
+            cur = 0xffffffffu;
+          }
+          uint4 &f = first.back();
+          const bool add = cur != sg;
+          if (add) {
+            room -= kSliceCost;
+            cur = sg;
+            if (f.w & 0xfffu) items.push_back(make_uint4(sg, t, t, 0));
+            else f = make_uint4(sg, t, t, f.w);
+            ++f.w;
+          }
+          const uint32_t take = (uint32_t)std::min<uint64_t>(ht[g + 1] - t, std::max<uint64_t>(1, room / c));
+          t += take;
+          ((f.w & 0xfffu) == 1 ? f : items.back()).z = t;
+          room -= std::min<uint64_t>(room, (uint64_t)take * c);
+        }
+      }
+      if (first.size() <= groups || nseg > (uint64_t)groups * 4000) break;
+    }
+    // Workgroup b runs on XCD b % kXcds: neighbours in the list, which share a
+    // slice, go to one XCD and load it through one L2.
+    constexpr size_t kXcds = 8;
+    const size_t per = (first.size() + kXcds - 1) / kXcds;
+    std::vector<uint4> order(per * kXcds, make_uint4(0, 0, 0, 0));
+    for (size_t b = 0; b < order.size(); ++b) {
+      const size_t l = b % kXcds * per + b / kXcds;
+      if (l < first.size()) order[b] = first[l];
+    }
+    first.swap(order);
+    if (items.size() >= (1u << 20)) return fail(OLV_ERANGE, "pull plan: %zu segment items", items.size());
+  }
+  bp.ngroups = (uint32_t)first.size();  // (some may have no items)
+  // 5. the plan's arrays
+  Arena ar;
+  const size_t o_first = ar.take(first.size() * sizeof(uint4)), o_items = ar.take((items.size() + 1) * sizeof(uint4)),
+               o_desc = ar.take((size_t)task * sizeof(uint2)), o_lidx = ar.take((size_t)task * kTask * 2),
+               o_rp = ar.take(((size_t)n + 1) * 4), o_pos = ar.take((size_t)bp.ncmb * 4),
+               o_rows = ar.take((size_t)n * 4), o_part = ar.take((size_t)part * 4),
+               o_w = ar.take(eid ? ((size_t)task * kTask + bp.ncmb) * 4 : 0);
+  OLV_HIP(hipMalloc(&bp.mem, std::max<size_t>(ar.size, 256)));
+  char *base = static_cast<char *>(bp.mem);
+  bp.wg_first = reinterpret_cast<uint4 *>(base + o_first);
+  bp.wg_items = reinterpret_cast<uint4 *>(base + o_items);
+  bp.desc = reinterpret_cast<uint2 *>(base + o_desc);
+  bp.lidx = reinterpret_cast<uint16_t *>(base + o_lidx);
+  bp.cmb_rp = reinterpret_cast<uint32_t *>(base + o_rp);
+  bp.cmb_pos = reinterpret_cast<uint32_t *>(base + o_pos);
+  bp.partial = reinterpret_cast<float *>(base + o_part);
+  if (eid) {
+    bp.weid = reinterpret_cast<uint32_t *>(base + o_w);
+    bp.nweights = (size_t)task * kTask + bp.ncmb;
+  }
+  OLV_HIP(hipMemcpyAsync(gtask, ht.data(), ht.size() * 4, hipMemcpyHostToDevice, s));
+  if (!first.empty())
+    OLV_HIP(hipMemcpyAsync(bp.wg_first, first.data(), first.size() * sizeof(uint4), hipMemcpyHostToDevice, s));
+  if (!items.empty())
+    OLV_HIP(hipMemcpyAsync(bp.wg_items, items.data(), items.size() * sizeof(uint4), hipMemcpyHostToDevice, s));
+  OLV_HIP(hipMemcpyAsync(bp.cmb_rp, crp.p, ((size_t)n + 1) * 4, hipMemcpyDeviceToDevice, s));
+  OLV_TRY(fill_u32(reinterpret_cast<uint32_t *>(bp.lidx), kSegSize | kSegSize << 16, (size_t)task * kTask / 2));
+  if (eid) OLV_TRY(fill_u32(bp.weid, kEidZero, (size_t)task * kTask));
+  hipLaunchKernelGGL(task_desc_kernel, dim3(ngr), dim3(256), 0, s, gtask, gpart, bp.desc);
+  uint32_t *wcmb_eid = eid ? bp.weid + (size_t)task * kTask : nullptr;
+  hipLaunchKernelGGL(piece_place_kernel<V>, dim3(pgrid(pieces)), dim3(256), 0, s, by.vals<uint32_t>(), by.keys(),
+                     gstart, gtask, gpart, pstart, cofs, key, val, eid, pieces, nseg, bp.cmb_pos, wcmb_eid, epos);
+  hipLaunchKernelGGL(entry_place_kernel<V>, dim3(pgrid(m)), dim3(256), 0, s, key, val, scan.as<uint32_t>(), m, pstart,
+                     epos, eid, bp.lidx, bp.weid);
+  OLV_HIP(hipGetLastError());
+  OLV_TRY(list_tiers(bp, reinterpret_cast<uint32_t *>(base + o_rows)));
+  OLV_HIP(hipStreamSynchronize(s));  // the uploads read this function's vectors
+  return OLV_OK;
 }
 
 }  // namespace
 
-int build_blocked_host(const std::vector<uint32_t> &rp, const uint32_t *col, bool with_slots, uint32_t groups,
-                       uint32_t unit_edges, BlockedHost &h) {
-  if (unit_edges < kPieceMax || unit_edges > kUnitEdges || unit_edges % 8)
-    return fail(OLV_EINTERNAL, "blocked plan: %u entries per unit", unit_edges);
-  const uint32_t n = (uint32_t)(rp.size() - 1);
-  const uint32_t m = rp[n];
-  h.n = n;
-  h.m = m;
-  uint32_t n_live = n;
-  while (n_live > 0 && rp[n_live] == rp[n_live - 1]) --n_live;
-  h.n_live = n_live;
-  const uint32_t nseg = n ? ((n - 1) >> kSegBits) + 1 : 0;
-  h.nseg = nseg;
-
-  // 1. entries stably sorted by the segment of their source: within a
-  //    segment, rows ascending and each row's entries in slot order (a
-  //    counting sort over row ranges on host threads; each entry's slot,
-  //    row and 16-bit offset carried along)
-  std::vector<uint32_t> soff((size_t)nseg + 1, 0);
-  std::vector<uint32_t> perm(m), prow(m);
-  std::vector<uint16_t> loff(m);
-  {
-    const unsigned T = host_threads(m);
-    std::vector<uint32_t> rb(T + 1, n);  // row ranges of about m / T entries
-    for (unsigned t = 0; t < T; ++t)
-      rb[t] = (uint32_t)(std::lower_bound(rp.begin(), rp.end() - 1, (uint32_t)((uint64_t)m * t / T)) - rp.begin());
-    std::vector<uint32_t> cur((size_t)T * nseg, 0);  // per range: counts, then cursors
-    std::vector<uint8_t> bad(T, 0);
-    host_parallel(T, [&](unsigned t) {
-      uint32_t *c = cur.data() + (size_t)t * nseg;
-      for (uint32_t k = rp[rb[t]]; k < rp[rb[t + 1]]; ++k) {
-        if (col[k] >= n) {
-          bad[t] = 1;
-          return;
-        }
-        c[col[k] >> kSegBits]++;
-      }
-    });
-    for (unsigned t = 0; t < T; ++t)
-      if (bad[t]) return fail(OLV_EINTERNAL, "blocked plan: an entry is out of range (n = %u)", n);
-    uint32_t run = 0;
-    for (uint32_t s = 0; s < nseg; ++s) {
-      soff[s] = run;
-      for (unsigned t = 0; t < T; ++t) {
-        const uint32_t x = cur[(size_t)t * nseg + s];
-        cur[(size_t)t * nseg + s] = run;
-        run += x;
-      }
-    }
-    soff[nseg] = run;
-    host_parallel(T, [&](unsigned t) {
-      uint32_t *c = cur.data() + (size_t)t * nseg;
-      for (uint32_t v = rb[t]; v < rb[t + 1]; ++v)
-        for (uint32_t k = rp[v]; k < rp[v + 1]; ++k) {
-          const uint32_t pos = c[col[k] >> kSegBits]++;
-          perm[pos] = k;
-          prow[pos] = v;
-          loff[pos] = (uint16_t)(col[k] & (kSegSize - 1));
-        }
-    });
-  }
-
-  // 2. pieces: runs of one row within a segment, cut at kPieceMax entries;
-  //    slots grouped by row in creation order (segment, then chunk)
-  struct Piece {
-    uint32_t start, len, slot;
-  };
-  std::vector<uint32_t> npc(n, 0);
-  size_t npieces = 0;
-  for (uint32_t s = 0; s < nseg; ++s)
-    for (uint32_t p = soff[s]; p < soff[s + 1];) {
-      uint32_t e = p;
-      while (e < soff[s + 1] && prow[e] == prow[p]) ++e;
-      const uint32_t chunks = (e - p + kPieceMax - 1) / kPieceMax;
-      npc[prow[p]] += chunks;
-      npieces += chunks;
-      p = e;
-    }
-  if (npieces >= 0xffffffffull) return fail(OLV_ERANGE, "blocked plan: %zu pieces", npieces);
-  std::vector<uint32_t> &cmb = h.cmb_rp;
-  cmb.assign((size_t)n + 1, 0);
-  for (uint32_t v = 0; v < n; ++v) cmb[v + 1] = cmb[v] + npc[v];
-  // rows with more partials than one lane combines, listed by tier
-  h.cmb_mid.clear();
-  h.cmb_big.clear();
-  for (uint32_t v = 0; v < n; ++v) {
-    if (npc[v] > kCmbMid) h.cmb_big.push_back(v);
-    else if (npc[v] > kCmbLight) h.cmb_mid.push_back(v);
-  }
-  std::vector<uint32_t> slot_cur(cmb.begin(), cmb.end() - 1);
-  std::vector<Piece> order;  // final piece order: segment, then bucket (longest first), then row
-  order.reserve(npieces);
-  std::vector<uint4> &units = h.units;
-  units.clear();
-  std::vector<double> unit_cost;
-  std::vector<Piece> byb[kBuckets];
-  uint32_t edge_cursor = 0;  // first entry of the next unit
-  for (uint32_t s = 0; s < nseg; ++s) {
-    for (auto &b : byb) b.clear();
-    for (uint32_t p = soff[s]; p < soff[s + 1];) {
-      uint32_t e = p;
-      while (e < soff[s + 1] && prow[e] == prow[p]) ++e;
-      const uint32_t v = prow[p];
-      for (uint32_t c = p; c < e; c += kPieceMax) {
-        const uint32_t len = std::min(kPieceMax, e - c);
-        byb[piece_bucket(len)].push_back(Piece{c, len, slot_cur[v]++});
-      }
-      p = e;
-    }
-    for (int b = kBuckets - 1; b >= 0; --b) {
-      // units of at most unit_edges entries and kUnitPieces pieces over this
-      // (segment, bucket) group
-      size_t i = 0;
-      while (i < byb[b].size()) {
-        const uint32_t first = (uint32_t)order.size();
-        uint32_t edges = 0, pieces = 0;
-        while (i < byb[b].size() &&
-               (pieces == 0 || (pieces < kUnitPieces && edges + byb[b][i].len <= unit_edges))) {
-          edges += byb[b][i].len;
-          ++pieces;
-          order.push_back(byb[b][i++]);
-        }
-        units.push_back(make_uint4(s, (uint32_t)b, first, edge_cursor));
-        for (uint32_t q = first; q < (uint32_t)order.size(); ++q) edge_cursor += order[q].len;
-        // every unit starts on an 8-entry (16-byte) boundary: staged with
-        // 16-byte loads and LDS stores
-        if ((uint64_t)edge_cursor + 7 >= 0xffffffffull) return fail(OLV_ERANGE, "blocked plan: entries overflow");
-        edge_cursor = (edge_cursor + 7) & ~7u;
-        // cost in us, fitted to per-unit timestamps of RMAT-20 iterations
-        // on MI355X: staging and the barriers around it ~1.3, then
-        // kStepUs[b] per step (one piece per group of G lanes) and 0.04 per
-        // thousand entries
-        constexpr double kStepUs[kBuckets] = {0.15, 0.25, 0.41, 0.20, 0.29, 0.37, 0.38, 0.41, 0.37};
-        const uint32_t per_step = kBlkThreads / kBucketLanes[b];
-        const uint32_t steps = (pieces + per_step - 1) / per_step;
-        unit_cost.push_back(1.3 + kStepUs[b] * steps + 4e-5 * edges);
-      }
-    }
-  }
-
-  // 3. entry arrays in piece order, each unit from its (aligned) first
-  //    entry.  The last piece of a unit runs up to the next unit's first
-  //    entry: the gap holds kSegSize, the staged slice's zero slot, as do 8
-  //    spare entries at the end for the staging's 16-byte reads.
-  std::vector<uint32_t> &lslot = h.lslot;
-  std::vector<uint16_t> &pbeg = h.pbeg, &lidx = h.lidx;
-  const uint32_t o = edge_cursor;
-  pbeg.assign(npieces, 0);
-  lidx.assign((size_t)o + 8, (uint16_t)kSegSize);
-  lslot.assign(with_slots ? (size_t)o + 8 : 0, kNoSlot);
-  {
-    const unsigned T = host_threads(o);
-    const size_t nu = units.size();
-    host_parallel(T, [&](unsigned t) {  // units' entries are disjoint
-      for (size_t un = nu * t / T; un < nu * (t + 1) / T; ++un) {
-        const uint32_t e0 = units[un].w;
-        uint32_t e = e0;
-        const uint32_t qe = un + 1 < nu ? units[un + 1].z : (uint32_t)npieces;
-        for (uint32_t q = units[un].z; q < qe; ++q) {
-          const Piece &pc = order[q];
-          pbeg[q] = (uint16_t)(e - e0);
-          std::memcpy(&lidx[e], &loff[pc.start], pc.len * sizeof(uint16_t));
-          if (with_slots) std::memcpy(&lslot[e], &perm[pc.start], pc.len * sizeof(uint32_t));
-          e += pc.len;
-        }
-      }
-    });
-  }
-  // each row's partials in segment order: cmb_pos[cmb_rp[v] + j] is the
-  // piece (and partial) index of the row's j-th piece
-  h.cmb_pos.assign(npieces, 0);
-  {
-    const unsigned T = host_threads(npieces);
-    host_parallel(T, [&](unsigned t) {  // slots are a permutation of the pieces
-      for (size_t q = npieces * t / T; q < npieces * (t + 1) / T; ++q) h.cmb_pos[order[q].slot] = (uint32_t)q;
-    });
-  }
-
-  // 4. units to workgroups: longest first, each to the workgroup where it
-  //    ends earliest, counting a slice load (~1 us) when the workgroup
-  //    has no unit of that segment yet; each workgroup then runs its units
-  //    in segment order.  A sentinel unit closes the list (its first piece
-  //    and entry are the totals).
-  const uint32_t nunits = (uint32_t)units.size();
-  units.push_back(make_uint4(nseg, 0, (uint32_t)npieces, o));
-  const uint32_t ng = std::max<uint32_t>(1, std::min<uint32_t>(groups ? groups : 1, std::max<uint32_t>(nunits, 1)));
-  {
-    std::vector<uint32_t> byc(nunits);
-    for (uint32_t u = 0; u < nunits; ++u) byc[u] = u;
-    std::stable_sort(byc.begin(), byc.end(), [&](uint32_t a, uint32_t b) { return unit_cost[a] > unit_cost[b]; });
-    std::vector<double> load(ng, 0.0);
-    load[0] = 1.5;  // workgroup 0 also applies the stop rule (a residual sum and two barriers)
-    std::vector<std::vector<uint32_t>> mine(ng);
-    std::vector<uint8_t> has((size_t)ng * nseg, 0);  // workgroup w already loads segment s
-    constexpr double kSliceUs = 1.0;
-    for (uint32_t u : byc) {
-      const uint32_t sg = units[u].x;
-      uint32_t best = 0;
-      double bv = 0;
-      for (uint32_t w = 0; w < ng; ++w) {
-        const double v = load[w] + unit_cost[u] + (has[(size_t)w * nseg + sg] ? 0.0 : kSliceUs);
-        if (w == 0 || v < bv) {
-          bv = v;
-          best = w;
-        }
-      }
-      load[best] = bv;
-      has[(size_t)best * nseg + sg] = 1;
-      mine[best].push_back(u);
-    }
-    h.wg_ptr.assign(ng + 1, 0);
-    h.wg_list.clear();
-    h.wg_list.reserve(nunits);
-    for (uint32_t w = 0; w < ng; ++w) {
-      std::sort(mine[w].begin(), mine[w].end());  // unit order = segment order
-      h.wg_ptr[w] = (uint32_t)h.wg_list.size();
-      h.wg_list.insert(h.wg_list.end(), mine[w].begin(), mine[w].end());
-    }
-    h.wg_ptr[ng] = (uint32_t)h.wg_list.size();
-  }
-  static_assert(kUnitPieces < 0x10000 && kUnitEdges < 0x10000, "a unit's counts pack into 16 bits each");
-  h.wg_units.resize(h.wg_list.size());
-  for (size_t i = 0; i < h.wg_list.size(); ++i) {
-    const uint4 a = units[h.wg_list[i]], b = units[h.wg_list[i] + 1];
-    h.wg_units[i] = make_uint4(a.x << kBucketBits | a.y, a.z, a.w, (b.z - a.z) | (b.w - a.w) << 16);
-  }
-  h.wg_first.assign(ng, make_uint4(0, 0, 0, 0));
-  for (uint32_t w = 0; w < ng; ++w)
-    if (h.wg_ptr[w] < h.wg_ptr[w + 1]) h.wg_first[w] = h.wg_units[h.wg_ptr[w]];
-
-  h.npieces = (uint32_t)npieces;
-  h.nent = o + 8;
-  h.nunits = nunits;
-  h.ngroups = ng;
-  return OLV_OK;
-}
-
-int build_blocked_plan(const std::vector<uint32_t> &rp, const uint32_t *col, bool with_slots, uint32_t groups,
-                       uint32_t unit_edges, BlockedPlan &bp) {
+int build_blocked_plan(const uint32_t *rp, const uint32_t *col, const uint32_t *eid, uint32_t n, uint32_t m,
+                       uint32_t max_row, uint32_t groups, BlockedPlan &bp) {
   bp.release();
-  BlockedHost h;
-  OLV_TRY(build_blocked_host(rp, col, with_slots, groups, unit_edges, h));
-  bp.unit_edges = unit_edges;
-  bp.nent = h.nent;
-  bp.n = h.n;
-  bp.m = h.m;
-  bp.n_live = h.n_live;
-  bp.n_mid = (uint32_t)h.cmb_mid.size();
-  bp.n_big = (uint32_t)h.cmb_big.size();
-  bp.nseg = h.nseg;
-  bp.npieces = h.npieces;
-  bp.nunits = h.nunits;
-  bp.ngroups = h.ngroups;
-  OLV_TRY(upload_vec(&bp.wg_ptr, h.wg_ptr));
-  OLV_TRY(upload_vec(&bp.wg_units, h.wg_units));
-  OLV_TRY(upload_vec(&bp.wg_first, h.wg_first));
-  OLV_TRY(upload_vec(&bp.pbeg, h.pbeg));
-  OLV_TRY(upload_vec(&bp.lidx, h.lidx));
-  if (with_slots) OLV_TRY(upload_vec(&bp.lslot, h.lslot));
-  OLV_TRY(upload_vec(&bp.cmb_rp, h.cmb_rp));
-  OLV_TRY(upload_vec(&bp.cmb_pos, h.cmb_pos));
-  OLV_TRY(upload_vec(&bp.cmb_mid, h.cmb_mid));
-  OLV_TRY(upload_vec(&bp.cmb_big, h.cmb_big));
-  OLV_HIP(hipMalloc(reinterpret_cast<void **>(&bp.partial), std::max<size_t>(h.npieces, 1) * sizeof(float)));
+  if (n == 0 || n >= kIsPartial) return fail(OLV_ERANGE, "pull plan: %u vertices", n);
+  bp.n = n;
+  bp.m = m;
+  int rc = OLV_OK;
+  if (m < kPassMinEntries && max_row <= kDirectRowMax) {
+    ScratchBuf w;
+    rc = w.alloc(4);
+    if (rc == OLV_OK) {
+      hipLaunchKernelGGL(live_rows_kernel, dim3(1), dim3(1), 0, stream(), rp, n, m, w.as<uint32_t>());
+      rc = to_host(&bp.n_live, w.p, 4);
+    }
+    if (rc == OLV_OK) rc = build_solo(rp, col, eid, bp);
+  } else if (eid) {
+    rc = build_segmented<uint2>(rp, col, eid, std::max(1u, groups), bp);
+  } else {
+    rc = build_segmented<uint32_t>(rp, col, eid, std::max(1u, groups), bp);
+  }
+  if (rc != OLV_OK) {
+    bp.release();
+    return rc;
+  }
   bp.ready = true;
   return OLV_OK;
 }

@@ -4,34 +4,50 @@
 // per CU).
 //
 // The iterate's source vector is cut into segments of kSegSize consecutive
-// vertices (64 KB of fp32, one LDS slice).  The in-edges of every
+// vertices (128 KB of fp32, one LDS slice).  The in-edges of every
 // destination are grouped by the segment of their source into "pieces"
-// (destination, segment), each piece's entries kept in the row's slot order
-// and stored as 16-bit offsets into its segment; pieces longer than
-// kPieceMax entries are cut into chunks.  One iteration is two launches:
+// (destination, segment) of at most kPieceMax entries.  One iteration is two
+// launches:
 //
-//   segment pass  each workgroup owns a run of work units (a unit: at most
-//                 kUnitPieces pieces and kUnitEdges entries of one segment
-//                 and one length bucket).  Per unit it stages, with
-//                 coalesced loads, the unit's entries and piece offsets in
-//                 LDS (and the segment of the source vector, when the
-//                 segment changes), then sums every piece from LDS alone --
-//                 1 to 64 lanes per piece by length -- and stores one
-//                 partial per piece, in piece order (coalesced stores);
-//   combine       per destination, its partials (listed by cmb_pos in
-//                 segment order) are added in a fixed order -- by one lane
-//                 for up to kCmbLight partials, 8 lanes up to kCmbMid, a
-//                 wave beyond -- and the vertex update runs.
+//   segment pass  sums every piece from the staged slice and stores one
+//                 partial per piece;
+//   combine       adds, per destination, its terms -- partials, in segment
+//                 order -- and applies the vertex update.
 //
-// A piece's terms are summed in a fixed order and the partials in segment
-// order, so an iteration is bit-reproducible from run to run.  With the
-// vertices numbered by descending in-degree (the renumbered CSRs of the
-// PageRank solver) a skewed graph's in-edges fall into few pieces: RMAT-20
-// has 16.8 M in-edges in 2.3 M pieces, most of them in segment 0.  Per
-// iteration the pass reads 2 B per edge and 2 B per piece and writes 4 B per
-// piece, and every gather is an LDS read.
+// A term may also be a single source, read straight from the vector.  That
+// gather is random, so it costs about 2.4 partials (180 against 420 G/s on a
+// uniform graph: the partials of neighbouring rows are neighbours), and it is
+// used only where the pass does not pay: for the entries of a segment too
+// small to be worth a slice (kSegMinEntries), and for a whole CSR of few
+// edges (kPassMinEntries), which then takes one launch per iteration.
+//
+// Layout of the segment pass.  A piece of c entries is padded to a capacity
+// of 1, 2, 4, ..., 512 entries (its class) with the slice's zero slot, and the
+// pieces of one (segment, class) are stored back to back, so a task -- 512
+// consecutive 16-bit entries, 1 KB -- holds 512 pieces of class 0 down to one
+// piece of class 9 and every lane of a wave reads its 8 entries with one
+// 16-byte load.  A lane holds 8 pieces (class 0), 4, 2, one (class 3), or a
+// 2^i-th of one (the group's sum is taken with DPP moves).  All tasks have the
+// same shape, so a wave streams its tasks through a ring of registers kBlkRing
+// deep with no LDS staging and no barrier inside a segment; weighted passes
+// read 8 fp32 weights per lane beside the entries.
+//
+// Pieces of more than kPieceMax entries are cut, and so is the tail of one
+// that would fill at most 3/4 of its capacity (from kCutCap on), at half the
+// capacity: RMAT-20's padding falls from 27 to 10 % for 5 % more partials.
+//
+// What bounds it (RMAT-20, 16.8 M edges, 1.83 M partials): plain, the segment
+// pass takes 14.0 us -- 4 us until the workgroups' first slices are in LDS,
+// then 6-7 us of LDS gathers over 37 MB of entries, the rest launch and
+// imbalance -- and the combine 9.7 us, 4 of them its launch and the others
+// its gathered partials; 24.5 us per iteration against 32.4 when every unit
+// of entries was staged in LDS with 16K-source slices.  Weighted, the pass
+// reads 110 MB in 22 us (28 before) at the rate of the caches behind L2.
+//
+// A piece's terms are summed in a fixed order and the terms of a row in
+// segment order, so an iteration is bit-reproducible from run to run.
 #pragma once
-#include <vector>
+#include <type_traits>
 
 #include "device.hpp"
 #include "internal.hpp"
@@ -39,122 +55,111 @@
 
 namespace olv {
 
-constexpr uint32_t kSegBits = 14;
-constexpr uint32_t kSegSize = 1u << kSegBits;  // sources per LDS slice (64 KB of fp32), plus a zero slot
+constexpr uint32_t kSegBits = 15;
+constexpr uint32_t kSegSize = 1u << kSegBits;  // sources per LDS slice (128 KB of fp32), plus a zero slot
 static_assert(kSegSize <= 0xffff, "entries hold a slice offset or the zero slot in 16 bits");
-constexpr int kBlkThreads = 1024;              // segment-pass workgroup (one per CU: 130-144 KB of LDS)
-constexpr uint32_t kPieceMax = 512;            // longest piece (one wave step); longer ones are cut into chunks
-constexpr uint32_t kUnitEdges = 32768;         // entries per work unit, at most (64 KB staged)
-constexpr uint32_t kUnitEdgesW = 8192;         // with per-entry weights (16 + 32 KB staged)
-constexpr uint32_t kNoSlot = 0xffffffffu;      // lslot of the alignment gaps
-constexpr uint32_t kUnitPieces = 8192;         // pieces per work unit, at most (16 KB staged)
-constexpr uint32_t kCmbLight = 16;             // partials of a row combined by one lane, at most
-constexpr uint32_t kCmbMid = 128;              // by kCmbMidLanes lanes, at most; a wave beyond
-constexpr uint32_t kCmbMidLanes = 8;           // (16 partials each, all in flight)
+constexpr int kBlkThreads = 1024;              // segment-pass workgroup (one per CU: 128 KB of LDS)
+constexpr uint32_t kBlkWaves = kBlkThreads / kWave;
+constexpr uint32_t kClasses = 10;              // class c: pieces of up to 1 << c entries
+constexpr uint32_t kPieceMax = 1u << (kClasses - 1);
+constexpr uint32_t kCutCap = 32;               // capacities cut in two when at most 3/4 full
+constexpr uint32_t kTask = 512;                // entries of a task: 64 lanes x 8
+static_assert(kPieceMax == kTask, "the longest piece fills one task");
+// Tasks in flight per wave (1 KB each, weighted 3 KB): 64 and 96 KB per CU
+// cover the latency of the stream; a deeper weighted ring spills registers
+// (4 tasks: 41 against 22 us per RMAT-20 pass).
+template <bool kW>
+constexpr int kBlkRing = kW ? 2 : 4;
+constexpr uint32_t kSegMinEntries = 2048;      // entries of a staged segment, at least
+// Edges of a CSR with a segment pass, at least: one launch of m random
+// gathers (4.5 us + m / 180 G/s) against two launches (about 8.6 us on 1 M
+// edges, where the single launch takes 10.8; on 65 K edges it takes 5.5).
+constexpr uint32_t kPassMinEntries = 500000;
+constexpr uint32_t kDirectRowMax = 16384;      // without a segment pass: entries per row, at most
+constexpr uint32_t kIsPartial = 0x80000000u;   // combine term: a partial's index, else a source
+constexpr uint32_t kEidZero = 0xffffffffu;     // weight source of a padding entry: 0
+constexpr uint32_t kEidOne = 0xfffffffeu;      // weight source of a partial in the combine: 1
+constexpr uint32_t kCmbLight = 16;             // terms of a row combined by one lane, at most
+constexpr uint32_t kCmbMid = 128;              // by kCmbMidLanes lanes, at most
+constexpr uint32_t kCmbMidLanes = 8;
+constexpr uint32_t kCmbBig = 1024;             // by a wave, at most; a workgroup beyond
+constexpr uint32_t kCmbPer = 16;               // terms in flight per lane
 
-// Device arrays of a segmented pull over one CSR.
+// Device arrays of a segmented pull over one CSR (one allocation).
 struct BlockedPlan {
-  uint32_t n = 0, m = 0, n_live = 0;  // vertices, entries, rows with entries (a prefix of the rows)
-  uint32_t n_mid = 0, n_big = 0;      // rows with kCmbLight < partials <= kCmbMid, and more
-  uint32_t nseg = 0, npieces = 0, nunits = 0, ngroups = 0;
-  uint32_t unit_edges = 0, nent = 0;  // entries per unit at most; entries with gaps and spares
-  uint32_t *wg_ptr = nullptr;    // ngroups + 1: each segment-pass workgroup's range in wg_units
-  uint4 *wg_units = nullptr;     // nunits: the units of each workgroup in segment order, packed as
-                                 // (segment << 4 | bucket, first piece, first entry,
-                                 // pieces | entries << 16); bucket 0..8: lanes and reads per piece
-  uint4 *wg_first = nullptr;     // ngroups: each workgroup's first unit (zeros if it has none)
-  uint16_t *pbeg = nullptr;      // npieces: each piece's first entry, counted from its unit's first
-                                 // entry (a unit's last piece ends at the unit's aligned entry count)
-  uint16_t *lidx = nullptr;      // source offset within the segment, in piece order; each unit starts
-                                 // on an 8-entry boundary; the gaps and 8 spare entries at the end
-                                 // hold kSegSize (the slice's zero slot)
-  uint32_t *lslot = nullptr;     // (weighted solves only) CSR slot each entry came from, aligned as lidx
-                                 // (kNoSlot in the gaps and spares); its owner may map it in place
+  uint32_t n = 0, m = 0, n_live = 0;         // vertices, entries, rows up to the last one with entries
+  uint32_t n_mid = 0, n_big = 0, n_huge = 0; // rows with more than kCmbLight / kCmbMid / kCmbBig terms
+  uint32_t ntasks = 0, ngroups = 0;          // tasks, segment-pass workgroups (0: no segment pass)
+  uint32_t nparts = 0, ncmb = 0;             // partials (with class padding), combine terms
+  size_t nweights = 0;                       // weighted: ntasks * kTask + ncmb
+  void *mem = nullptr;
+  uint4 *wg_first = nullptr;     // ngroups: each workgroup's first item (segment, first task, end task,
+                                 // items | index of its second item in wg_items << 12)
+  uint4 *wg_items = nullptr;     // the workgroups' further items (segment, first task, end task, -)
+  uint2 *desc = nullptr;         // ntasks: class, first partial
+  uint16_t *lidx = nullptr;      // ntasks * kTask: source offset in the segment (kSegSize: padding)
   uint32_t *cmb_rp = nullptr;    // n + 1: each row's range in cmb_pos
-  uint32_t *cmb_pos = nullptr;   // npieces: partial index of each row's pieces, in segment order
-  uint32_t *cmb_mid = nullptr;   // n_mid: the rows with kCmbLight < partials <= kCmbMid, ascending
-  uint32_t *cmb_big = nullptr;   // n_big: the rows with more than kCmbMid partials, ascending
-  float *partial = nullptr;      // npieces
+  uint32_t *cmb_pos = nullptr;   // ncmb: kIsPartial | partial, or a source; by row, in segment order
+  uint32_t *cmb_rows = nullptr;  // rows of the mid, big and huge tiers, each ascending
+  float *partial = nullptr;      // nparts
+  // weighted plans: where the weight of every entry (in the order the segment
+  // pass reads them, see wpos) and then of every combine term comes from: an
+  // edge id, kEidZero or kEidOne
+  uint32_t *weid = nullptr;      // nweights
   bool ready = false;
   void release() {
-    void *ps[] = {wg_ptr, wg_units, wg_first, pbeg, lidx, lslot, cmb_rp, cmb_pos, cmb_mid, cmb_big, partial};
-    for (void *p : ps)
-      if (p) (void)hipFree(p);
-    wg_units = wg_first = nullptr;
-    wg_ptr = lslot = cmb_rp = cmb_pos = cmb_mid = cmb_big = nullptr;
-    pbeg = lidx = nullptr;
-    partial = nullptr;
-    ready = false;
+    if (mem) (void)hipFree(mem);
+    *this = BlockedPlan();
   }
 };
 
-// Host form of the plan (the arrays before upload).  units: nunits + 1
-// (segment, bucket, first piece, first entry), the last a sentinel (-, -,
-// npieces, entries); wg_list: the units of each workgroup.
-struct BlockedHost {
-  uint32_t n = 0, m = 0, n_live = 0, nseg = 0, npieces = 0, nunits = 0, ngroups = 0, nent = 0;
-  std::vector<uint4> units, wg_units, wg_first;
-  std::vector<uint32_t> wg_ptr, wg_list, lslot, cmb_rp, cmb_pos, cmb_mid, cmb_big;
-  std::vector<uint16_t> pbeg, lidx;
-};
-int build_blocked_host(const std::vector<uint32_t> &rp, const uint32_t *col, bool with_slots, uint32_t groups,
-                       uint32_t unit_edges, BlockedHost &h);
-
-// Builds the plan for a CSR whose rows are given by host offsets rp (n + 1)
-// and host entries col (m, source ids); rows must be ordered so that the rows
-// without entries come last (n_live = first such row).  with_slots keeps the
-// CSR slot of every entry (to gather per-slot data such as edge weights into
-// piece order).  groups: segment-pass workgroups to balance the units over;
-// unit_edges: entries per unit at most (kUnitEdges, or kUnitEdgesW for a
-// pass that stages per-entry weights).
-int build_blocked_plan(const std::vector<uint32_t> &rp, const uint32_t *col, bool with_slots, uint32_t groups,
-                       uint32_t unit_edges, BlockedPlan &bp);
+// Builds the plan on the device for the CSR rp (n + 1), col (m, source ids
+// < n).  eid (not null: a weighted plan): the edge id of every slot.
+// max_row: the longest row.  groups: workgroups of the segment pass.
+int build_blocked_plan(const uint32_t *rp, const uint32_t *col, const uint32_t *eid, uint32_t n, uint32_t m,
+                       uint32_t max_row, uint32_t groups, BlockedPlan &bp);
 
 struct BlkDev {
-  const uint32_t *wg_ptr;
-  const uint4 *wg_units;
   const uint4 *wg_first;
-  const uint16_t *pbeg;
+  const uint4 *wg_items;
+  const uint2 *desc;
   const uint16_t *lidx;
   const uint32_t *cmb_rp;
   const uint32_t *cmb_pos;
-  const uint32_t *cmb_mid, *cmb_big;
+  const uint32_t *cmb_mid, *cmb_big, *cmb_huge;
   float *partial;
-  const float *wpiece;  // per-entry weights in the plan's entry order (weighted passes)
-  uint32_t n, n_live, n_mid, n_big;
+  const float *went;  // weights of the entries, kTask per task (weighted passes)
+  const float *wcmb;  // weights of the combine terms
+  uint32_t n, n_live, n_mid, n_big, n_huge;
 };
 
-inline BlkDev make_blk_dev(const BlockedPlan &p, const float *wpiece = nullptr) {
-  return BlkDev{p.wg_ptr,  p.wg_units, p.wg_first, p.pbeg,  p.lidx, p.cmb_rp, p.cmb_pos, p.cmb_mid,
-                p.cmb_big, p.partial,  wpiece,     p.n,     p.n_live, p.n_mid, p.n_big};
+inline BlkDev make_blk_dev(const BlockedPlan &p, const float *weights = nullptr) {
+  BlkDev d;
+  d.wg_first = p.wg_first;
+  d.wg_items = p.wg_items;
+  d.desc = p.desc;
+  d.lidx = p.lidx;
+  d.cmb_rp = p.cmb_rp;
+  d.cmb_pos = p.cmb_pos;
+  d.cmb_mid = p.cmb_rows;
+  d.cmb_big = p.cmb_rows + p.n_mid;
+  d.cmb_huge = p.cmb_rows + p.n_mid + p.n_big;
+  d.partial = p.partial;
+  d.went = weights;
+  d.wcmb = weights ? weights + (size_t)p.ntasks * kTask : nullptr;
+  d.n = p.n;
+  d.n_live = p.n_live;
+  d.n_mid = p.n_mid;
+  d.n_big = p.n_big;
+  d.n_huge = p.n_huge;
+  return d;
 }
 
-// Lane j's share of a piece of a unit whose pieces take G lanes each: the
-// sum of sv(lidx[k]) over k = beg + j + i G, i < U (lidx and the slice in
-// LDS), all reads in flight at once and the terms added pairwise.  Such a
-// piece has at most U G entries (the length buckets), so this covers it;
-// the k past its end (up to `end`, the unit's alignment padding, or beyond)
-// read the slice's zero slot (kSegSize) instead of branching.
-constexpr int kStepReads = 8;  // reads per lane, at most
-constexpr uint32_t kBucketBits = 4;
-static_assert(kPieceMax <= kStepReads * kWave, "a piece fits one step of a wave");
-template <int G, int U, class SV>
-__device__ __forceinline__ float piece_step(const SV &sv, const uint16_t *lidx, uint32_t beg, uint32_t end,
-                                            uint32_t j) {
-  uint32_t ix[U];
-#pragma unroll
-  for (int i = 0; i < U; ++i) {
-    const uint32_t k = beg + j + (uint32_t)i * G;
-    ix[i] = k < end ? (uint32_t)lidx[k] : kSegSize;
-  }
-  float acc[U];
-#pragma unroll
-  for (int i = 0; i < U; ++i) acc[i] = sv(beg + j + (uint32_t)i * G, ix[i]);
-#pragma unroll
-  for (int w = U / 2; w > 0; w >>= 1)
-#pragma unroll
-    for (int i = 0; i < w; ++i) acc[i] += acc[i + w];
-  return acc[0];
+// Where the weight of entry x of a task sits among the task's kTask weights:
+// lane x / 8 reads its 8 weights with two 16-byte loads, each contiguous over
+// the wave.
+__host__ __device__ __forceinline__ uint32_t wpos(uint32_t x) {
+  return ((x >> 2) & 1u) * (kTask / 2) + (x >> 3) * 4 + (x & 3u);
 }
 
 // DPP move of x (rows of 16 lanes outside RowMask receive 0)
@@ -187,268 +192,288 @@ __device__ __forceinline__ float blk_group_sum(float v) {
   return v;
 }
 
-// Pieces of a unit summed G lanes each, U reads a lane; lane G - 1 of the
-// group stores the partial.
-template <int G, int U, class SV>
-__device__ __forceinline__ void blk_pieces(const BlkDev &d, const SV &sv, const uint16_t *s_lidx,
-                                           const uint16_t *s_pbeg, uint32_t np, uint32_t q0) {
-  const uint32_t j = threadIdx.x % G;
-  for (uint32_t q = threadIdx.x / G; q < np; q += kBlkThreads / G) {
-    const float s = blk_group_sum<G>(piece_step<G, U>(sv, s_lidx, s_pbeg[q], s_pbeg[q + 1], j));
-    if (j == G - 1) d.partial[q0 + q] = s;
+// One task: the 8 terms of this lane, summed by class into partials from
+// `part` on.
+__device__ __forceinline__ void blk_task(uint32_t cls, float *__restrict__ part, const float *v) {
+  const uint32_t lane = lane_id();
+  const float a0 = v[0] + v[1], a1 = v[2] + v[3], a2 = v[4] + v[5], a3 = v[6] + v[7];
+  if (cls == 1) {
+    reinterpret_cast<float4 *>(part)[lane] = make_float4(a0, a1, a2, a3);
+    return;
+  }
+  if (cls == 0) {
+    float4 *p = reinterpret_cast<float4 *>(part) + 2 * lane;
+    p[0] = make_float4(v[0], v[1], v[2], v[3]);
+    p[1] = make_float4(v[4], v[5], v[6], v[7]);
+    return;
+  }
+  if (cls == 2) {
+    reinterpret_cast<float2 *>(part)[lane] = make_float2(a0 + a1, a2 + a3);
+    return;
+  }
+  const float s = (a0 + a1) + (a2 + a3);
+  auto store = [&](float x, uint32_t lg) {  // groups of 2^lg lanes; the last one stores
+    const uint32_t g = (1u << lg) - 1;
+    if ((lane & g) == g) part[lane >> lg] = x;
+  };
+  switch (cls) {
+    case 3: part[lane] = s; break;
+    case 4: store(blk_group_sum<2>(s), 1); break;
+    case 5: store(blk_group_sum<4>(s), 2); break;
+    case 6: store(blk_group_sum<8>(s), 3); break;
+    case 7: store(blk_group_sum<16>(s), 4); break;
+    case 8: store(blk_group_sum<32>(s), 5); break;
+    default: store(blk_group_sum<kWave>(s), 6); break;
   }
 }
 
-// Segment pass of iteration k.  With a control block (ctl != nullptr) it
-// first applies the stop rule of the iteration loop: returns at once when
-// done; workgroup 0 alone sets done when iteration k - 1 left an L1 residual
-// below eps (the other workgroups' partials of that pass are then unused:
-// the combine launch returns on done) and clears the residual slots of
-// iteration k + 1.
-// SV: void bind(const float *slice, const float *wts) and
-// float operator()(uint32_t k, uint32_t i) const -- the summand of the
-// unit's entry k whose source is slice[i] (wts: the unit's staged weights,
-// kW only); it is also called with i = kSegSize (the zero slot) and k up to
-// kPieceMax past a piece's end, where slice[i] is 0 and wts[k] finite.
-// kW: units of at most kUnitEdgesW entries (plans built with that limit)
-// whose weights (d.wpiece) are staged in LDS beside their offsets.
-template <class SV, bool kW = false>
-__global__ void __launch_bounds__(kBlkThreads) blk_segment_kernel(BlkDev d, SV sv, const float *__restrict__ src,
+// Segment pass of iteration k over `src`.  It first applies the stop rule of
+// the iteration loop: returns at once when done; workgroup 0 alone sets done
+// when iteration k - 1 left an L1 residual below eps (the other workgroups'
+// partials of that pass are then unused: the combine launch returns on done)
+// and clears the residual slots of iteration k + 1.
+// kW: every entry's value is multiplied by its weight (d.went).
+template <bool kW>
+__global__ void __launch_bounds__(kBlkThreads) blk_segment_kernel(BlkDev d, const float *__restrict__ src,
                                                                    IterCtl *ctl, uint32_t k) {
-  constexpr uint32_t kUE = kW ? kUnitEdgesW : kUnitEdges;
-  constexpr uint32_t kWS = kW ? kUnitEdgesW + kPieceMax : 4;  // staged weights and a finite margin
-  __shared__ float slice[kSegSize + 4];  // slice[kSegSize] is the zero slot of the padding entries
-  __shared__ __align__(16) uint16_t s_lidx[kUE];
-  __shared__ __align__(16) float s_w[kWS];
-  __shared__ uint16_t s_pbeg[kUnitPieces + 2];  // piece starts and the unit's end
-  const uint32_t tid = threadIdx.x;
-  const uint32_t u0 = d.wg_ptr[blockIdx.x], u1 = d.wg_ptr[blockIdx.x + 1];
-  const uint4 first = d.wg_first[blockIdx.x];  // in flight with wg_ptr and during the checks
-  if (ctl) {
-    if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-    if (blockIdx.x == 0) {
-      if (k > 0) {
-        const double res = err_total(ctl, (k - 1) % 3);
-        if (res < ctl->eps) {
-          if (threadIdx.x == 0) {
-            ctl->iters = k;
-            ctl->residual = res;
-            __hip_atomic_store(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          }
-          return;
+  __shared__ __align__(16) float slice[kSegSize + 4];  // slice[kSegSize] is the zero slot of the padding entries
+  constexpr int R = kBlkRing<kW>;
+  const uint32_t tid = threadIdx.x, lane = lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  uint4 item = d.wg_first[blockIdx.x];  // in flight during the checks
+  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  if (blockIdx.x == 0) {
+    if (k > 0) {
+      const double res = err_total(ctl, (k - 1) % 3);
+      if (res < ctl->eps) {
+        if (threadIdx.x == 0) {
+          ctl->iters = k;
+          ctl->residual = res;
+          __hip_atomic_store(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+        return;
       }
-      double *z = &ctl->errs[(k + 1) % 3][0].v;
-      for (uint32_t i = threadIdx.x; i < kErrSlots * (sizeof(ErrSlot) / sizeof(double)); i += kBlkThreads) z[i] = 0.0;
     }
+    double *z = &ctl->errs[(k + 1) % 3][0].v;
+    for (uint32_t i = threadIdx.x; i < kErrSlots * (sizeof(ErrSlot) / sizeof(double)); i += kBlkThreads) z[i] = 0.0;
   }
-  if (u0 >= u1) return;
-  if (tid == 0) slice[kSegSize] = 0.f;  // read after the loop's first barrier
-  if constexpr (kW)
-    for (uint32_t i = tid; i < kWS; i += kBlkThreads) s_w[i] = 0.f;  // finite past any unit's weights
-  constexpr uint32_t kLi = kUE / (8 * kBlkThreads), kPi = kUnitPieces / kBlkThreads;
-  constexpr uint32_t kWv = kW ? kUE / (4 * kBlkThreads) : 1;
+  const uint32_t nitems = __builtin_amdgcn_readfirstlane(item.w & 0xfffu);
+  const uint32_t inext = __builtin_amdgcn_readfirstlane(item.w >> 12);
+  if (tid == 0) slice[kSegSize] = 0.f;  // read after the first barrier
   constexpr uint32_t kSl = kSegSize / (4 * kBlkThreads);
-  // The next unit's staged data -- and its segment of the source vector when
-  // that changes -- are loaded into registers while the current unit is
-  // summed, and the descriptor of the unit after it too: no load waits on
-  // another.  Entries move 8 at a time (units start on 8-entry boundaries).
-  uint4 li[kLi];
-  float4 wv[kWv];
-  uint32_t pb[kPi];
-  float4 sl[kSl];
-  auto load_unit = [&](const uint4 c, uint32_t have) {
-    const uint32_t np = c.w & 0xffffu, ne = c.w >> 16, seg = c.x >> kBucketBits;
-    const uint4 *lsrc = reinterpret_cast<const uint4 *>(d.lidx + c.z);
-#pragma unroll
-    for (uint32_t j = 0; j < kLi; ++j) {
-      const uint32_t i = tid + j * kBlkThreads;
-      li[j] = i * 8 < ne ? lsrc[i] : make_uint4(0, 0, 0, 0);
+  for (uint32_t it = 0; it < nitems; ++it) {
+    if (it) {
+      item = d.wg_items[inext + it - 1];
+      __syncthreads();  // the previous segment's sums are done with the slice
     }
-    if constexpr (kW) {
-      const float4 *wsrc = reinterpret_cast<const float4 *>(d.wpiece + c.z);
+    const uint32_t seg = __builtin_amdgcn_readfirstlane(item.x);
+    const uint32_t t0 = __builtin_amdgcn_readfirstlane(item.y) + wave;
+    const uint32_t t1 = __builtin_amdgcn_readfirstlane(item.z);
+    // this wave's tasks: t0, t0 + kBlkWaves, ...; lane i holds the
+    // descriptor of the i-th of up to 64 of them
+    uint32_t nt = t0 < t1 ? (t1 - t0 + kBlkWaves - 1) / kBlkWaves : 0u;
+    uint4 e[R];
+    float4 wa[kW ? R : 1], wb[kW ? R : 1];
+    auto load = [&](int j, uint32_t t) {
+      e[j] = reinterpret_cast<const uint4 *>(d.lidx + (size_t)t * kTask)[lane];
+      if constexpr (kW) {
+        const float4 *w = reinterpret_cast<const float4 *>(d.went + (size_t)t * kTask);
+        wa[j] = w[lane];
+        wb[j] = w[kWave + lane];
+      }
+    };
+    float4 sl[kSl];  // the slice first: the ring's loads then stay in flight behind it
+    const uint32_t base = seg << kSegBits, cnt = d.n - base;
+    if (cnt >= kSegSize) {
 #pragma unroll
-      for (uint32_t j = 0; j < kWv; ++j) {
-        const uint32_t i = tid + j * kBlkThreads;
-        wv[j] = i * 4 < ne ? wsrc[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (uint32_t j = 0; j < kSl; ++j)
+        sl[j] = *reinterpret_cast<const float4 *>(src + base + (tid + j * kBlkThreads) * 4);
+    } else {  // the last, partial segment
+#pragma unroll
+      for (uint32_t j = 0; j < kSl; ++j) {
+        const uint32_t i = (tid + j * kBlkThreads) * 4;
+        sl[j].x = i < cnt ? src[base + i] : 0.f;
+        sl[j].y = i + 1 < cnt ? src[base + i + 1] : 0.f;
+        sl[j].z = i + 2 < cnt ? src[base + i + 2] : 0.f;
+        sl[j].w = i + 3 < cnt ? src[base + i + 3] : 0.f;
       }
     }
+    uint2 ds = make_uint2(0, 0);
+    if (nt) {
+      if (lane < nt) ds = d.desc[t0 + lane * kBlkWaves];
 #pragma unroll
-    for (uint32_t j = 0; j < kPi; ++j) {
-      const uint32_t i = tid + j * kBlkThreads;
-      pb[j] = i < np ? d.pbeg[c.y + i] : 0u;
+      for (int j = 0; j < R; ++j) load(j, t0 + min((uint32_t)j, nt - 1) * kBlkWaves);
     }
-    if (seg != have) {
-      const uint32_t base = seg << kSegBits, cnt = d.n - base;
-      if (cnt >= kSegSize) {  // uniform: the descriptor is scalar
 #pragma unroll
-        for (uint32_t j = 0; j < kSl; ++j)
-          sl[j] = *reinterpret_cast<const float4 *>(src + base + (tid + j * kBlkThreads) * 4);
-      } else {  // the last, partial segment
+    for (uint32_t j = 0; j < kSl; ++j)
+      *reinterpret_cast<float4 *>(&slice[(tid + j * kBlkThreads) * 4]) = sl[j];
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < nt; i0 += kWave) {  // 64 tasks per batch of descriptors
+      if (i0 && lane < nt - i0) ds = d.desc[t0 + (i0 + lane) * kBlkWaves];
+      const uint32_t i1 = min(nt, i0 + kWave);
+      for (uint32_t i = i0; i < i1; i += R) {
 #pragma unroll
-        for (uint32_t j = 0; j < kSl; ++j) {
-          const uint32_t i = (tid + j * kBlkThreads) * 4;
-          sl[j].x = i < cnt ? src[base + i] : 0.f;
-          sl[j].y = i + 1 < cnt ? src[base + i + 1] : 0.f;
-          sl[j].z = i + 2 < cnt ? src[base + i + 2] : 0.f;
-          sl[j].w = i + 3 < cnt ? src[base + i + 3] : 0.f;
+        for (int j = 0; j < R; ++j) {
+          if (i + j < i1) {
+            const uint32_t x[4] = {e[j].x, e[j].y, e[j].z, e[j].w};
+            float v[8];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              v[2 * q] = slice[x[q] & 0xffffu];
+              v[2 * q + 1] = slice[x[q] >> 16];
+            }
+            if constexpr (kW) {
+              v[0] *= wa[j].x;
+              v[1] *= wa[j].y;
+              v[2] *= wa[j].z;
+              v[3] *= wa[j].w;
+              v[4] *= wb[j].x;
+              v[5] *= wb[j].y;
+              v[6] *= wb[j].z;
+              v[7] *= wb[j].w;
+            }
+            const uint32_t cls = __builtin_amdgcn_readlane(ds.x, i + j - i0);
+            float *part = d.partial + __builtin_amdgcn_readlane(ds.y, i + j - i0);
+            load(j, t0 + min(i + j + R, nt - 1) * kBlkWaves);
+            blk_task(cls, part, v);
+          }
         }
       }
-    }
-  };
-  // descriptors are the same for the whole workgroup: held in scalar registers
-  auto scalar = [](const uint4 c) {
-    return make_uint4(__builtin_amdgcn_readfirstlane(c.x), __builtin_amdgcn_readfirstlane(c.y),
-                      __builtin_amdgcn_readfirstlane(c.z), __builtin_amdgcn_readfirstlane(c.w));
-  };
-  uint4 cd = scalar(first);  // the unit whose data the registers hold
-  load_unit(cd, 0xffffffffu);
-  uint4 nd = u0 + 1 < u1 ? d.wg_units[u0 + 1] : cd;
-  uint32_t cur = 0xffffffffu;
-  for (uint32_t u = u0; u < u1; ++u) {
-    const uint32_t seg = cd.x >> kBucketBits, bucket = cd.x & ((1u << kBucketBits) - 1), q0 = cd.y;
-    const uint32_t np = cd.w & 0xffffu, ne = cd.w >> 16;
-    __syncthreads();  // the previous unit is done with the staged arrays
-    if (seg != cur) {
-#pragma unroll
-      for (uint32_t j = 0; j < kSl; ++j) *reinterpret_cast<float4 *>(&slice[(tid + j * kBlkThreads) * 4]) = sl[j];
-      cur = seg;
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kLi; ++j) {
-      const uint32_t i = tid + j * kBlkThreads;
-      if (i * 8 < ne) reinterpret_cast<uint4 *>(s_lidx)[i] = li[j];
-    }
-    if constexpr (kW) {
-#pragma unroll
-      for (uint32_t j = 0; j < kWv; ++j) {
-        const uint32_t i = tid + j * kBlkThreads;
-        if (i * 4 < ne) reinterpret_cast<float4 *>(s_w)[i] = wv[j];
-      }
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kPi; ++j) {
-      const uint32_t i = tid + j * kBlkThreads;
-      if (i < np) s_pbeg[i] = (uint16_t)pb[j];
-    }
-    if (tid == 0) s_pbeg[np] = (uint16_t)ne;
-    if (u + 1 < u1) {
-      cd = scalar(nd);
-      load_unit(cd, seg);
-      if (u + 2 < u1) nd = d.wg_units[u + 2];
-    }
-    __syncthreads();
-    sv.bind(slice, s_w);
-    // G lanes per piece and U reads per lane by bucket (pieces of up to U G
-    // entries)
-    switch (bucket) {
-      case 0:  // up to 2 entries
-        blk_pieces<1, 2>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 1:  // up to 4
-        blk_pieces<1, 4>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 2:  // up to 8
-        blk_pieces<1, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 3:
-        blk_pieces<2, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 4:
-        blk_pieces<4, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 5:
-        blk_pieces<8, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 6:
-        blk_pieces<16, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      case 7:
-        blk_pieces<32, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
-      default:  // up to kPieceMax
-        blk_pieces<kWave, 8>(d, sv, s_lidx, s_pbeg, np, q0);
-        break;
     }
   }
 }
 
-// Combine of iteration k: row v's partials added in a fixed order, then
+// Combine of iteration k: row v's terms added in a fixed order, then
 // fin.finish(v, sum, err, fin.pre(v)) (pre: the row's other inputs, loaded
-// ahead); the residual goes to errs[k % 3] (ctl != nullptr).
-// Rows by their number of partials: more than kCmbMid (the list cmb_big)
-// a wave each -- lane j adds partials j, j + 64, ... (four loads in flight),
-// then a DPP sum -- in the first big_blocks workgroups; kCmbLight + 1 to
-// kCmbMid (cmb_mid) kCmbMidLanes = 8 lanes each -- lane j adds partials j,
-// j + 8, ..., j + 120, all in flight, then a DPP sum -- in the next mid_blocks
-// workgroups; every other row a lane each, up to kCmbLight loads in flight
-// added in segment order, 256 consecutive rows per workgroup in the rest.
-// Rows without entries (v >= n_live) get a constant update: iterations 0
-// and 1 write it into both ping-pong buffers, later iterations skip them.
-template <class Fin>
-__global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, IterCtl *ctl, uint32_t k,
-                                                           uint32_t big_blocks, uint32_t mid_blocks) {
-  if (ctl && __hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+// ahead); the residual goes to errs[k % 3].  A term is a partial of the
+// segment pass or an element of `src`; kW: times its weight (1 for a partial).
+// Rows by their number of terms: more than kCmbBig a workgroup each (the
+// first huge_blocks workgroups), more than kCmbMid a wave, more than
+// kCmbLight kCmbMidLanes lanes, each lane with kCmbPer terms in flight and the
+// lanes' sums added with DPP moves; every other row a lane, its terms all in
+// flight and added in order, 256 consecutive rows per workgroup in the rest.
+// Rows past n_live get a constant update: iterations 0 and 1 write it into
+// both ping-pong buffers, later iterations skip them.
+// kSolo: there is no segment pass, so this launch applies the stop rule
+// (every workgroup reads the residual of iteration k - 1).
+template <class Fin, bool kW, bool kSolo>
+__global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, const float *__restrict__ src,
+                                                          IterCtl *ctl, uint32_t k, uint32_t huge_blocks,
+                                                          uint32_t big_blocks, uint32_t mid_blocks) {
+  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  if constexpr (kSolo) {
+    if (k > 0) {
+      const double res = err_total(ctl, (k - 1) % 3);
+      if (res < ctl->eps) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+          ctl->iters = k;
+          ctl->residual = res;
+          __hip_atomic_store(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        return;
+      }
+    }
+    if (blockIdx.x == 0) {
+      double *z = &ctl->errs[(k + 1) % 3][0].v;
+      for (uint32_t i = threadIdx.x; i < kErrSlots * (sizeof(ErrSlot) / sizeof(double)); i += 256) z[i] = 0.0;
+    }
+  }
   __shared__ float s_red[256 / kWave];
-  const uint32_t nv = (!ctl || k >= 2) ? d.n_live : d.n;
+  const uint32_t nv = k >= 2 ? d.n_live : d.n;
   float err = 0.f;
   const uint32_t lane = threadIdx.x % kWave;
-  if (blockIdx.x < big_blocks) {
-    for (uint32_t i = (blockIdx.x * 256 + threadIdx.x) / kWave; i < d.n_big; i += big_blocks * (256 / kWave)) {
-      const uint32_t v = d.cmb_big[i];  // the same for the whole wave
-      const uint32_t a = d.cmb_rp[v], b = d.cmb_rp[v + 1];
-      float s = 0.f;
-      for (uint32_t q0 = a + lane; q0 < b; q0 += 4 * kWave) {
-        uint32_t ix[4];
+  // U terms of a range from q on, `stride` apart, all in flight; 0 past end
+  auto terms = [&](auto u, uint32_t q, uint32_t stride, uint32_t end, float *p) {
+    constexpr uint32_t U = decltype(u)::value;
+    uint32_t ix[U];
+    float w[kW ? U : 1];
 #pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) ix[t] = q0 + t * kWave < b ? d.cmb_pos[q0 + t * kWave] : 0u;
-        float p[4];
+    for (uint32_t t = 0; t < U; ++t) ix[t] = q + t * stride < end ? d.cmb_pos[q + t * stride] : 0u;
+    if constexpr (kW) {  // beside a segment pass nearly every term is a partial: no weight to load
 #pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) p[t] = q0 + t * kWave < b ? d.partial[ix[t]] : 0.f;
-#pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) s += p[t];
+      for (uint32_t t = 0; t < U; ++t) {
+        const bool has = kSolo ? q + t * stride < end : (q + t * stride < end && !(ix[t] & kIsPartial));
+        w[t] = has ? d.wcmb[q + t * stride] : 1.f;
       }
-      s = blk_group_sum<kWave>(s);
+    }
+#pragma unroll
+    for (uint32_t t = 0; t < U; ++t) {
+      const float *b = (ix[t] & kIsPartial) ? d.partial : src;
+      p[t] = q + t * stride < end ? b[ix[t] & ~kIsPartial] : 0.f;
+    }
+    if constexpr (kW) {
+#pragma unroll
+      for (uint32_t t = 0; t < U; ++t) p[t] *= w[t];
+    }
+  };
+  using Per = std::integral_constant<uint32_t, kCmbPer>;
+  uint32_t blk = blockIdx.x;
+  if (blk < huge_blocks) {
+    for (uint32_t i = blk; i < d.n_huge; i += huge_blocks) {
+      const uint32_t v = d.cmb_huge[i];
+      const uint32_t b = d.cmb_rp[v + 1];
+      float s = 0.f;
+      for (uint32_t q = d.cmb_rp[v] + threadIdx.x; q < b; q += kCmbPer * 256) {
+        float p[kCmbPer];
+        terms(Per{}, q, 256, b, p);
+#pragma unroll
+        for (uint32_t w = kCmbPer / 2; w > 0; w >>= 1)
+#pragma unroll
+          for (uint32_t t = 0; t < w; ++t) p[t] += p[t + w];
+        s += p[0];
+      }
+      s = block_sum<256, float>(s, s_red);
+      if (threadIdx.x == 0) fin.finish(v, s, err, fin.pre(v));
+    }
+  } else if ((blk -= huge_blocks) < big_blocks) {
+    for (uint32_t i = (blk * 256 + threadIdx.x) / kWave; i < d.n_big; i += big_blocks * (256 / kWave)) {
+      const uint32_t v = d.cmb_big[i];  // the same for the whole wave
+      float p[kCmbPer];
+      terms(Per{}, d.cmb_rp[v] + lane, kWave, d.cmb_rp[v + 1], p);
+#pragma unroll
+      for (uint32_t w = kCmbPer / 2; w > 0; w >>= 1)
+#pragma unroll
+        for (uint32_t t = 0; t < w; ++t) p[t] += p[t + w];
+      const float s = blk_group_sum<kWave>(p[0]);
       if (lane == 0) fin.finish(v, s, err, fin.pre(v));
     }
-  } else if (blockIdx.x < big_blocks + mid_blocks) {
-    constexpr uint32_t G = kCmbMidLanes, kPer = kCmbMid / G;
+  } else if ((blk -= big_blocks) < mid_blocks) {
+    constexpr uint32_t G = kCmbMidLanes;
     const uint32_t j = threadIdx.x % G;
-    for (uint32_t i = ((blockIdx.x - big_blocks) * 256 + threadIdx.x) / G; i < d.n_mid; i += mid_blocks * (256 / G)) {
+    for (uint32_t i = (blk * 256 + threadIdx.x) / G; i < d.n_mid; i += mid_blocks * (256 / G)) {
       const uint32_t v = d.cmb_mid[i];  // the same for the group's lanes (inside one DPP row)
-      const uint32_t a = d.cmb_rp[v], b = d.cmb_rp[v + 1];
-      uint32_t ix[kPer];
+      float p[kCmbPer];
+      terms(Per{}, d.cmb_rp[v] + j, G, d.cmb_rp[v + 1], p);
 #pragma unroll
-      for (uint32_t t = 0; t < kPer; ++t) ix[t] = a + j + t * G < b ? d.cmb_pos[a + j + t * G] : 0u;
-      float p[kPer];
+      for (uint32_t w = kCmbPer / 2; w > 0; w >>= 1)
 #pragma unroll
-      for (uint32_t t = 0; t < kPer; ++t) p[t] = a + j + t * G < b ? d.partial[ix[t]] : 0.f;
-      float s = 0.f;
-#pragma unroll
-      for (uint32_t t = 0; t < kPer; ++t) s += p[t];
-      s = blk_group_sum<G>(s);
+        for (uint32_t t = 0; t < w; ++t) p[t] += p[t + w];
+      const float s = blk_group_sum<G>(p[0]);
       if (j == 0) fin.finish(v, s, err, fin.pre(v));
     }
   } else {
-    const uint32_t lb = blockIdx.x - big_blocks - mid_blocks, nlb = gridDim.x - big_blocks - mid_blocks;
-    for (uint32_t v = lb * 256 + threadIdx.x; v < nv; v += nlb * 256) {
+    blk -= mid_blocks;
+    const uint32_t nlb = gridDim.x - huge_blocks - big_blocks - mid_blocks;
+    for (uint32_t v = blk * 256 + threadIdx.x; v < nv; v += nlb * 256) {
       const uint32_t a = d.cmb_rp[v], b = d.cmb_rp[v + 1];
       if (b - a > kCmbLight) continue;  // a listed row
       const auto pre = fin.pre(v);
-      uint32_t ix[kCmbLight];
-#pragma unroll
-      for (uint32_t t = 0; t < kCmbLight; ++t) ix[t] = a + t < b ? d.cmb_pos[a + t] : 0u;
-      float p[kCmbLight];
-#pragma unroll
-      for (uint32_t t = 0; t < kCmbLight; ++t) p[t] = a + t < b ? d.partial[ix[t]] : 0.f;
+      // the wave takes 4, 8 or 16 terms a lane by its longest row
+      const bool over4 = ballot(b - a > 4) != 0, over8 = ballot(b - a > 8) != 0;
       float s = 0.f;
+      auto run = [&](auto u) {
+        constexpr uint32_t U = decltype(u)::value;
+        float p[U];
+        terms(u, a, 1, b, p);
 #pragma unroll
-      for (uint32_t t = 0; t < kCmbLight; ++t)
-        if (a + t < b) s += p[t];
+        for (uint32_t t = 0; t < U; ++t) s += p[t];
+      };
+      if (over8) run(std::integral_constant<uint32_t, 16>{});
+      else if (over4) run(std::integral_constant<uint32_t, 8>{});
+      else run(std::integral_constant<uint32_t, 4>{});
       fin.finish(v, s, err, pre);
     }
   }
-  if (!ctl) return;
   err = block_sum<256, float>(err, s_red);
   if (threadIdx.x == 0 && err != 0.f) atomicAdd(&ctl->errs[k % 3][blockIdx.x % kErrSlots].v, (double)err);
 }

@@ -99,8 +99,7 @@ struct olv_graph {
   // (built on first use; shared by the PageRank pull and the BFS twin).
   uint32_t *rl_pi = nullptr;       // vertex -> new number
   uint32_t *rl_order = nullptr;    // new number -> vertex
-  std::vector<uint32_t> h_rl_pi;   // host copies of rl_pi (seed mapping) and rl_order
-  std::vector<uint32_t> h_rl_order;
+  std::vector<uint32_t> h_rl_pi;   // host copy of rl_pi (seed mapping; made with the twin)
   olv_graph *twin = nullptr;       // this graph renumbered by rl_pi (BFS runs on it)
   const uint32_t *out_map = nullptr;  // a twin: its vertex -> the original graph's (not owned)
   uint32_t *union_map = nullptr;   // multigraph: unused here
@@ -118,15 +117,17 @@ bool seg_plan_stale(const SegPlan &plan, const Tuning &t);
 // A graph never tuned takes its signature's entry in the tuning cache named
 // by the OLV_TUNE_CACHE environment variable, if any (autotune.hip).
 int apply_cached_tuning(olv_graph *g);
-// In-degree numbering of g (g->rl_pi, g->rl_order, g->h_rl_pi), built
-// once; needs the in-CSR.  order (optional) receives new number -> vertex.
-int indeg_order(olv_graph *g, std::vector<uint32_t> *order);
+// In-degree numbering of g (g->rl_pi, g->rl_order), built once; needs the
+// in-CSR.
+int indeg_order(olv_graph *g);
 // g->twin: g renumbered by its in-degree numbering, with its transpose.
 int ensure_twin(olv_graph *g);
 int ensure_in_head(olv_graph *g);
 int compute_inv_outdeg(const uint32_t *rp, uint32_t n, float *inv);  // 1/outdeg (0 for sinks)
 // Device exclusive prefix sum (ingest.hip): out[0..n), out[n] = total < 2^32.
 int exclusive_scan(const uint32_t *in, uint32_t *out, size_t n);
+// row[e] = the row of slot e of a CSR (n + 1 offsets, m slots; ingest.hip).
+int slot_rows(const uint32_t *rp, uint32_t n, uint32_t m, uint32_t *row);
 void free_bfs_work(olv_graph *g);
 // This device's address of the allocation-free BFS's static work array
 // (looked up once per device).

@@ -21,6 +21,7 @@
 
 #include "blocked.hpp"
 #include "internal.hpp"
+#include "radix.hpp"
 #include "seg_core.hpp"
 
 namespace olv {
@@ -55,8 +56,7 @@ struct PrRelabel {
   RelabelSide in, out;
   BlockedPlan blk_in;    // source-segmented pull over the renumbered in-CSR
   // the same for the weighted solves: [0] over the renumbered in-CSR
-  // (forward), [1] over the out-CSR (adjoint); their lslot holds each
-  // entry's edge id (the slot mapped through the side's eid when built)
+  // (forward), [1] over the out-CSR (adjoint)
   BlockedPlan blk_w[2];
   float *inv = nullptr;  // n: 1/outdeg by new number
   void release() {
@@ -81,9 +81,8 @@ struct PrWork {
   float *wslot[2] = {nullptr, nullptr};  // m floats each
   const float *wslot_src[2] = {nullptr, nullptr};
   const uint32_t *wslot_eid[2] = {nullptr, nullptr};
-  // The same in the entry order of the segmented pulls (rl.blk_w[side]):
-  // w[eid[lslot[e]]] at entry e, 0 in the alignment gaps.
-  float *wpiece[2] = {nullptr, nullptr};  // rl.blk_w[side].nent floats each
+  // The same in the order of the segmented pulls (rl.blk_w[side].weid).
+  float *wpiece[2] = {nullptr, nullptr};  // rl.blk_w[side].nweights floats each
   const float *wpiece_src[2] = {nullptr, nullptr};
   const uint32_t *wpiece_eid[2] = {nullptr, nullptr};
   IterCtl *ctl = nullptr;
@@ -150,31 +149,31 @@ static int ensure_plan(olv_graph *g, bool in_edges) {
   return OLV_OK;
 }
 
+// len[i] = length of row order[i] of the source CSR
+__global__ void row_len_kernel(const uint32_t *__restrict__ src_rp, const uint32_t *__restrict__ order, uint32_t n,
+                               uint32_t *__restrict__ len) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    len[i] = src_rp[order[i] + 1] - src_rp[order[i]];
+}
+
 // Row i of a renumbered CSR is row order[i] of the source CSR with every
 // entry u replaced by pi[u]; eid (if not null) receives each slot's edge id,
-// src_eid[slot] or, with src_eid null, the source slot itself.  One wave per
-// row.
-__global__ void relabel_rows_kernel(const uint32_t *__restrict__ order, const uint32_t *__restrict__ pi,
-                                    const uint32_t *__restrict__ src_rp, const uint32_t *__restrict__ src_col,
-                                    const uint32_t *__restrict__ src_eid, const uint32_t *__restrict__ rp, uint32_t n,
-                                    uint32_t *__restrict__ col, uint32_t *__restrict__ eid) {
-  const uint32_t waves = gridDim.x * (blockDim.x / kWave);
-  const uint32_t lane = threadIdx.x % kWave;
-  for (uint32_t i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; i < n; i += waves) {
-    const uint32_t v = order[i];
-    const uint32_t b = src_rp[v], len = src_rp[v + 1] - b, o = rp[i];
-    for (uint32_t j0 = lane; j0 < len; j0 += 4 * kWave) {  // four loads in flight per lane
-      uint32_t c[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) c[q] = j0 + q * kWave < len ? src_col[b + j0 + q * kWave] : 0u;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        if (j0 + q * kWave < len) {
-          const uint32_t k = b + j0 + q * kWave;
-          col[o + j0 + q * kWave] = pi[c[q]];
-          if (eid) eid[o + j0 + q * kWave] = src_eid ? src_eid[k] : k;
-        }
-    }
+// src_eid[slot] or, with src_eid null, the source slot itself.  A workgroup
+// takes a tile of consecutive slots, so a hub's row is shared like any other
+// (a wave per row took 536 us on RMAT-20).
+__global__ void __launch_bounds__(kIB)
+    relabel_slots_kernel(const uint32_t *__restrict__ order, const uint32_t *__restrict__ pi,
+                         const uint32_t *__restrict__ src_rp, const uint32_t *__restrict__ src_col,
+                         const uint32_t *__restrict__ src_eid, const uint32_t *__restrict__ rp, uint32_t n, uint32_t m,
+                         uint32_t *__restrict__ col, uint32_t *__restrict__ eid) {
+  __shared__ uint32_t s_row[kITile];
+  const uint32_t base = blockIdx.x * kITile, cnt = min(kITile, m - base);
+  const uint32_t first = tile_rows(rp, n, base, cnt, s_row);
+  for (uint32_t j = threadIdx.x; j < cnt; j += kIB) {
+    const uint32_t i = first + s_row[j];
+    const uint32_t k = src_rp[order[i]] + (base + j - rp[i]);
+    col[base + j] = pi[src_col[k]];
+    if (eid) eid[base + j] = src_eid ? src_eid[k] : k;
   }
 }
 
@@ -191,43 +190,39 @@ static unsigned ew_grid(size_t n);
 // edge ids when with_eid (weighted solves).
 static int ensure_side(olv_graph *g, PrWork *w, bool in_edges, bool with_eid) {
   RelabelSide &sd = in_edges ? w->rl.in : w->rl.out;
-  if (sd.ready && (sd.eid || !with_eid)) {
-    if (seg_plan_stale(sd.plan, g->tune)) {  // the bucket bounds changed: new plan, same arrays
-      std::vector<uint32_t> rp((size_t)g->n + 1);
-      OLV_HIP(hipMemcpy(rp.data(), sd.rp, rp.size() * 4, hipMemcpyDeviceToHost));
-      OLV_TRY(build_seg_plan_rp(rp, g->tune.seg_bounds, sd.plan));
-    }
-    return OLV_OK;
-  }
+  if (sd.ready && (sd.eid || !with_eid)) return OLV_OK;
   sd.release();
   const uint32_t n = g->n, m = g->m;
   if (in_edges && !g->in_row_ptr) OLV_TRY(olv_graph_build_transpose(g));
-  std::vector<uint32_t> order;
-  OLV_TRY(indeg_order(g, &order));
-  const uint32_t *d_src_rp = in_edges ? g->in_row_ptr : g->row_ptr;
-  std::vector<uint32_t> src_rp((size_t)n + 1), rp((size_t)n + 1);
-  OLV_HIP(hipMemcpy(src_rp.data(), d_src_rp, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost));
-  rp[0] = 0;
-  for (uint32_t i = 0; i < n; ++i) rp[i + 1] = rp[i] + (src_rp[order[i] + 1] - src_rp[order[i]]);
+  OLV_TRY(indeg_order(g));
+  const uint32_t *src_rp = in_edges ? g->in_row_ptr : g->row_ptr;
   OLV_HIP(hipMalloc(reinterpret_cast<void **>(&sd.rp), ((size_t)n + 1) * 4));
   OLV_HIP(hipMalloc(reinterpret_cast<void **>(&sd.col), std::max<size_t>(m, 1) * 4));
   if (with_eid) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&sd.eid), std::max<size_t>(m, 1) * 4));
-  OLV_HIP(hipMemcpy(sd.rp, rp.data(), ((size_t)n + 1) * 4, hipMemcpyHostToDevice));
   if (!w->rl.inv) {
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&w->rl.inv), std::max<size_t>(n, 1) * 4));
-    if (n)
-      hipLaunchKernelGGL(gather_kernel<float>, dim3(ew_grid(n)), dim3(256), 0, stream(),
-                         (const float *)g->inv_outdeg, g->rl_order, n, w->rl.inv);
+    hipLaunchKernelGGL(gather_kernel<float>, dim3(ew_grid(n)), dim3(256), 0, stream(), (const float *)g->inv_outdeg,
+                       g->rl_order, n, w->rl.inv);
   }
-  if (n)
-    hipLaunchKernelGGL(relabel_rows_kernel, dim3(ew_grid((size_t)n * kWave)), dim3(256), 0, stream(), g->rl_order,
-                       g->rl_pi, d_src_rp, in_edges ? g->in_col : g->col, in_edges ? g->in_eid : nullptr, sd.rp, n,
-                       sd.col, sd.eid);
+  hipLaunchKernelGGL(row_len_kernel, dim3(ew_grid(n)), dim3(256), 0, stream(), src_rp, g->rl_order, n, sd.rp);
+  OLV_TRY(exclusive_scan(sd.rp, sd.rp, n));
+  if (m)
+    hipLaunchKernelGGL(relabel_slots_kernel, dim3((unsigned)(((size_t)m + kITile - 1) / kITile)), dim3(kIB), 0,
+                       stream(), g->rl_order, g->rl_pi, src_rp, in_edges ? g->in_col : g->col,
+                       in_edges ? g->in_eid : nullptr, sd.rp, n, m, sd.col, sd.eid);
   OLV_HIP(hipGetLastError());
-  OLV_TRY(build_seg_plan_rp(rp, g->tune.seg_bounds, sd.plan));
   OLV_HIP(hipStreamSynchronize(stream()));
   sd.ready = true;
   return OLV_OK;
+}
+
+// The degree buckets of a side's rows (the per-row pulls), built on first
+// use and again when the bucket bounds change.
+static int ensure_side_plan(olv_graph *g, RelabelSide &sd) {
+  if (sd.plan.list && !seg_plan_stale(sd.plan, g->tune)) return OLV_OK;
+  std::vector<uint32_t> rp((size_t)g->n + 1);
+  OLV_HIP(hipMemcpy(rp.data(), sd.rp, rp.size() * 4, hipMemcpyDeviceToHost));
+  return build_seg_plan_rp(rp, g->tune.seg_bounds, sd.plan);
 }
 
 // The source-segmented pull plan over the renumbered in-CSR (built once).
@@ -235,37 +230,19 @@ static int ensure_blocked(olv_graph *g, PrWork *w) {
   BlockedPlan &bp = w->rl.blk_in;
   if (bp.ready) return OLV_OK;
   OLV_TRY(ensure_side(g, w, true, false));
-  const uint32_t n = g->n, m = g->m;
-  std::vector<uint32_t> rp((size_t)n + 1), col(std::max<uint32_t>(m, 1));
-  OLV_HIP(hipMemcpy(rp.data(), w->rl.in.rp, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost));
-  if (m) OLV_HIP(hipMemcpy(col.data(), w->rl.in.col, (size_t)m * 4, hipMemcpyDeviceToHost));
-  return build_blocked_plan(rp, col.data(), false, (uint32_t)cu_count(), kUnitEdges, bp);
-}
-
-// lslot[e] <- eid[lslot[e]] where lslot[e] is a slot
-__global__ void slot_to_edge_kernel(uint32_t *__restrict__ lslot, const uint32_t *__restrict__ eid, uint32_t nent) {
-  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < nent; e += gridDim.x * blockDim.x) {
-    const uint32_t s = lslot[e];
-    if (s != kNoSlot) lslot[e] = eid[s];
-  }
+  return build_blocked_plan(w->rl.in.rp, w->rl.in.col, nullptr, g->n, g->m, g->max_indeg, (uint32_t)cu_count(), bp);
 }
 
 // The segmented pull plan of a weighted solve over the renumbered in-CSR
-// (side 0) or out-CSR (side 1), with every entry's edge id and units small
-// enough to stage their weights (built once per side).
+// (side 0) or out-CSR (side 1), with every entry's edge id (built once per
+// side).
 static int ensure_wblocked(olv_graph *g, PrWork *w, int side) {
   BlockedPlan &bp = w->rl.blk_w[side];
   if (bp.ready) return OLV_OK;
   OLV_TRY(ensure_side(g, w, side == 0, true));
   const RelabelSide &sd = side == 0 ? w->rl.in : w->rl.out;
-  const uint32_t n = g->n, m = g->m;
-  std::vector<uint32_t> rp((size_t)n + 1), col(std::max<uint32_t>(m, 1));
-  OLV_HIP(hipMemcpy(rp.data(), sd.rp, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost));
-  if (m) OLV_HIP(hipMemcpy(col.data(), sd.col, (size_t)m * 4, hipMemcpyDeviceToHost));
-  OLV_TRY(build_blocked_plan(rp, col.data(), true, (uint32_t)cu_count(), kUnitEdgesW, bp));
-  hipLaunchKernelGGL(slot_to_edge_kernel, dim3(ew_grid(bp.nent)), dim3(256), 0, stream(), bp.lslot, sd.eid, bp.nent);
-  OLV_HIP(hipGetLastError());
-  return OLV_OK;
+  return build_blocked_plan(sd.rp, sd.col, sd.eid, g->n, g->m, side == 0 ? g->max_indeg : g->max_outdeg,
+                            (uint32_t)cu_count(), bp);
 }
 
 // ----------------------------------------------------------------- ops
@@ -286,24 +263,6 @@ struct PrOp {
     r[v] = rn;
     contrib_next[v] = rn * inv_outdeg[v];
   }
-};
-
-// Summand of the segmented pull for plain PageRank: the staged contribution.
-struct SliceVal {
-  const float *sl = nullptr;
-  __device__ __forceinline__ void bind(const float *s, const float *) { sl = s; }
-  __device__ __forceinline__ float operator()(uint32_t, uint32_t i) const { return sl[i]; }
-};
-
-// Summand of a weighted segmented pull: the entry's staged weight times the
-// staged source value (the iterate for the forward, lambda for the adjoint).
-struct WSliceVal {
-  const float *sl = nullptr, *w = nullptr;
-  __device__ __forceinline__ void bind(const float *s, const float *ws) {
-    sl = s;
-    w = ws;
-  }
-  __device__ __forceinline__ float operator()(uint32_t k, uint32_t i) const { return w[k] * sl[i]; }
 };
 
 // The update of WprOp::finish for the combine of the segmented pull.
@@ -394,23 +353,32 @@ struct AdjOp {
   }
 };
 
-// grad_w[e=(u,v)] = d * r_u * lambda_v, written while walking the out-CSR
-// (Mapped: a renumbered out-CSR, whose slot k holds edge eid[k]).
-template <bool Mapped>
-struct GradOp {
-  const uint32_t *ci;
-  const float *r;
-  const float *lam;
-  float *grad_w;
-  const uint32_t *eid;
-  float d;
-  __device__ __forceinline__ uint32_t idx(uint32_t k) const { return ld_stream(&ci[k]); }
-  __device__ __forceinline__ float val(uint32_t u, uint32_t k, uint32_t v) const {
-    __builtin_nontemporal_store(d * r[u] * lam[v], &grad_w[Mapped ? ld_stream(&eid[k]) : k]);
-    return 0.f;
+// grad_w[e=(u,v)] = d * r_u * lambda_v over the graph's own out-CSR, r and
+// lambda in its numbering: a workgroup takes a tile of consecutive edges, so
+// the column reads and the gradient stores are whole lines: 132 us on RMAT-20,
+// bound by the gathers of lambda (walking the renumbered rows and storing
+// through each slot's edge id took 180).
+__global__ void __launch_bounds__(kIB)
+    edge_grad_kernel(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col, uint32_t n, uint32_t m,
+                     const float *__restrict__ r, const float *__restrict__ lam, float d, float *__restrict__ grad_w) {
+  __shared__ uint32_t s_row[kITile];
+  const uint32_t base = blockIdx.x * kITile, cnt = min(kITile, m - base);
+  uint32_t v[kIItems];
+#pragma unroll
+  for (int i = 0; i < kIItems; ++i) {
+    const uint32_t j = threadIdx.x + i * kIB;
+    v[i] = j < cnt ? col[base + j] : 0u;
   }
-  __device__ __forceinline__ void finish(uint32_t, float, float &) const {}
-};
+  const uint32_t first = tile_rows(rp, n, base, cnt, s_row);
+  float lv[kIItems];
+#pragma unroll
+  for (int i = 0; i < kIItems; ++i) lv[i] = lam[v[i]];
+#pragma unroll
+  for (int i = 0; i < kIItems; ++i) {
+    const uint32_t j = threadIdx.x + i * kIB;
+    if (j < cnt) grad_w[base + j] = d * r[first + s_row[j]] * lv[i];
+  }
+}
 
 // --------------------------------------------------------------- kernels
 // Zero the control block and set eps (all threads of the calling workgroup).
@@ -481,25 +449,32 @@ static int slot_weights(const olv_graph *g, PrWork *pw, int side, const float *w
   return OLV_OK;
 }
 
-// out[e] = w[edge[e]], 0 where edge[e] is kNoSlot
-__global__ void piece_weight_kernel(const float *__restrict__ w, const uint32_t *__restrict__ edge, uint32_t nent,
+// out[e] = w[eid[e]], 0 or 1 where eid[e] is kEidZero or kEidOne
+__global__ void piece_weight_kernel(const float *__restrict__ w, const uint32_t *__restrict__ eid, size_t count,
                                     float *__restrict__ out) {
-  for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < nent; e += gridDim.x * blockDim.x) {
-    const uint32_t x = edge[e];
-    out[e] = x != kNoSlot ? w[x] : 0.f;
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < count; e += (size_t)gridDim.x * blockDim.x) {
+    const uint32_t x = eid[e];
+    out[e] = x < kEidOne ? w[x] : (x == kEidOne ? 1.f : 0.f);
   }
 }
 
-// The weights w in the entry order of the weighted segmented pull of side 0
+static int enqueue_piece_weights(const BlockedPlan &bp, const float *w, float *out) {
+  if (bp.nweights)
+    hipLaunchKernelGGL(piece_weight_kernel, dim3(ew_grid(bp.nweights)), dim3(256), 0, stream(), w, bp.weid, bp.nweights,
+                       out);
+  OLV_HIP(hipGetLastError());
+  return OLV_OK;
+}
+
+// The weights w in the order of the weighted segmented pull of side 0
 // (in-CSR) or 1 (out-CSR), cached like slot_weights' copies.
 static int piece_weights(PrWork *pw, int side, const float *w, const uint32_t *eid, bool reuse, bool staged,
                          const float **out) {
   const BlockedPlan &bp = pw->rl.blk_w[side];
-  if (!pw->wpiece[side]) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&pw->wpiece[side]), (size_t)bp.nent * 4));
+  if (!pw->wpiece[side])
+    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&pw->wpiece[side]), std::max<size_t>(bp.nweights, 1) * 4));
   if (!(reuse && !staged && pw->wpiece_src[side] == w && pw->wpiece_eid[side] == eid)) {
-    hipLaunchKernelGGL(piece_weight_kernel, dim3(ew_grid(bp.nent)), dim3(256), 0, stream(), w, bp.lslot, bp.nent,
-                       pw->wpiece[side]);
-    OLV_HIP(hipGetLastError());
+    OLV_TRY(enqueue_piece_weights(bp, w, pw->wpiece[side]));
     pw->wpiece_src[side] = staged ? nullptr : w;
     pw->wpiece_eid[side] = eid;
     if (!reuse && pw->wpiece_src[side ^ 1] == w) pw->wpiece_src[side ^ 1] = nullptr;
@@ -563,22 +538,28 @@ static int enqueue_iteration(const SegDev &d, const uint32_t *rp, const Op &op, 
   return OLV_OK;
 }
 
-// One iteration of a segmented pull: the segment pass over `src` with
-// summand SV, then the combine applying `fin`.
-template <class SV, bool kW, class Fin>
-static int enqueue_blocked(const BlockedPlan &bp, const BlkDev &bd, const float *src, const Fin &fin, PrWork *w,
+// One iteration of a segmented pull over `src` (weights: null, or the plan's
+// weights): the segment pass, if the plan has one, then the combine applying
+// `fin`.
+template <bool kW, class Fin>
+static int enqueue_blocked(const BlockedPlan &bp, const float *weights, const float *src, const Fin &fin, PrWork *w,
                            uint32_t k, KernelProfile *prof = nullptr) {
-  // combine: a wave per listed big row, kCmbMidLanes lanes per listed mid
-  // row, then a lane per row
+  const BlkDev bd = make_blk_dev(bp, weights);
   const unsigned cu = (unsigned)cu_count();
-  const unsigned gb = std::min<unsigned>((bp.n_big + 3) / 4, cu * 4);
+  const unsigned gh = std::min<unsigned>(bp.n_huge, cu * 4);
+  const unsigned gb = std::min<unsigned>((bp.n_big + 3) / 4, cu * 8);
   const unsigned gm = std::min<unsigned>((bp.n_mid + 256 / kCmbMidLanes - 1) / (256 / kCmbMidLanes), cu * 16);
-  const unsigned gc = gb + gm + ew_grid(bp.n);
+  const dim3 gc(gh + gb + gm + ew_grid(bp.n));
   hipEvent_t a = prof ? prof->next() : nullptr, b = prof ? prof->next() : nullptr;
   if (a) OLV_HIP(hipEventRecord(a, stream()));
-  hipLaunchKernelGGL((blk_segment_kernel<SV, kW>), dim3(bp.ngroups), dim3(kBlkThreads), 0, stream(), bd, SV{}, src,
-                     w->ctl, k);
-  hipLaunchKernelGGL(blk_combine_kernel<Fin>, dim3(gc), dim3(256), 0, stream(), bd, fin, w->ctl, k, gb, gm);
+  if (bp.ngroups) {
+    hipLaunchKernelGGL(blk_segment_kernel<kW>, dim3(bp.ngroups), dim3(kBlkThreads), 0, stream(), bd, src, w->ctl, k);
+    hipLaunchKernelGGL((blk_combine_kernel<Fin, kW, false>), gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh,
+                       gb, gm);
+  } else {
+    hipLaunchKernelGGL((blk_combine_kernel<Fin, kW, true>), gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh, gb,
+                       gm);
+  }
   if (b) OLV_HIP(hipEventRecord(b, stream()));
   OLV_HIP(hipGetLastError());
   return OLV_OK;
@@ -649,7 +630,7 @@ static int weighted_solve(const olv_graph *g, const SegDev &d, const uint32_t *r
     for (; it < stop; ++it) {
       if (bp) {
         const WprFin fin{w->buf[it & 1], w->buf[(it + 1) & 1], t, damping, 1.0f - damping};
-        OLV_TRY((enqueue_blocked<WSliceVal, true>(*bp, make_blk_dev(*bp, wp), w->buf[it & 1], fin, w, it)));
+        OLV_TRY(enqueue_blocked<true>(*bp, wp, w->buf[it & 1], fin, w, it));
       } else {
         WprOp op{ci, ws, w->buf[it & 1], w->buf[(it + 1) & 1], t, damping, 1.0f - damping};
         OLV_TRY(enqueue_iteration(d, rp, op, w, it));
@@ -666,16 +647,22 @@ static int weighted_solve(const olv_graph *g, const SegDev &d, const uint32_t *r
 // The in-CSR arrays a weighted pull runs over: the renumbered copy, or the
 // graph's own with OLV_GRAPH_ORDER.  eid: each slot's edge id.
 struct PullView {
-  SegDev d;
+  SegDev d;  // (not for the segmented pull)
   const uint32_t *rp, *ci, *eid;
-  bool relabel;
+  bool relabel, blocked;
 };
 
 static int pull_view(olv_graph *g, PrWork *w, unsigned flags, PullView *v) {
   v->relabel = (flags & OLV_GRAPH_ORDER) == 0;
+  v->blocked = v->relabel && !(flags & OLV_PR_ROW_PULL) && g->n < kIsPartial;
   if (v->relabel) {
     OLV_TRY(ensure_side(g, w, true, true));
-    v->d = make_seg_dev(w->rl.in.plan, g->tune);
+    if (v->blocked) {
+      OLV_TRY(ensure_wblocked(g, w, 0));
+    } else {
+      OLV_TRY(ensure_side_plan(g, w->rl.in));
+      v->d = make_seg_dev(w->rl.in.plan, g->tune);
+    }
     v->rp = w->rl.in.rp;
     v->ci = w->rl.in.col;
     v->eid = w->rl.in.eid;
@@ -710,8 +697,9 @@ int olv_pagerank_f32(const olv_graph *cg, float damping, uint32_t max_iters, dou
   PrWork *w = nullptr;
   OLV_TRY(get_pr_work(g, &w));
   if (relabel) OLV_TRY(ensure_side(g, w, true, false));
-  const bool blocked = relabel && !(flags & OLV_PR_ROW_PULL);
+  const bool blocked = relabel && !(flags & OLV_PR_ROW_PULL) && g->n < kIsPartial;
   if (blocked) OLV_TRY(ensure_blocked(g, w));
+  else if (relabel) OLV_TRY(ensure_side_plan(g, w->rl.in));
   const SegDev dr = make_seg_dev(relabel ? w->rl.in.plan : g->plan_in, g->tune);
   const uint32_t *rp = relabel ? w->rl.in.rp : g->in_row_ptr;
   const uint32_t *ci = relabel ? w->rl.in.col : g->in_col;
@@ -731,10 +719,9 @@ int olv_pagerank_f32(const olv_graph *cg, float damping, uint32_t max_iters, dou
   const float base = (float)((1.0 - (double)damping) / (double)g->n);
   if (blocked) {
     const BlockedPlan &bp = w->rl.blk_in;
-    const BlkDev bd = make_blk_dev(bp);
     for (uint32_t it = 0; it < max_iters; ++it)
-      OLV_TRY((enqueue_blocked<SliceVal, false>(bp, bd, w->buf[it & 1], PrFin{w->buf[(it + 1) & 1], ri, inv, damping, base},
-                                                w, it, &prof)));
+      OLV_TRY(enqueue_blocked<false>(bp, nullptr, w->buf[it & 1], PrFin{w->buf[(it + 1) & 1], ri, inv, damping, base}, w,
+                                     it, &prof));
   } else {
     for (uint32_t it = 0; it < max_iters; ++it) {
       PrOp op{ci, w->buf[it & 1], w->buf[(it + 1) & 1], ri, inv, damping, base};
@@ -775,8 +762,7 @@ int olv_pagerank_weighted_f32(const olv_graph *cg, const float *wts, const float
   OLV_TRY(get_pr_work(g, &w));
   PullView pv;
   OLV_TRY(pull_view(g, w, flags, &pv));
-  const bool blocked = pv.relabel && !(flags & OLV_PR_ROW_PULL);
-  if (blocked) OLV_TRY(ensure_wblocked(g, w, 0));
+  const bool blocked = pv.blocked;
   const bool host = (flags & OLV_PTR_HOST) != 0;
   int s = OLV_OK;
   Stage sw, st_t, so;
@@ -833,8 +819,7 @@ int olv_pagerank_jvp_f32(const olv_graph *cg, const float *wts, const float *ran
   OLV_TRY(get_pr_work(g, &w));
   PullView pv;
   OLV_TRY(pull_view(g, w, flags, &pv));
-  const bool blocked = pv.relabel && !(flags & OLV_PR_ROW_PULL);
-  if (blocked) OLV_TRY(ensure_wblocked(g, w, 0));
+  const bool blocked = pv.blocked;
   const bool host = (flags & OLV_PTR_HOST) != 0;
   int s = OLV_OK;
   Stage sw, sr, sdw, sdt, so;
@@ -848,12 +833,13 @@ int olv_pagerank_jvp_f32(const olv_graph *cg, const float *wts, const float *ran
   OLV_TRY(s);
   float *out = so.out(dranks, g->n, host, &s);
   OLV_TRY(s);
-  ScratchBuf rb, tb, dwb;  // r and dt in the new numbering; dw in slot order
+  ScratchBuf rb, tb, dwb;  // r and dt in the new numbering; dw in the solver's order
   if (pv.relabel) {
     OLV_TRY(rb.alloc(std::max<size_t>(g->n, 1) * 4));
     OLV_TRY(tb.alloc(std::max<size_t>(g->n, 1) * 4));
   }
-  OLV_TRY(dwb.alloc(std::max<size_t>(g->m, 1) * 4));
+  const BlockedPlan *bp = blocked ? &w->rl.blk_w[0] : nullptr;
+  OLV_TRY(dwb.alloc(std::max<size_t>(bp ? bp->nweights : g->m, 1) * 4));
   Timer t;
   t.start();
   if (pv.relabel) {
@@ -864,11 +850,18 @@ int olv_pagerank_jvp_f32(const olv_graph *cg, const float *wts, const float *ran
   }
   // source term s = d * dP^T r + (1-d) dt: one forward iteration with the
   // weights dw, applied to r, and the teleport dt
-  if (g->m)
-    hipLaunchKernelGGL(permute_kernel, dim3(ew_grid(g->m)), dim3(256), 0, stream(), ddw, pv.eid, g->m, dwb.as<float>());
   hipLaunchKernelGGL(ctl_init_kernel, dim3(1), dim3(256), 0, stream(), w->ctl, 0.0);
-  WprOp src_op{pv.ci, dwb.as<float>(), dr_in, w->buf[2], ddt, damping, 1.0f - damping};
-  OLV_TRY(enqueue_iteration(pv.d, pv.rp, src_op, w, 0));
+  if (blocked) {
+    OLV_TRY(enqueue_piece_weights(*bp, ddw, dwb.as<float>()));
+    const WprFin fin{dr_in, w->buf[2], ddt, damping, 1.0f - damping};
+    OLV_TRY(enqueue_blocked<true>(*bp, dwb.as<float>(), dr_in, fin, w, 0));
+  } else {
+    if (g->m)
+      hipLaunchKernelGGL(permute_kernel, dim3(ew_grid(g->m)), dim3(256), 0, stream(), ddw, pv.eid, g->m,
+                         dwb.as<float>());
+    WprOp src_op{pv.ci, dwb.as<float>(), dr_in, w->buf[2], ddt, damping, 1.0f - damping};
+    OLV_TRY(enqueue_iteration(pv.d, pv.rp, src_op, w, 0));
+  }
   // dr = d * P^T dr + s, i.e. the forward fixed point with teleport s / (1-d)
   hipLaunchKernelGGL(scale_kernel, dim3(ew_grid(g->n)), dim3(256), 0, stream(), w->buf[2], 1.0f / (1.0f - damping),
                      g->n, w->buf[3]);
@@ -909,10 +902,11 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
   OLV_TRY(get_pr_work(g, &w));
   // the out-CSR the adjoint runs over: the renumbered copy (by the segmented
   // pull unless OLV_PR_ROW_PULL) or the graph's own
-  const bool blocked = relabel && !(flags & OLV_PR_ROW_PULL);
+  const bool blocked = relabel && !(flags & OLV_PR_ROW_PULL) && g->n < kIsPartial;
   if (relabel) OLV_TRY(ensure_side(g, w, false, true));
   else OLV_TRY(ensure_plan(g, false));
   if (blocked) OLV_TRY(ensure_wblocked(g, w, 1));
+  else if (relabel) OLV_TRY(ensure_side_plan(g, w->rl.out));
   const SegDev d = make_seg_dev(relabel ? w->rl.out.plan : g->plan_out, g->tune);
   const uint32_t *rp = relabel ? w->rl.out.rp : g->row_ptr;
   const uint32_t *ci = relabel ? w->rl.out.col : g->col;
@@ -931,20 +925,15 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
   OLV_TRY(s);
   float *dl = sl.out(lambda_out, g->n, host, &s);
   OLV_TRY(s);
-  ScratchBuf rb, gb;  // r and gbar in the new numbering
-  if (relabel) {
-    OLV_TRY(rb.alloc(std::max<size_t>(g->n, 1) * 4));
-    OLV_TRY(gb.alloc(std::max<size_t>(g->n, 1) * 4));
-  }
+  ScratchBuf gb;  // gbar in the new numbering
+  if (relabel) OLV_TRY(gb.alloc(std::max<size_t>(g->n, 1) * 4));
   Timer t;
   t.start();
-  const float *wv = dw, *rv = dr, *gv = dg, *wp = nullptr;
+  const float *wv = dw, *gv = dg, *wp = nullptr;
   if (relabel) {
     if (blocked) OLV_TRY(piece_weights(w, 1, dw, w->rl.out.eid, (flags & OLV_W_UNCHANGED) != 0, host, &wp));
     else OLV_TRY(slot_weights(g, w, 1, dw, w->rl.out.eid, (flags & OLV_W_UNCHANGED) != 0, host, &wv));
-    gather_f32(dr, g->rl_order, g->n, rb.as<float>());
     gather_f32(dg, g->rl_order, g->n, gb.as<float>());
-    rv = rb.as<float>();
     gv = gb.as<float>();
   }
   // buffers 2/3 hold lambda (0/1 left free for a concurrent forward's state)
@@ -966,7 +955,7 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
       if (blocked) {
         const BlockedPlan &bp = w->rl.blk_w[1];
         const AdjFin fin{lam[it & 1], lam[(it + 1) & 1], gv, damping};
-        OLV_TRY((enqueue_blocked<WSliceVal, true>(bp, make_blk_dev(bp, wp), lam[it & 1], fin, w, it)));
+        OLV_TRY(enqueue_blocked<true>(bp, wp, lam[it & 1], fin, w, it));
       } else {
         AdjOp op{ci, wv, lam[it & 1], lam[(it + 1) & 1], gv, damping};
         OLV_TRY(enqueue_iteration(d, rp, op, w, it));
@@ -978,15 +967,15 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
   }
   const uint32_t iters = res.iters;
   const float *lf = lam[iters & 1];
+  // grad_w first: the other outputs may share memory with ranks
   if (dgw && g->m) {
-    // chunked hub rows write their edges inside the chunk blocks
-    if (relabel) {
-      GradOp<true> gop{ci, rv, lf, dgw, w->rl.out.eid, damping};
-      launch_seg(d, rp, gop, (IterCtl *)nullptr, 0u);
-    } else {
-      GradOp<false> gop{ci, rv, lf, dgw, nullptr, damping};
-      launch_seg(d, rp, gop, (IterCtl *)nullptr, 0u);
+    const float *lo = lf;  // lambda in the graph's numbering
+    if (relabel) {  // into the scratch of the renumbered gbar, which is done with
+      gather_f32(lf, g->rl_pi, g->n, gb.as<float>());
+      lo = gb.as<float>();
     }
+    hipLaunchKernelGGL(edge_grad_kernel, dim3((unsigned)(((size_t)g->m + kITile - 1) / kITile)), dim3(kIB), 0, stream(),
+                       g->row_ptr, g->col, g->n, g->m, dr, lo, damping, dgw);
   }
   if (dgt) {
     if (relabel) {

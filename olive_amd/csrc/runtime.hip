@@ -14,6 +14,7 @@
 #include "bfs_core.hpp"
 #include "device.hpp"
 #include "internal.hpp"
+#include "radix.hpp"
 
 namespace olv {
 
@@ -409,75 +410,64 @@ static void graph_free(olv_graph *g) {
   delete g;
 }
 
-int indeg_order(olv_graph *g, std::vector<uint32_t> *order_out) {
-  if (g->rl_pi) {
-    if (order_out) *order_out = g->h_rl_order;
-    return OLV_OK;
-  }
+// key[v] = maxd - in-degree of v
+__global__ void indeg_key_kernel(const uint32_t *__restrict__ irp, uint32_t n, uint32_t maxd,
+                                 uint32_t *__restrict__ key) {
+  for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
+    key[v] = maxd - (irp[v + 1] - irp[v]);
+}
+
+// inv[p[i]] = i
+__global__ void invert_kernel(const uint32_t *__restrict__ p, uint32_t n, uint32_t *__restrict__ inv) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) inv[p[i]] = i;
+}
+
+// A stable radix sort by descending in-degree on the device.
+int indeg_order(olv_graph *g) {
+  if (g->rl_pi) return OLV_OK;
   if (!g->in_row_ptr) OLV_TRY(olv_graph_build_transpose(g));
   const uint32_t n = g->n;
-  std::vector<uint32_t> in_rp((size_t)n + 1);
-  OLV_HIP(hipMemcpy(in_rp.data(), g->in_row_ptr, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost));
-  // counting sort by in-degree, descending, stable in the vertex id
-  uint32_t maxd = 0;
-  for (uint32_t v = 0; v < n; ++v) maxd = std::max(maxd, in_rp[v + 1] - in_rp[v]);
-  std::vector<uint32_t> start((size_t)maxd + 2, 0);
-  for (uint32_t v = 0; v < n; ++v) ++start[maxd - (in_rp[v + 1] - in_rp[v]) + 1];
-  for (size_t k = 1; k < start.size(); ++k) start[k] += start[k - 1];
-  std::vector<uint32_t> order(n), pi(n);
-  for (uint32_t v = 0; v < n; ++v) {
-    const uint32_t i = start[maxd - (in_rp[v + 1] - in_rp[v])]++;
-    order[i] = v;
-    pi[v] = i;
-  }
-  uint32_t *d_pi = nullptr, *d_order = nullptr;
-  int st = upload(&d_pi, pi.data(), n);
-  if (st == OLV_OK) st = upload(&d_order, order.data(), n);
-  if (st != OLV_OK) {  // leave the graph without a half-built numbering
-    if (d_pi) (void)hipFree(d_pi);
-    if (d_order) (void)hipFree(d_order);
-    return st;
-  }
-  g->rl_pi = d_pi;
-  g->rl_order = d_order;
-  g->h_rl_pi = std::move(pi);
-  g->h_rl_order = std::move(order);
-  if (order_out) *order_out = g->h_rl_order;
+  DevBuf pi, order;  // published once complete
+  OLV_TRY(pi.alloc((size_t)n * 4));
+  OLV_TRY(order.alloc((size_t)n * 4));
+  ScratchBuf key;
+  OLV_TRY(key.alloc((size_t)n * 4));
+  hipLaunchKernelGGL(indeg_key_kernel, dim3(fill_grid(n)), dim3(256), 0, stream(), g->in_row_ptr, n, g->max_indeg,
+                     key.as<uint32_t>());
+  SortBufs b;
+  OLV_TRY(radix_sort<uint32_t>(key.as<uint32_t>(), LoadIndex{}, n, bits_for(g->max_indeg + 1), b));
+  OLV_HIP(hipMemcpyAsync(order.p, b.vals<uint32_t>(), (size_t)n * 4, hipMemcpyDeviceToDevice, stream()));
+  hipLaunchKernelGGL(invert_kernel, dim3(fill_grid(n)), dim3(256), 0, stream(), order.as<uint32_t>(), n,
+                     pi.as<uint32_t>());
+  OLV_HIP(hipGetLastError());
+  OLV_HIP(hipStreamSynchronize(stream()));
+  g->rl_pi = pi.as<uint32_t>();
+  g->rl_order = order.as<uint32_t>();
+  pi.p = order.p = nullptr;
   return OLV_OK;
 }
 
-// s[e] = pi[u], d[e] = pi[col[e]] for every edge e = (u, col[e]); one wave
-// per row.
-__global__ void coo_relabel_kernel(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
-                                   const uint32_t *__restrict__ pi, uint32_t n, uint32_t *__restrict__ s,
-                                   uint32_t *__restrict__ d) {
-  const uint32_t waves = gridDim.x * (blockDim.x / kWave);
-  const uint32_t lane = threadIdx.x % kWave;
-  for (uint32_t u = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; u < n; u += waves) {
-    const uint32_t b = rp[u], e = rp[u + 1], pu = pi[u];
-    for (uint32_t k0 = b + lane; k0 < e; k0 += 4 * kWave) {  // four loads in flight per lane
-      uint32_t c[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] = k0 + i * kWave < e ? col[k0 + i * kWave] : 0u;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (k0 + i * kWave < e) {
-          s[k0 + i * kWave] = pu;
-          d[k0 + i * kWave] = pi[c[i]];
-        }
-    }
+// s[e] = pi[row[e]] (in place), d[e] = pi[col[e]] for every edge e.
+__global__ void coo_relabel_kernel(const uint32_t *__restrict__ col, const uint32_t *__restrict__ pi, uint32_t m,
+                                   uint32_t *__restrict__ s, uint32_t *__restrict__ d) {
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < m; e += (size_t)gridDim.x * blockDim.x) {
+    s[e] = pi[s[e]];
+    d[e] = pi[col[e]];
   }
 }
 
 int ensure_twin(olv_graph *g) {
   if (g->twin) return OLV_OK;
-  OLV_TRY(indeg_order(g, nullptr));
+  OLV_TRY(indeg_order(g));
+  std::vector<uint32_t> h_pi(g->n);
+  OLV_HIP(hipMemcpy(h_pi.data(), g->rl_pi, (size_t)g->n * 4, hipMemcpyDeviceToHost));
   ScratchBuf s, d;
   OLV_TRY(s.alloc(std::max<size_t>(g->m, 1) * 4));
   OLV_TRY(d.alloc(std::max<size_t>(g->m, 1) * 4));
   if (g->m) {
-    hipLaunchKernelGGL(coo_relabel_kernel, dim3(fill_grid((size_t)g->n * kWave)), dim3(256), 0, stream(), g->row_ptr,
-                       g->col, g->rl_pi, g->n, s.as<uint32_t>(), d.as<uint32_t>());
+    OLV_TRY(slot_rows(g->row_ptr, g->n, g->m, s.as<uint32_t>()));
+    hipLaunchKernelGGL(coo_relabel_kernel, dim3(fill_grid(g->m)), dim3(256), 0, stream(), g->col, g->rl_pi, g->m,
+                       s.as<uint32_t>(), d.as<uint32_t>());
     OLV_HIP(hipGetLastError());
   }
   olv_graph *t = nullptr;
@@ -486,6 +476,7 @@ int ensure_twin(olv_graph *g) {
   OLV_HIP(hipStreamSynchronize(stream()));
   t->device = g->device;
   t->out_map = g->rl_order;
+  g->h_rl_pi = std::move(h_pi);
   g->twin = t;
   return OLV_OK;
 }
