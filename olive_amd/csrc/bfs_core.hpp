@@ -158,15 +158,19 @@ __device__ void push_expand(const uint32_t *queue, uint32_t qsize, const uint2 *
     if (threadIdx.x == 0) insp += end - beg;
     visit_range<U>(vis, beg + threadIdx.x, end, BLOCK, pl);
   }
-  // Queue entries per workgroup and pass: a full workgroup's worth when the
-  // queue fills the grid, else an even share, so that a short queue of
-  // high-degree vertices is not left to the first workgroup.
-  const uint32_t per = qsize >= nvb * BLOCK ? BLOCK : (qsize + nvb - 1) / nvb;
-  for (uint32_t base = vb * per; base < qsize; base += nvb * per) {
-    const uint32_t i = base + threadIdx.x;
+  // Queue entries are dealt to the workgroups in runs of 2^lg consecutive
+  // entries (16, one line, when there are enough), not in one block each: a
+  // queue is about in vertex order and neighbouring vertices are alike, so
+  // the first workgroups of an RMAT frontier would hold most of its edges.
+  const uint32_t lg = qsize >= 16 * nvb ? 4u : (qsize >= 4 * nvb ? 2u : 0u);
+  const uint32_t runs = (qsize + (1u << lg) - 1) >> lg;
+  const uint32_t per = ((runs + nvb - 1) / nvb) << lg;  // entries of a workgroup
+  for (uint32_t base = 0; base < per; base += BLOCK) {
+    const uint32_t j = base + threadIdx.x;
+    const uint64_t i = (((uint64_t)(j >> lg) * nvb + vb) << lg) + (j & ((1u << lg) - 1));
     uint32_t beg = 0, end = 0;
     P pl{};
-    if (threadIdx.x < per && i < qsize) {
+    if (j < per && i < qsize) {
       const uint32_t q = queue[i];
       const uint32_t u = vis.row(q);
       beg = row_ptr[u];

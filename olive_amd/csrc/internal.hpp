@@ -69,6 +69,7 @@ constexpr uint32_t kHubThrMin = 256;  // smallest hub item (sizes the hub item b
 
 struct BfsWork;   // bfs.hip
 struct PrWork;    // pagerank.hip
+struct SsspWork;     // sssp.hip
 struct SsspBinWork;  // sssp_bin.hip
 
 }  // namespace olv
@@ -94,6 +95,7 @@ struct olv_graph {
   bool plan_in_ready = false, plan_out_ready = false;
   olv::BfsWork *bfs = nullptr;
   olv::PrWork *pr = nullptr;
+  olv::SsspWork *sssp = nullptr;         // direct SSSP work (for the last k sources)
   olv::SsspBinWork *sssp_bin = nullptr;  // binned SSSP work (for the last k sources)
   // In-degree numbering: vertices by descending in-degree, ties by id
   // (built on first use; shared by the PageRank pull and the BFS twin).
@@ -134,10 +136,12 @@ void free_bfs_work(olv_graph *g);
 int noalloc_scratch(unsigned char **out);
 void free_pr_work(olv_graph *g);
 void free_sssp_bin(olv_graph *g);
-// Binned SSSP (sssp_bin.hip) for k instances from device sources; *used =
-// false when the graph does not fit it (the caller then relaxes directly).
+void free_sssp_work(olv_graph *g);
+// Binned SSSP (sssp_bin.hip): whether k instances of g take it, and its run
+// from device sources.
+bool sssp_bin_fits(const olv_graph *g, uint32_t k);
 int sssp_bin_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, const int32_t *weights, int32_t *dist,
-                 int32_t delta, unsigned flags, olv_stats *st, bool *used);
+                 int32_t delta, unsigned flags, olv_stats *st);
 
 // RAII device buffer for temporaries inside an entry point.
 struct DevBuf {

@@ -12,13 +12,19 @@
 //
 // Near-far ordering (Davidson et al., IPDPS'14): with a split distance T, an
 // improved vertex joins the next round's frontier only if its new distance
-// is below T; otherwise its bit goes to a far bitmap.  When the near
-// frontier runs dry, T grows by delta and the far vertices now below T (read
-// from dist) form the next frontier.  Vertices are then mostly expanded once
-// with their final distance instead of once per improvement, and the fixed
-// point -- hence every distance -- is the same.  Negative weights turn the
-// ordering off (plain rounds, so the reference's n-round negative-cycle rule
-// applies unchanged).
+// is below T; otherwise it stays marked.  When the near frontier runs dry, T
+// moves to the smallest marked distance + delta (never an empty promotion)
+// and the marked vertices below it form the next frontier.  Vertices are then
+// mostly expanded once with their final distance instead of once per
+// improvement, and the fixed point -- hence every distance -- is the same.
+// Negative weights turn the ordering off (plain rounds, so the reference's
+// n-round negative-cycle rule applies unchanged).
+//
+// A vertex whose distance dropped is marked with a plain byte store: the
+// bitmap atomics that marked it before cost as much as the distance atomics
+// and serialised on the words of an RMAT graph's hubs, and extracting a
+// frontier from them took a lane per 32 vertices (16-28 us per large round;
+// 5-7 from the bytes).
 //
 // k sources run as k instances over one shared CSR: instance s owns virtual
 // vertices s*n .. s*n+n-1 (dist row s), so one launch per round relaxes all
@@ -29,6 +35,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstddef>
 #include <cstring>
 #include <type_traits>
 #include <vector>
@@ -41,20 +48,34 @@ namespace olv {
 constexpr int kSBlock = 256;
 constexpr uint32_t kSSpin = 1u << 24;
 
-template <bool Multi>
+// A marked vertex has a distance not expanded yet: kMarkNew, lowered since the
+// last compaction; kMarkFar, at or above the split then.
+constexpr uint8_t kMarkNew = 1, kMarkFar = 2;
+
+// Candidate copies.  A relaxation probes dist and lowers a candidate kept
+// apart from it: an atomic is performed at the memory side and takes the line
+// from the caches that the other relaxations probe.  Atomics to one address
+// also serialise there (about 12 ns each), and in a large round of an RMAT
+// graph many relaxations improve on the same hub, so workgroup b lowers copy
+// b % kCopies; the compaction, a launch later, takes the smallest of a marked
+// vertex's copies.  RMAT 250K x 4M: 601 us lowering dist itself, 502, 474, 452,
+// 455 with 1, 2, 4, 8 copies; RMAT 1M x 16M: 1095 and 959.  Past 1M vertices
+// the copies no longer stay cached (2M x 16M: 1458 and 1418; 4M x 32M: 1532
+// and 2040), so relaxations lower dist there.
+constexpr uint32_t kCopies = 4;
+constexpr uint64_t kCopiesMaxVertices = 1u << 20;
+
+template <bool Multi, bool Copies>
 struct SsspVisitor {
   using P = typename std::conditional<Multi, unsigned long long, int32_t>::type;
   const uint32_t *col;
   const int32_t *w;
-  int32_t *dist;
-  uint32_t *next_bm;
-  uint32_t *far_bm;  // nullptr: plain rounds
-  int32_t split;     // near-far split distance T
+  const int32_t *dist;
+  int32_t *low;  // what relaxations lower: dist, or this workgroup's copy of the candidates
+  uint8_t *mark;
   uint32_t n;
-  uint32_t nf = 0;
-  __device__ SsspVisitor(const uint32_t *c, const int32_t *ww, int32_t *d, uint32_t *nb, uint32_t *fb, int32_t t,
-                         uint32_t nn)
-      : col(c), w(ww), dist(d), next_bm(nb), far_bm(fb), split(t), n(nn) {}
+  __device__ SsspVisitor(const uint32_t *c, const int32_t *ww, const int32_t *d, int32_t *lo, uint8_t *mk, uint32_t nn)
+      : col(c), w(ww), dist(d), low(lo), mark(mk), n(nn) {}
   __device__ __forceinline__ uint32_t row(uint32_t q) const { return Multi ? q % n : q; }
   __device__ __forceinline__ P load(uint32_t q) const {
     if constexpr (Multi)
@@ -76,40 +97,42 @@ struct SsspVisitor {
     return make_uint2(base + col[e], (uint32_t)du + (uint32_t)w[e]);
   }
   __device__ __forceinline__ int32_t state(uint2 t) const { return dist[t.x]; }
-  // Relax: lower dist[v] and mark v.  Both atomics are non-returning (no
-  // lane waits on them): a relaxation that loses a race to a lower distance
-  // still marks v, which only re-expands v with its final distance, and nf
-  // may count a vertex more than once -- it only has to be non-zero exactly
-  // when something improved.
+  // Relax: lower v and mark it.  No lane waits on the atomic: a relaxation
+  // that loses a race to a lower distance still marks v, which only re-expands
+  // v with its final distance.
   __device__ __forceinline__ void apply(uint2 t, int32_t cur, P) {
-    const uint32_t v = t.x;
     const int32_t cand = (int32_t)t.y;
     if (cand >= cur) return;
-    __hip_atomic_fetch_min(&dist[v], cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const uint32_t bit = 1u << (v & 31);
-    uint32_t *bm = (far_bm && cand >= split) ? far_bm : next_bm;
-    __hip_atomic_fetch_or(&bm[v >> 5], bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (bm == next_bm) nf += 1;
+    __hip_atomic_fetch_min(&low[t.x], cand, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    mark[t.x] = kMarkNew;
   }
 };
 
+enum : uint32_t { kModeNear = 0, kModeResplit = 1, kModeDone = 2 };
+
+// Smallest marked distance at or above the split, one copy per 128-byte line
+// (workgroup b updates copy b % kCtrSlots).
+struct alignas(128) MinSlot {
+  int32_t v;
+  uint32_t pad[31];
+};
+
 struct SsspCtl {
-  uint32_t round;     // next round to relax (written by compact)
-  uint32_t round_e;   // round being compacted (written by relax)
   uint32_t done;
   uint32_t rounds;    // result
-  uint32_t capped;    // result: n rounds without convergence
+  uint32_t capped;    // result: max_rounds without convergence
+  uint32_t round;     // next round to relax (written by compact)
+  uint32_t round_e;   // round being compacted (written by relax)
   uint32_t pad;
+  unsigned long long relax;  // result: edges read
+  uint32_t mode[2];   // mode of round R, slot R & 1
+  int32_t split[2];   // split that the frontier of round R was built with
   uint32_t qfill[2];  // frontier queue length of round R, slot R & 1
   uint32_t hfill[2];  // hub items of round R, slot R & 1
-  unsigned long long relax;  // result: edges read
-  int32_t split[2];   // near-far split T of round R, slot R & 1
-  uint32_t promo[2];  // round R's frontier came from the far bitmap
-  uint32_t kept[2];   // far bits left by the promotion that built round R
-  uint32_t phases;    // result: near-far phases
-  uint32_t pad2;
-  CtrSet cnt[3];
+  MinSlot minfar[2][kCtrSlots];
+  CtrSet cnt[2];      // edges read by round R, slot R & 1
 };
+constexpr size_t kSsspCtlHead = offsetof(SsspCtl, mode);  // what the host reads back
 
 struct SsspParams {
   const uint32_t *row_ptr;
@@ -118,12 +141,12 @@ struct SsspParams {
   int32_t *dist;     // ninst x n
   uint32_t *queue;   // virtual ids
   uint2 *hubs;       // hub items (virtual id, chunk)
-  uint32_t *bms;     // 2 x nwp
+  uint8_t *mark;     // one byte per vertex (padded to 4): kMarkNew, kMarkFar or 0
+  int32_t *cand;     // kCopies x nv candidates, or nullptr: relaxations lower dist
   SsspCtl *ctl;
   GridBar *bar;
-  uint32_t *far_bm;  // nwp words, or nullptr for plain rounds
   int32_t delta;     // near-far step (0: plain rounds)
-  uint32_t n, ninst, nw, nwp;
+  uint32_t n, ninst, nv;
   uint32_t wave_thr, block_thr, hub_thr;
   uint32_t max_rounds;
 };
@@ -134,102 +157,142 @@ struct ModRow {
   __device__ __forceinline__ uint32_t operator()(uint32_t v) const { return v % n; }
 };
 
-template <bool Multi>
-__device__ __forceinline__ void sssp_round(const SsspParams &p, uint32_t qsize, uint32_t nhubs, uint32_t *nextb,
-                                           int32_t split, uint32_t vb, uint32_t nvb, uint32_t &nf,
-                                           unsigned long long &insp) {
-  SsspVisitor<Multi> vis(p.col, p.w, p.dist, nextb, p.far_bm, split, p.n);
+template <bool Multi, bool Copies>
+__device__ __forceinline__ void sssp_round(const SsspParams &p, uint32_t qsize, uint32_t nhubs, uint32_t vb,
+                                           uint32_t nvb, unsigned long long &insp) {
+  SsspVisitor<Multi, Copies> vis(p.col, p.w, p.dist, Copies ? p.cand + (size_t)(vb % kCopies) * p.nv : p.dist, p.mark,
+                               p.n);
   push_expand<kSBlock>(p.queue, qsize, p.hubs, nhubs, p.row_ptr, p.wave_thr, p.block_thr, p.hub_thr, vb, nvb, vis,
                        insp);
-  nf += vis.nf;
 }
 
-template <bool Multi>
+// Marked vertices with a distance below `split` -> queue and hub items (their
+// marks cleared); the smallest other marked distance -> *minfar.  A lane
+// takes the mark bytes of four vertices.
+template <int BLOCK>
+__device__ void sssp_take(const SsspParams &p, int32_t split, uint32_t *qcount, uint32_t *hcount, int32_t *minfar,
+                          uint32_t vb, uint32_t nvb) {
+  __shared__ uint32_t s_scan[BLOCK / kWave + 1];
+  __shared__ uint32_t s_base;
+  __shared__ int32_t s_mf[BLOCK / kWave];
+  const ModRow row{p.n};
+  const uint32_t nw = (p.nv + 3) / 4;
+  uint32_t *words = reinterpret_cast<uint32_t *>(p.mark);
+  int32_t mf = kInf;
+  for (uint32_t w0 = vb * BLOCK; w0 < nw; w0 += nvb * BLOCK) {
+    const uint32_t w = w0 + threadIdx.x;
+    const uint32_t word = w < nw ? words[w] : 0u;
+    uint32_t keep = word, take = 0;  // take: bit b, vertex 4 w + b goes to the queue
+    if (word) {
+      int32_t d[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) d[b] = (word >> (8 * b)) & 0xffu ? p.dist[w * 4u + b] : kInf;
+      if (p.cand) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          if (((word >> (8 * b)) & 0xffu) != kMarkNew) continue;
+          int32_t c[kCopies], m = d[b];
+#pragma unroll
+          for (uint32_t x = 0; x < kCopies; ++x) c[x] = p.cand[(size_t)x * p.nv + w * 4u + b];
+#pragma unroll
+          for (uint32_t x = 0; x < kCopies; ++x) m = c[x] < m ? c[x] : m;
+          if (m < d[b]) p.dist[w * 4u + b] = d[b] = m;
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (!((word >> (8 * b)) & 0xffu)) continue;
+        keep &= ~(0xffu << (8 * b));
+        if (d[b] >= split) {
+          mf = d[b] < mf ? d[b] : mf;
+          keep |= (uint32_t)kMarkFar << (8 * b);
+          continue;
+        }
+        const uint32_t x = w * 4u + b, u = p.ninst > 1 ? row(x) : x;
+        const uint32_t deg = p.row_ptr[u + 1] - p.row_ptr[u];
+        if (deg >= p.hub_thr) {
+          const uint32_t k = (deg + p.hub_thr - 1) / p.hub_thr;
+          const uint32_t hb = atomicAdd(hcount, k);
+          for (uint32_t j = 0; j < k; ++j) p.hubs[hb + j] = make_uint2(x, j);
+        } else {
+          take |= 1u << b;
+        }
+      }
+      if (keep != word) words[w] = keep;
+    }
+    uint32_t total;
+    const uint32_t off = block_exclusive_scan<BLOCK>((uint32_t)__popc(take), s_scan, &total);
+    if (threadIdx.x == 0) s_base = total ? atomicAdd(qcount, total) : 0u;
+    __syncthreads();
+    uint32_t pos = s_base + off;
+    for (uint32_t x = take; x; x &= x - 1) p.queue[pos++] = w * 4u + __ffs(x) - 1;
+    __syncthreads();
+  }
+  mf = wave_min(mf);
+  if (lane_id() == 0) s_mf[threadIdx.x / kWave] = mf;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int i = 1; i < BLOCK / kWave; ++i) mf = s_mf[i] < mf ? s_mf[i] : mf;
+    if (mf < kInf) atomicMin(minfar, mf);
+  }
+}
+
+// Round R: decide from the frontier that the last compaction built (its
+// vertices, or none: re-split past the smallest marked distance, or done) and
+// relax it.
+template <bool Multi, bool Copies>
 __global__ void __launch_bounds__(kSBlock) sssp_relax_kernel(SsspParams p) {
   SsspCtl *ctl = p.ctl;
   if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-  const uint32_t R = ctl->round;
+  const uint32_t R = ctl->round, t = threadIdx.x;
   const uint32_t qsize = ctl->qfill[R & 1], nhubs = ctl->hfill[R & 1];
-  uint32_t *nextb = p.bms + (size_t)(R & 1) * p.nwp;
-  uint32_t *clearb = p.bms + (size_t)((R + 1) & 1) * p.nwp;
-  for (uint32_t i = blockIdx.x * kSBlock + threadIdx.x; i < p.nwp; i += gridDim.x * kSBlock) clearb[i] = 0u;
   if (blockIdx.x == 0) {
-    if (threadIdx.x == 0) {
+    __shared__ int32_t s_mf;
+    if (t < kWave) {
+      const int32_t mf = wave_min(t < kCtrSlots ? ctl->minfar[R & 1][t].v : kInf);
+      if (t == 0) s_mf = mf;
+    }
+    __syncthreads();
+    if (t == 0) {
+      const uint32_t mode = (qsize + nhubs) ? kModeNear : (s_mf < kInf ? kModeResplit : kModeDone);
+      const int32_t split = ctl->split[R & 1];
       ctl->round_e = R;
+      ctl->mode[R & 1] = mode;
+      ctl->split[(R + 1) & 1] = mode == kModeNear ? split : (s_mf > kInf - p.delta ? kInf : s_mf + p.delta);
       ctl->qfill[(R + 1) & 1] = 0;
       ctl->hfill[(R + 1) & 1] = 0;
-      ctl->kept[(R + 1) & 1] = 0;
+      if (mode == kModeDone || R >= p.max_rounds) {
+        ctl->rounds = R;
+        ctl->capped = mode != kModeDone;
+        ctl->done = 1u;
+      }
     }
-    ctr_clear(&ctl->cnt[(R + 1) % 3]);
+    if (t < kCtrSlots) ctl->minfar[(R + 1) & 1][t].v = kInf;
   }
-  uint32_t nf = 0;
+  if (qsize + nhubs == 0 || R >= p.max_rounds) return;
   unsigned long long insp = 0;
-  sssp_round<Multi>(p, qsize, nhubs, nextb, ctl->split[R & 1], blockIdx.x, gridDim.x, nf, insp);
-  flush_counters<kSBlock>(&ctl->cnt[R % 3], nf, 0ull, insp);
+  sssp_round<Multi, Copies>(p, qsize, nhubs, blockIdx.x, gridDim.x, insp);
+  flush_counters<kSBlock>(&ctl->cnt[R & 1], 0u, 0ull, insp);
 }
 
 __global__ void __launch_bounds__(kSBlock) sssp_compact_kernel(SsspParams p) {
   SsspCtl *ctl = p.ctl;
   if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
   const uint32_t R = ctl->round_e;
-  const CtrSum c = ctr_total(&ctl->cnt[R % 3]);
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  if (lead) ctl->relax += c.inspected;
-  const int32_t split = ctl->split[R & 1];
-  // near frontier dry: finished in plain mode, or when the far bitmap was
-  // found empty by the promotion that built this round's (empty) frontier
-  const bool dry = c.nf == 0;
-  const bool finished =
-      dry && (p.delta == 0 || (ctl->promo[R & 1] && ctl->qfill[R & 1] == 0 && ctl->hfill[R & 1] == 0 &&
-                               ctl->kept[R & 1] == 0));
-  if (finished || R + 1 >= p.max_rounds) {
-    if (lead) {
-      ctl->rounds = R + 1;
-      ctl->capped = !finished;
-      ctl->done = 1u;
-    }
-    return;
-  }
-  if (!dry) {
-    if (lead) {
-      ctl->split[(R + 1) & 1] = split;
-      ctl->promo[(R + 1) & 1] = 0;
+  if (blockIdx.x == 0) {
+    const CtrSum c = ctr_total(&ctl->cnt[R & 1]);
+    if (threadIdx.x == 0) {
+      ctl->relax += c.inspected;
       ctl->round = R + 1;
     }
-    compact_step<kSBlock>(p.bms + (size_t)(R & 1) * p.nwp, p.nw, p.row_ptr, p.hub_thr, p.queue,
-                          &ctl->qfill[(R + 1) & 1], p.hubs, &ctl->hfill[(R + 1) & 1], blockIdx.x, gridDim.x,
-                          ModRow{p.n});
-    return;
+    ctr_clear(&ctl->cnt[(R + 1) & 1]);
   }
-  // promotion: T += delta; far vertices now below T become the frontier
-  const int32_t nsplit = split > kInf - p.delta ? kInf : split + p.delta;
-  if (lead) {
-    ctl->split[(R + 1) & 1] = nsplit;
-    ctl->promo[(R + 1) & 1] = 1;
-    ctl->phases += 1;
-    ctl->round = R + 1;
-  }
-  uint32_t kept = 0;
-  const int32_t *dist = p.dist;
-  uint32_t *far = p.far_bm;
-  auto take = [&](uint32_t w) -> uint32_t {
-    const uint32_t word = far[w];
-    uint32_t sel = 0;
-    for (uint32_t x = word; x; x &= x - 1) {
-      const uint32_t b = __ffs(x) - 1;
-      if (dist[w * 32u + b] < nsplit) sel |= 1u << b;
-    }
-    if (sel) far[w] = word & ~sel;
-    kept += __popc(word & ~sel);
-    return sel;
-  };
-  compact_words<kSBlock>(p.nw, take, p.row_ptr, p.hub_thr, p.queue, &ctl->qfill[(R + 1) & 1], p.hubs,
-                         &ctl->hfill[(R + 1) & 1], blockIdx.x, gridDim.x, ModRow{p.n});
-  __shared__ unsigned long long s_red[kSBlock / kWave];
-  const unsigned long long tk = block_sum<kSBlock, unsigned long long>(kept, s_red);
-  if (threadIdx.x == 0 && tk) atomicAdd(&ctl->kept[(R + 1) & 1], (uint32_t)tk);
+  sssp_take<kSBlock>(p, ctl->split[(R + 1) & 1], &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1],
+                     &ctl->minfar[(R + 1) & 1][blockIdx.x % kCtrSlots].v, blockIdx.x, gridDim.x);
 }
 
+// All rounds (plain: every marked vertex is expanded) in one cooperative
+// launch.
 template <bool Multi>
 __global__ void __launch_bounds__(kSBlock) sssp_persistent_kernel(SsspParams p) {
   GridBarLocal gb;
@@ -237,52 +300,55 @@ __global__ void __launch_bounds__(kSBlock) sssp_persistent_kernel(SsspParams p) 
   SsspCtl *ctl = p.ctl;
   const uint32_t vb = blockIdx.x, nvb = gridDim.x;
   const bool lead = vb == 0 && threadIdx.x == 0;
-  unsigned long long insp_all = 0;
+  unsigned long long insp = 0;
   for (uint32_t R = 0;; ++R) {
-    uint32_t *nextb = p.bms + (size_t)(R & 1) * p.nwp;
-    uint32_t *clearb = p.bms + (size_t)((R + 1) & 1) * p.nwp;
     const uint32_t qsize = __hip_atomic_load(&ctl->qfill[R & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t nhubs = __hip_atomic_load(&ctl->hfill[R & 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (uint32_t i = vb * kSBlock + threadIdx.x; i < p.nwp; i += nvb * kSBlock) clearb[i] = 0u;
-    if (vb == 0) {
-      if (threadIdx.x == 0) {
-        ctl->qfill[(R + 1) & 1] = 0;
-        ctl->hfill[(R + 1) & 1] = 0;
-      }
-      ctr_clear(&ctl->cnt[(R + 1) % 3]);
-    }
-    uint32_t nf = 0;
-    unsigned long long insp = 0;
-    sssp_round<Multi>(p, qsize, nhubs, nextb, kInf, vb, nvb, nf, insp);
-    flush_counters<kSBlock>(&ctl->cnt[R % 3], nf, 0ull, insp);
-    if (!grid_barrier(p.bar, gb, kSSpin)) break;
-    const CtrSum c = ctr_total(&ctl->cnt[R % 3]);
-    insp_all += c.inspected;
-    if (c.nf == 0 || R + 1 >= p.max_rounds) {
+    if (qsize + nhubs == 0 || R >= p.max_rounds) {
       if (lead) {
-        ctl->rounds = R + 1;
-        ctl->capped = c.nf != 0;
-        ctl->relax = insp_all;
+        ctl->rounds = R;
+        ctl->capped = qsize + nhubs != 0;
         ctl->done = 1u;
       }
       break;
     }
-    compact_step<kSBlock>(nextb, p.nw, p.row_ptr, p.hub_thr, p.queue, &ctl->qfill[(R + 1) & 1], p.hubs,
-                          &ctl->hfill[(R + 1) & 1], vb, nvb, ModRow{p.n});
+    if (lead) {
+      ctl->qfill[(R + 1) & 1] = 0;
+      ctl->hfill[(R + 1) & 1] = 0;
+    }
+    sssp_round<Multi, false>(p, qsize, nhubs, vb, nvb, insp);
+    if (!grid_barrier(p.bar, gb, kSSpin)) break;
+    sssp_take<kSBlock>(p, kInf, &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1], &ctl->minfar[0][vb % kCtrSlots].v, vb,
+                       nvb);
     if (!grid_barrier(p.bar, gb, kSSpin)) break;
   }
+  __shared__ unsigned long long s_red[kSBlock / kWave];
+  const unsigned long long total = block_sum<kSBlock, unsigned long long>(insp, s_red);
+  if (threadIdx.x == 0 && total) atomicAdd(&ctl->relax, total);
 }
 
-// dist = INF, bitmaps (near x2, far)/control/barrier = 0, split = delta.
-__global__ void sssp_reset_kernel(int32_t *__restrict__ dist, size_t total, uint32_t *__restrict__ bms,
-                                  uint32_t nwp, SsspCtl *__restrict__ ctl, GridBar *__restrict__ bar, int32_t delta) {
+// dist and candidates = INF, marks/control/barrier = 0, minfar = INF, split = delta.  With a
+// single source (k == 1: src) the seeding is done here as well -- its
+// distance by the lane that owns it, the frontier by workgroup 0 after
+// clearing the control block -- one launch instead of two.
+__global__ void sssp_reset_kernel(SsspParams p, uint32_t src) {
   const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = tid; i < total; i += stride) dist[i] = kInf;
-  for (size_t i = tid; i < (size_t)nwp * 3; i += stride) bms[i] = 0u;
-  for (size_t i = tid; i < sizeof(SsspCtl) / 4; i += stride) reinterpret_cast<uint32_t *>(ctl)[i] = 0u;
-  for (size_t i = tid; i < sizeof(GridBar) / 4; i += stride) reinterpret_cast<uint32_t *>(bar)[i] = 0u;
-  if (tid == 0) ctl->split[0] = delta > 0 ? delta : kInf;
+  const bool one = p.ninst == 1;
+  for (size_t i = tid; i < p.nv; i += stride) p.dist[i] = one && i == src ? 0 : kInf;
+  for (size_t i = tid; i < ((size_t)p.nv + 3) / 4; i += stride) reinterpret_cast<uint32_t *>(p.mark)[i] = 0u;
+  if (p.cand)
+    for (size_t i = tid; i < (size_t)p.nv * kCopies; i += stride) p.cand[i] = kInf;
+  if (blockIdx.x != 0) return;
+  for (uint32_t i = threadIdx.x; i < sizeof(SsspCtl) / 4; i += blockDim.x) reinterpret_cast<uint32_t *>(p.ctl)[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < sizeof(GridBar) / 4; i += blockDim.x) reinterpret_cast<uint32_t *>(p.bar)[i] = 0u;
+  __syncthreads();
+  if (threadIdx.x < 2 * kCtrSlots) p.ctl->minfar[threadIdx.x / kCtrSlots][threadIdx.x % kCtrSlots].v = kInf;
+  if (threadIdx.x == 0) p.ctl->split[0] = p.delta > 0 ? p.delta : kInf;
+  if (!one) return;
+  unsigned long long deg;
+  seed_frontier(&src, 1u, p.row_ptr, p.hub_thr, p.queue, &p.ctl->qfill[0], p.hubs, &p.ctl->hfill[0],
+                [&](uint32_t) -> uint32_t { return src; }, ModRow{p.n}, &deg);
 }
 
 // One workgroup: instance s starts from virtual vertex s*n + srcs[s].
@@ -297,30 +363,55 @@ __global__ void sssp_seed_kernel(const uint32_t *__restrict__ srcs, uint32_t k, 
                 ModRow{p.n}, &deg);
 }
 
+// Work arrays for k instances, kept on the graph for the next call with the
+// same k (allocating them took 0.35 ms of every call).
 struct SsspWork {
-  uint32_t nw = 0, nwp = 0;
-  uint32_t *queue = nullptr, *bms = nullptr;
+  uint32_t k = 0;
+  uint32_t *queue = nullptr;
+  uint8_t *mark = nullptr;
+  int32_t *cand = nullptr;
   uint2 *hubs = nullptr;
   SsspCtl *ctl = nullptr, *h_ctl = nullptr;
   GridBar *bar = nullptr;
   ~SsspWork() {
-    void *ps[] = {queue, bms, hubs, ctl, bar};
+    void *ps[] = {queue, mark, cand, hubs, ctl, bar};
     for (void *p : ps)
       if (p) (void)hipFree(p);
     if (h_ctl) (void)hipHostFree(h_ctl);
   }
-  int alloc(uint64_t nv, uint32_t k, uint64_t m) {
-    nw = (uint32_t)((nv + 31) / 32);
-    nwp = (nw + 63) / 64 * 64;
+  int alloc(uint64_t nv, uint32_t kk, uint64_t m) {
+    k = kk;
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&queue), (size_t)nv * 4));
+    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&mark), ((size_t)nv + 3) / 4 * 4));
+    if (nv <= kCopiesMaxVertices) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&cand), (size_t)nv * kCopies * 4));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&hubs), hub_capacity(m) * k * sizeof(uint2)));
-    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&bms), (size_t)nwp * 12));  // near x2, far
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&ctl), sizeof(SsspCtl)));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&bar), sizeof(GridBar)));
     OLV_HIP(hipHostMalloc(reinterpret_cast<void **>(&h_ctl), sizeof(SsspCtl), hipHostMallocDefault));
     return OLV_OK;
   }
 };
+
+void free_sssp_work(olv_graph *g) {
+  delete g->sssp;
+  g->sssp = nullptr;
+}
+
+// The graph's work for k instances, published once complete.
+static int get_sssp_work(olv_graph *g, uint32_t k, SsspWork **out) {
+  if (!g->sssp || g->sssp->k != k) {
+    free_sssp_work(g);
+    SsspWork *w = new SsspWork();
+    const int rc = w->alloc((uint64_t)k * g->n, k, g->m);
+    if (rc != OLV_OK) {
+      delete w;
+      return rc;
+    }
+    g->sssp = w;
+  }
+  *out = g->sssp;
+  return OLV_OK;
+}
 
 static unsigned sgrid(size_t items, size_t per) {
   size_t b = (items + per - 1) / per;
@@ -391,55 +482,56 @@ static int sssp_delta(const olv_graph *g, const int32_t *w, int32_t *delta) {
 }
 
 static int sssp_read(SsspWork &w) {
-  OLV_HIP(hipMemcpyAsync(w.h_ctl, w.ctl, sizeof(SsspCtl), hipMemcpyDeviceToHost, stream()));
+  OLV_HIP(hipMemcpyAsync(w.h_ctl, w.ctl, kSsspCtlHead, hipMemcpyDeviceToHost, stream()));
   OLV_HIP(hipStreamSynchronize(stream()));
   return OLV_OK;
 }
 
-// k instances from device sources d_srcs[0..k); dist is k x n.
-static int sssp_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, const int32_t *weights, int32_t *dist,
+// k instances from the host sources srcs[0..k); dist is k x n.
+static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const int32_t *weights, int32_t *dist,
                     unsigned flags, olv_stats *st) {
   const uint64_t nv = (uint64_t)k * g->n;
   if (nv >= (1ull << 32)) return fail(OLV_ERANGE, "sssp: %u sources x %u vertices exceed 2^32 ids", k, g->n);
   const bool multi = k > 1;
+  olv_graph *gm = const_cast<olv_graph *>(g);
+  hipStream_t s = stream();
   int32_t delta = 0;
   if (!(flags & OLV_PERSISTENT)) OLV_TRY(sssp_delta(g, weights, &delta));
-  // destination binning (sssp_bin.hip) unless asked to relax directly
-  if (delta > 0 && !(flags & (OLV_PERSISTENT | OLV_SSSP_DIRECT))) {
-    bool used = false;
-    OLV_TRY(sssp_bin_run(g, d_srcs, k, weights, dist, delta, flags, st, &used));
-    if (used) return OLV_OK;
+  const bool binned = delta > 0 && !(flags & (OLV_PERSISTENT | OLV_SSSP_DIRECT)) && sssp_bin_fits(g, k);
+  DevBuf ds;  // the sources, when they do not travel as an argument
+  if (multi || binned) {
+    OLV_TRY(ds.alloc((size_t)k * 4));
+    OLV_HIP(hipMemcpyAsync(ds.p, srcs, (size_t)k * 4, hipMemcpyHostToDevice, s));
   }
-  SsspWork w;
-  OLV_TRY(w.alloc(nv, k, g->m));
+  // destination binning (sssp_bin.hip) unless asked to relax directly
+  if (binned) return sssp_bin_run(g, ds.as<uint32_t>(), k, weights, dist, delta, flags, st);
+  SsspWork *w = nullptr;
+  OLV_TRY(get_sssp_work(gm, k, &w));
   SsspParams p;
   p.row_ptr = g->row_ptr;
   p.col = g->col;
   p.w = weights;
   p.dist = dist;
-  p.queue = w.queue;
-  p.hubs = w.hubs;
-  p.bms = w.bms;
-  p.ctl = w.ctl;
-  p.bar = w.bar;
+  p.queue = w->queue;
+  p.hubs = w->hubs;
+  p.mark = w->mark;
+  p.cand = (flags & OLV_PERSISTENT) ? nullptr : w->cand;
+  p.ctl = w->ctl;
+  p.bar = w->bar;
   p.n = g->n;
   p.ninst = k;
-  p.nw = w.nw;
-  p.nwp = w.nwp;
+  p.nv = (uint32_t)nv;
   p.wave_thr = g->tune.td_wave_thr;
   p.block_thr = g->tune.td_block_thr;
   p.hub_thr = g->tune.hub_thr;
   p.delta = delta;
-  p.far_bm = delta ? w.bms + (size_t)2 * w.nwp : nullptr;
   // plain rounds keep the reference's negative-cycle rule (n rounds); with
   // non-negative weights the cap only guards against a runaway loop
   p.max_rounds = delta ? (uint32_t)std::min<uint64_t>(4ull * g->n + 1024, 0xffffffffull) : g->n;
-  hipStream_t s = stream();
   Timer t;
   t.start();
-  hipLaunchKernelGGL(sssp_reset_kernel, dim3(sgrid(std::max<size_t>(nv, (size_t)w.nwp * 3), 256)), dim3(256), 0, s,
-                     dist, (size_t)nv, w.bms, w.nwp, w.ctl, w.bar, delta);
-  hipLaunchKernelGGL(sssp_seed_kernel, dim3(1), dim3(256), 0, s, d_srcs, k, p);
+  hipLaunchKernelGGL(sssp_reset_kernel, dim3(sgrid((size_t)nv * (p.cand ? kCopies : 1u), 256)), dim3(256), 0, s, p, srcs[0]);
+  if (multi) hipLaunchKernelGGL(sssp_seed_kernel, dim3(1), dim3(256), 0, s, ds.as<uint32_t>(), k, p);
   OLV_HIP(hipGetLastError());
   if (flags & OLV_PERSISTENT) {
     const void *fn = multi ? reinterpret_cast<const void *>(sssp_persistent_kernel<true>)
@@ -450,53 +542,54 @@ static int sssp_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, cons
     void *args[] = {&p};
     OLV_HIP(hipLaunchCooperativeKernel(fn, dim3(cu_count()), dim3(kSBlock), args, 0, s));
     t.stop();
-    OLV_TRY(sssp_read(w));
+    OLV_TRY(sssp_read(*w));
     GridBar hb;
-    OLV_HIP(hipMemcpy(&hb, w.bar, sizeof(hb), hipMemcpyDeviceToHost));
-    if (hb.err || !w.h_ctl->done) return fail(OLV_EINTERNAL, "olv_sssp: grid barrier timed out (co-residency lost)");
+    OLV_HIP(hipMemcpy(&hb, w->bar, sizeof(hb), hipMemcpyDeviceToHost));
+    if (hb.err || !w->h_ctl->done) return fail(OLV_EINTERNAL, "olv_sssp: grid barrier timed out (co-residency lost)");
   } else {
-    // relax workgroups per CU: the graph's tuning (uniform 2^22 x 2^25 graph:
-    // 6 gives 1.99 ms; 4: 2.00, 8: 2.03, 12: 2.01, 16: 2.05)
+    // relax workgroups per CU: the graph's tuning
     const unsigned gr = (unsigned)cu_count() * g->tune.sssp_relax_per_cu;
-    const unsigned gc = sgrid(w.nw, kSBlock);
+    const unsigned gc = sgrid(((size_t)nv + 3) / 4, kSBlock);
     // first chunk: the longest of the last few runs on this graph (8 at
-    // first); longer runs continue in doubling chunks after a host check
-    olv_graph *gm = const_cast<olv_graph *>(g);
+    // first; a run of r rounds takes r + 1 launch pairs, and two runs may
+    // differ by a round or two); longer runs continue in chunks of 8, 16, ...
+    // after a host check
     uint32_t hist = 8;
-    for (uint32_t r : gm->sssp_rounds) hist = std::max(hist, std::min(r, 4096u));
+    for (uint32_t r : gm->sssp_rounds) hist = std::max(hist, std::min(r + 3, 4096u));
     uint32_t chunk = (flags & OLV_HOST_LOOP) ? 1u : hist;
+    uint32_t more = 4;
     uint64_t enq = 0;
     for (;;) {
       for (uint32_t i = 0; i < chunk; ++i) {
-        if (multi)
-          hipLaunchKernelGGL(sssp_relax_kernel<true>, dim3(gr), dim3(kSBlock), 0, s, p);
+        if (p.cand && multi)
+          hipLaunchKernelGGL((sssp_relax_kernel<true, true>), dim3(gr), dim3(kSBlock), 0, s, p);
+        else if (p.cand)
+          hipLaunchKernelGGL((sssp_relax_kernel<false, true>), dim3(gr), dim3(kSBlock), 0, s, p);
+        else if (multi)
+          hipLaunchKernelGGL((sssp_relax_kernel<true, false>), dim3(gr), dim3(kSBlock), 0, s, p);
         else
-          hipLaunchKernelGGL(sssp_relax_kernel<false>, dim3(gr), dim3(kSBlock), 0, s, p);
+          hipLaunchKernelGGL((sssp_relax_kernel<false, false>), dim3(gr), dim3(kSBlock), 0, s, p);
         hipLaunchKernelGGL(sssp_compact_kernel, dim3(gc), dim3(kSBlock), 0, s, p);
       }
       OLV_HIP(hipGetLastError());
       t.stop();  // ahead of the read-back: host latency after the last round is not timed
       enq += chunk;
-      OLV_TRY(sssp_read(w));
-      if (w.h_ctl->done) break;
+      OLV_TRY(sssp_read(*w));
+      if (w->h_ctl->done) break;
       // the device stops by itself after p.max_rounds rounds (capped)
       if (enq > (uint64_t)p.max_rounds + 2) return fail(OLV_EINTERNAL, "olv_sssp: round loop did not terminate");
-      if (!(flags & OLV_HOST_LOOP)) chunk = std::min(chunk * 2, 256u);
+      if (!(flags & OLV_HOST_LOOP)) chunk = more = std::min(more * 2, 256u);
     }
   }
-  const double ms = t.ms();
-  {
-    olv_graph *gm = const_cast<olv_graph *>(g);
-    for (int i = 3; i > 0; --i) gm->sssp_rounds[i] = gm->sssp_rounds[i - 1];
-    gm->sssp_rounds[0] = w.h_ctl->rounds;
-  }
+  for (int i = 3; i > 0; --i) gm->sssp_rounds[i] = gm->sssp_rounds[i - 1];
+  gm->sssp_rounds[0] = w->h_ctl->rounds;
   if (st) {
     std::memset(st, 0, sizeof(*st));
-    st->elapsed_ms = ms;
-    st->iterations = w.h_ctl->rounds;
-    st->edges_inspected = w.h_ctl->relax;
+    st->elapsed_ms = t.ms();
+    st->iterations = w->h_ctl->rounds;
+    st->edges_inspected = w->h_ctl->relax;
   }
-  if (w.h_ctl->capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after n=%u rounds (negative cycle)", g->n);
+  if (w->h_ctl->capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after n=%u rounds (negative cycle)", g->n);
   return OLV_OK;
 }
 
@@ -541,7 +634,7 @@ static int sssp_entry(const olv_graph *g, const uint32_t *srcs, uint32_t k, cons
   const bool host = (flags & OLV_PTR_HOST) != 0;
   for (uint32_t i = 0; i < k; ++i)
     if (srcs[i] >= g->n) return fail(OLV_EINVAL, "olv_sssp: source %u out of range (n=%u)", srcs[i], g->n);
-  DevBuf dw, dd, ds;
+  DevBuf dw, dd;
   const int32_t *w = weights;
   if (!w) {
     if (g->wdtype != OLV_W_I32) return fail(OLV_EINVAL, "olv_sssp: graph has no int32 weights and none were given");
@@ -557,9 +650,7 @@ static int sssp_entry(const olv_graph *g, const uint32_t *srcs, uint32_t k, cons
     OLV_TRY(dd.alloc(total * 4));
     out = dd.as<int32_t>();
   }
-  OLV_TRY(ds.alloc((size_t)k * 4));
-  OLV_HIP(hipMemcpy(ds.p, srcs, (size_t)k * 4, hipMemcpyHostToDevice));
-  OLV_TRY(sssp_run(g, ds.as<uint32_t>(), k, w, out, flags, st));
+  OLV_TRY(sssp_run(g, srcs, k, w, out, flags, st));
   if (st) OLV_TRY(reach_stats(g, out, k, st));
   if (host) OLV_HIP(hipMemcpy(dist, out, total * 4, hipMemcpyDeviceToHost));
   return OLV_OK;

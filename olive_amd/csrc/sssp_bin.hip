@@ -1,42 +1,33 @@
-// SSSP by destination binning: each round's relaxations are scattered into
-// per-partition bins, then applied partition by partition in LDS.
+// SSSP by destination binning, for large graphs without hub vertices: each
+// round's relaxations are scattered into per-partition regions, then applied
+// partition by partition in LDS.
 //
 // Same fixed point as the frontier relaxation of SSSP.cu:146-163 (and the
 // direct path in sssp.hip): every vertex whose distance drops is expanded
 // again with its new distance until nothing drops, and shortest distances
 // are unique, so the order of relaxations changes no output.  What changes is
 // where the min-reductions happen.  A relaxation in the direct path is a
-// random 4-byte probe of dist and, when it improves, two device-scope atomics
-// (atomicMin on dist, atomicOr on a bitmap).  On MI355X those atomics are
-// performed at the memory side, and binning the probes by the XCD that owns
-// the destination does not help them: 20M random relaxations into a 16 MB
-// array cost about 735 us either way.  Here a round is two kernels:
-//
-//   expand (A): the frontier's out-edges become (target, candidate) pairs,
-//     staged in LDS by destination partition (2^sb consecutive virtual
-//     vertices) and written to that partition's bin as contiguous runs; one
-//     device-scope atomic per (tile, partition) reserves the run.  No dist
-//     probe, no per-edge atomic.
-//   apply (B): one workgroup per partition loads the partition's dist slice
-//     and dirty bits into LDS, takes the min of every binned candidate with
-//     LDS atomics, writes back the 256-byte wave spans that changed, and
-//     builds the next frontier from its own slice.
-//
-// 20M pairs: A about 90 us, B about 35 us, against 735 us for the same
-// relaxations done directly (measured with synthetic pairs).
+// random 4-byte probe of dist and, when it improves, a device-scope atomicMin.
+// On MI355X those atomics are performed at the memory side, and binning the
+// probes by the XCD that owns the destination does not help them: 20M random
+// relaxations into a 16 MB array cost about 735 us either way; scattering the
+// pairs into per-partition bins and applying each partition in LDS takes
+// about 90 + 35 us.
 //
 // Near-far order (Davidson et al., IPDPS'14) is kept with one "dirty" bit per
 // vertex: the distance dropped since the vertex was last expanded.  With
-// split T, the frontier is {dirty, dist < T}; B builds it for the next round
-// and records the smallest dirty distance >= T.  When the frontier is empty
-// the next round re-splits at (smallest dirty far distance) + delta -- no
-// empty promotion, the split always lands past at least one vertex -- and
-// when nothing is dirty the run is done.  A vertex leaves the dirty set when
-// it is expanded: B of round R+1 clears the bits of the frontier A of round
-// R+1 expanded, recomputed from the slice state B of round R left.
+// split T, the frontier is {dirty, dist < T}; when it is empty the next round
+// re-splits at (smallest dirty far distance) + delta -- no empty promotion,
+// the split always lands past at least one vertex -- and when nothing is
+// dirty the run is done.
 //
 // k sources run as k instances over virtual vertices s*n + v (as in
 // sssp.hip); partitions cover virtual ranges, so one launch serves all.
+//
+// A workgroup owns a slice of consecutive vertices, so a graph whose edges
+// crowd on some vertices leaves most of the chip idle, and small graphs have
+// too few slices: those take the direct path.
+//
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -49,437 +40,10 @@
 
 namespace olv {
 
-constexpr int kBinA = 512;                           // expand workgroup (~53 KB LDS: 3 per CU)
-constexpr int kBinSlots = 8;                         // pairs per thread per tile
-constexpr uint32_t kBinTile = kBinA * kBinSlots;     // 4096 pairs per tile
-constexpr uint32_t kBinPartMax = 1024;               // partitions
-constexpr int kBinB = 1024;                          // apply workgroup
-constexpr uint32_t kFillStride = 32;                 // one fill counter per 128-byte line
-// slice: 2^14 vertices (64 KB of dist; 16 pairs per partition run in a
-// 4096-pair tile of a 4M-vertex graph) up to 2^15 (128 KB)
-constexpr uint32_t kBinSbMin = 14, kBinSbMax = 15;
-
-enum : uint32_t { kModeNear = 0, kModeResplit = 1, kModeDone = 2 };
-
-// Smallest dirty far distance, one copy per 128-byte line (workgroup b of
-// the apply kernel updates copy b % kCtrSlots).
-struct alignas(128) MinSlot {
-  int32_t v;
-  uint32_t pad[31];
-};
-
-struct BinCtl {
-  uint32_t round;    // next round to expand (written by apply)
-  uint32_t round_b;  // round being applied (written by expand)
-  uint32_t done, rounds, capped, err, resplits, pad0;
-  uint32_t mode[2];  // mode of round R, slot R & 1
-  int32_t split[2];  // split[R & 1]: the split the frontier of round R was built with
-  uint32_t qn[2];    // frontier queue length of round R
-  uint32_t hn[2];    // frontier hub items of round R
-  unsigned long long relax;  // result: edges read
-  MinSlot minfar[2][kCtrSlots];
-  CtrSet cnt[2];     // edges read by the expand of round R (slot R & 1)
-};
-
-struct BinArgs {
-  const uint32_t *row_ptr;
-  const uint32_t *col;
-  const int32_t *w;
-  int32_t *dist;       // nv
-  uint32_t *dirty;     // nwp words
-  const uint32_t *hub_bm;  // rows with out-degree >= hub_thr (n bits)
-  uint32_t *queue[2];  // frontier entries (virtual ids) of round R in queue[R & 1]
-  uint2 *hubs[2];      // frontier hub items of round R
-  uint2 *bins;         // pairs (virtual target, candidate)
-  const uint32_t *pbase;  // nparts + 1: bin offsets (capacities = in-edges of the partition)
-  uint32_t *fill;      // nparts x kFillStride: pairs in the partition's bin this round
-  BinCtl *ctl;
-  uint32_t n, k, nv, nw, nparts, sb;
-  uint32_t hub_thr;
-  int32_t delta;
-  uint32_t max_rounds;
-};
-
-__device__ __forceinline__ uint32_t bin_row(const BinArgs &a, uint32_t x) { return a.k > 1 ? x % a.n : x; }
-
-// Virtual id -> CSR row.
-struct BinRow {
-  uint32_t n, k;
-  __device__ __forceinline__ uint32_t operator()(uint32_t x) const { return k > 1 ? x % n : x; }
-};
-
 __device__ __forceinline__ int32_t add_clamp(int32_t t, int32_t d) { return t > kInf - d ? kInf : t + d; }
 
-// ---------------------------------------------------------------- expand
-__global__ void __launch_bounds__(kBinA) ssspb_expand_kernel(BinArgs a) {
-  BinCtl *ctl = a.ctl;
-  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-  const uint32_t R = ctl->round;
-  const uint32_t t = threadIdx.x;
-  const bool lead = blockIdx.x == 0;
-  if (R >= a.max_rounds) {
-    if (lead && t == 0) {
-      ctl->rounds = R;
-      ctl->capped = 1u;
-      ctl->done = 1u;
-    }
-    return;
-  }
-  const uint32_t qn = ctl->qn[R & 1], hn = ctl->hn[R & 1];
-  const int32_t split = ctl->split[R & 1];
-  __shared__ int32_t s_mf;
-  if (t < kWave) {
-    int32_t mf = t < kCtrSlots ? ctl->minfar[R & 1][t].v : kInf;
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      const int32_t y = __shfl_xor(mf, o, kWave);
-      mf = y < mf ? y : mf;
-    }
-    if (t == 0) s_mf = mf;
-  }
-  __syncthreads();
-  const int32_t minfar = s_mf;
-  const uint32_t mode = (qn + hn) ? kModeNear : (minfar < kInf ? kModeResplit : kModeDone);
-  if (lead) {
-    if (t == 0) {
-      ctl->round_b = R;
-      ctl->mode[R & 1] = mode;
-      ctl->split[(R + 1) & 1] = mode == kModeNear ? split : add_clamp(minfar, a.delta);
-      ctl->qn[(R + 1) & 1] = 0;
-      ctl->hn[(R + 1) & 1] = 0;
-      if (mode == kModeResplit) ctl->resplits += 1;
-      if (mode == kModeDone) {
-        ctl->rounds = R;
-        ctl->done = 1u;
-      }
-    }
-    if (t < kCtrSlots) ctl->minfar[(R + 1) & 1][t].v = kInf;
-  }
-  if (mode != kModeNear) return;
-
-  __shared__ uint32_t s_off[kBinA + 1], s_beg[kBinA], s_xb[kBinA];
-  __shared__ int32_t s_du[kBinA];
-  __shared__ uint32_t s_scan[kBinA / kWave + 1];
-  __shared__ uint32_t s_cnt[kBinPartMax], s_po[kBinPartMax], s_g[kBinPartMax];
-  __shared__ uint2 s_st[kBinTile];
-  constexpr uint32_t kPP = kBinPartMax / kBinA;  // partitions per thread (scan)
-  for (uint32_t j = 0; j < kPP; ++j) s_cnt[t * kPP + j] = 0;
-
-  const uint32_t *queue = a.queue[R & 1];
-  const uint2 *hubs = a.hubs[R & 1];
-  const uint32_t nitems = qn + hn;
-  const uint32_t G = gridDim.x;
-  const uint32_t per = (nitems + G - 1) / G;
-  const uint32_t i0 = blockIdx.x * per;
-  const uint32_t i1 = min(nitems, i0 + per);
-  unsigned long long insp = 0;
-  for (uint32_t ib = i0; ib < i1; ib += kBinA) {
-    const uint32_t i = ib + t;
-    uint32_t beg = 0, deg = 0, xb = 0;
-    int32_t du = 0;
-    if (i < i1) {
-      uint32_t x, rb, re;
-      if (i < qn) {
-        x = queue[i];
-        const uint32_t row = bin_row(a, x);
-        rb = a.row_ptr[row];
-        re = a.row_ptr[row + 1];
-        beg = rb;
-        deg = re - rb;
-        xb = x - row;
-      } else {
-        const uint2 it = hubs[i - qn];
-        x = it.x;
-        const uint32_t row = bin_row(a, x);
-        rb = a.row_ptr[row];
-        re = a.row_ptr[row + 1];
-        beg = rb + it.y * a.hub_thr;
-        deg = beg < re ? min(a.hub_thr, re - beg) : 0u;
-        xb = x - row;
-      }
-      du = a.dist[x];
-    }
-    uint32_t E;
-    const uint32_t off = block_exclusive_scan<kBinA>(deg, s_scan, &E);
-    s_off[t] = i < i1 ? off : E;
-    s_beg[t] = beg;
-    s_xb[t] = xb;
-    s_du[t] = du;
-    if (t == 0) s_off[kBinA] = E;
-    insp += deg;
-    __syncthreads();
-    for (uint32_t tb = 0; tb < E; tb += kBinTile) {
-      const uint32_t tn = min(kBinTile, E - tb);
-      uint2 pr[kBinSlots];
-      uint32_t rk[kBinSlots];
-#pragma unroll
-      for (int j = 0; j < kBinSlots; ++j) {
-        const uint32_t kk = j * kBinA + t;
-        pr[j] = make_uint2(0xffffffffu, 0u);
-        if (kk < tn) {
-          const uint32_t slot = tb + kk;
-          // owner: the last item whose offset is <= slot
-          uint32_t lo = 0, hi = kBinA;  // s_off[lo] <= slot < s_off[hi]
-          while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (s_off[mid] <= slot)
-              lo = mid;
-            else
-              hi = mid;
-          }
-          const uint32_t e = s_beg[lo] + (slot - s_off[lo]);
-          const uint32_t v = s_xb[lo] + a.col[e];
-          pr[j] = make_uint2(v, (uint32_t)s_du[lo] + (uint32_t)a.w[e]);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kBinSlots; ++j)
-        if (pr[j].x != 0xffffffffu) rk[j] = atomicAdd(&s_cnt[pr[j].x >> a.sb], 1u);
-      __syncthreads();
-      // partition offsets in the tile, and one reservation per partition
-      uint32_t c[kPP], sum = 0;
-#pragma unroll
-      for (uint32_t j = 0; j < kPP; ++j) {
-        c[j] = s_cnt[t * kPP + j];
-        sum += c[j];
-      }
-      uint32_t tot;
-      uint32_t run = block_exclusive_scan<kBinA>(sum, s_scan, &tot);
-#pragma unroll
-      for (uint32_t j = 0; j < kPP; ++j) {
-        const uint32_t p = t * kPP + j;
-        s_po[p] = run;
-        uint32_t g = 0xffffffffu;
-        if (c[j]) {
-          const uint32_t old = atomicAdd(&a.fill[p * kFillStride], c[j]);
-          const uint32_t cap = a.pbase[p + 1] - a.pbase[p];
-          if (old + c[j] <= cap)
-            g = a.pbase[p] + old;
-          else
-            __hip_atomic_store(&ctl->err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        s_g[p] = g;
-        run += c[j];
-      }
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < kBinSlots; ++j)
-        if (pr[j].x != 0xffffffffu) s_st[s_po[pr[j].x >> a.sb] + rk[j]] = pr[j];
-      __syncthreads();
-      for (uint32_t q = t; q < tn; q += kBinA) {
-        const uint2 e = s_st[q];
-        const uint32_t p = e.x >> a.sb;
-        const uint32_t g = s_g[p];
-        if (g != 0xffffffffu) a.bins[g + (q - s_po[p])] = e;
-      }
-      __syncthreads();
-#pragma unroll
-      for (uint32_t j = 0; j < kPP; ++j) s_cnt[t * kPP + j] = 0;
-      __syncthreads();
-    }
-  }
-  // edges read: the sum of every lane's item degrees
-  flush_counters<kBinA>(&ctl->cnt[R & 1], 0u, 0ull, insp);
-}
-
-// ----------------------------------------------------------------- apply
-template <uint32_t SB>
-__global__ void __launch_bounds__(kBinB) ssspb_apply_kernel(BinArgs a) {
-  constexpr uint32_t S = 1u << SB;
-  constexpr uint32_t J = S / kBinB;
-  // the pre-apply values stay in registers up to 16 per lane; above that
-  // they are read again from dist (this workgroup's own slice, unchanged)
-  constexpr bool kKeep = J <= 16;
-  extern __shared__ uint32_t s_dyn[];
-  int32_t *s_d = reinterpret_cast<int32_t *>(s_dyn);  // S values
-  uint32_t *s_dw = s_dyn + S;                         // S / 32 dirty words
-  __shared__ uint32_t s_scan[kBinB / kWave + 1];
-  __shared__ uint32_t s_base;
-  __shared__ int32_t s_mf[kBinB / kWave];
-  BinCtl *ctl = a.ctl;
-  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-  const uint32_t R = ctl->round_b;
-  const uint32_t t = threadIdx.x;
-  const bool near_mode = ctl->mode[R & 1] == kModeNear;
-  const int32_t tc = ctl->split[R & 1];       // split of the frontier just expanded
-  const int32_t tb = ctl->split[(R + 1) & 1];  // split of the next frontier
-  if (blockIdx.x == 0) {
-    const CtrSum c = ctr_total(&ctl->cnt[R & 1]);
-    if (t == 0) {
-      ctl->relax += c.inspected;
-      ctl->round = R + 1;
-    }
-    ctr_clear(&ctl->cnt[(R + 1) & 1]);
-  }
-  uint32_t *nq = a.queue[(R + 1) & 1];
-  uint2 *nh = a.hubs[(R + 1) & 1];
-  const uint32_t lane = lane_id();
-  for (uint32_t p = blockIdx.x; p < a.nparts; p += gridDim.x) {
-    const uint32_t x0 = p << SB;
-    const uint32_t cv = min(S, a.nv - x0);  // vertices in this partition
-    int32_t old[kKeep ? J : 1];
-#pragma unroll
-    for (uint32_t j = 0; j < J; ++j) {
-      const uint32_t x = j * kBinB + t;
-      const int32_t o = x < cv ? a.dist[x0 + x] : kInf;
-      if (kKeep) old[kKeep ? j : 0] = o;
-      s_d[x] = o;
-    }
-    const uint32_t w0 = x0 >> 5;
-    for (uint32_t w = t; w < S / 32; w += kBinB) s_dw[w] = w0 + w < a.nw ? a.dirty[w0 + w] : 0u;
-    __syncthreads();
-    const uint32_t np = a.fill[p * kFillStride];
-    const uint32_t cap = a.pbase[p + 1] - a.pbase[p];
-    const uint32_t cnt = np <= cap ? np : cap;
-    const uint2 *b = a.bins + a.pbase[p];
-    // (every binned target lies in this slice; the mask only keeps a
-    // corrupted bin from reaching past the LDS array)
-    uint32_t i = t;
-    for (; i + 3 * kBinB < cnt; i += 4 * kBinB) {
-      const uint2 q0 = b[i], q1 = b[i + kBinB], q2 = b[i + 2 * kBinB], q3 = b[i + 3 * kBinB];
-      atomicMin(&s_d[(q0.x - x0) & (S - 1)], (int32_t)q0.y);
-      atomicMin(&s_d[(q1.x - x0) & (S - 1)], (int32_t)q1.y);
-      atomicMin(&s_d[(q2.x - x0) & (S - 1)], (int32_t)q2.y);
-      atomicMin(&s_d[(q3.x - x0) & (S - 1)], (int32_t)q3.y);
-    }
-    for (; i < cnt; i += kBinB) {
-      const uint2 q = b[i];
-      atomicMin(&s_d[(q.x - x0) & (S - 1)], (int32_t)q.y);
-    }
-    __syncthreads();
-    if (t == 0) a.fill[p * kFillStride] = 0u;
-    // classify: dirty' = (dirty & !expanded) | improved; next frontier =
-    // dirty' & dist < tb; far minimum over dirty' & dist >= tb
-    uint32_t nnear = 0;
-    uint32_t nearbits = 0;  // bit j: vertex j * kBinB + t joins the queue
-    uint32_t wasbits = 0;   // bit j: vertex j * kBinB + t was dirty
-#pragma unroll
-    for (uint32_t j = 0; j < J; ++j) {
-      const uint32_t x = j * kBinB + t;
-      wasbits |= ((s_dw[x >> 5] >> (x & 31)) & 1u) << j;
-    }
-    __syncthreads();  // every dirty word is read before any is replaced
-    int32_t mf = kInf;
-#pragma unroll
-    for (uint32_t j = 0; j < J; ++j) {
-      const uint32_t x = j * kBinB + t;
-      const int32_t nv = s_d[x];
-      const bool inb = x < cv;
-      const int32_t o = kKeep ? old[kKeep ? j : 0] : (inb ? a.dist[x0 + x] : kInf);
-      const bool improved = inb && nv < o;
-      const bool was = (wasbits >> j) & 1u;
-      const bool expanded = near_mode && was && o < tc;
-      const bool dirty = (was && !expanded) || improved;
-      const uint64_t any = ballot(improved);
-      if (any && inb) a.dist[x0 + x] = nv;  // whole wave span: no partial lines
-      const uint64_t db = ballot(dirty);
-      if (lane == 0) s_dw[x >> 5] = (uint32_t)db;
-      if (lane == 32) s_dw[x >> 5] = (uint32_t)(db >> 32);
-      if (dirty && nv < tb) {
-        bool hub = false;
-        if (a.hub_bm) {
-          const uint32_t row = bin_row(a, x0 + x);
-          hub = (a.hub_bm[row >> 5] >> (row & 31)) & 1u;
-        }
-        if (hub) {
-          const uint32_t row = bin_row(a, x0 + x);
-          const uint32_t d = a.row_ptr[row + 1] - a.row_ptr[row];
-          const uint32_t kk = (d + a.hub_thr - 1) / a.hub_thr;
-          const uint32_t hb = atomicAdd(&ctl->hn[(R + 1) & 1], kk);
-          for (uint32_t c = 0; c < kk; ++c) nh[hb + c] = make_uint2(x0 + x, c);
-        } else {
-          nearbits |= 1u << j;
-          ++nnear;
-        }
-      } else if (dirty) {
-        mf = nv < mf ? nv : mf;
-      }
-    }
-    __syncthreads();
-    for (uint32_t w = t; w < S / 32; w += kBinB)
-      if (w0 + w < a.nw) a.dirty[w0 + w] = s_dw[w];
-    uint32_t total;
-    const uint32_t off = block_exclusive_scan<kBinB>(nnear, s_scan, &total);
-    if (t == 0) s_base = total ? atomicAdd(&ctl->qn[(R + 1) & 1], total) : 0u;
-    for (int o = kWave / 2; o > 0; o >>= 1) {
-      const int32_t y = __shfl_xor(mf, o, kWave);
-      mf = y < mf ? y : mf;
-    }
-    if (lane == 0) s_mf[t / kWave] = mf;
-    __syncthreads();
-    uint32_t pos = s_base + off;
-#pragma unroll
-    for (uint32_t j = 0; j < J; ++j)
-      if ((nearbits >> j) & 1u) nq[pos++] = x0 + j * kBinB + t;
-    if (t == 0) {
-      int32_t m = kInf;
-      for (int q = 0; q < kBinB / kWave; ++q) m = s_mf[q] < m ? s_mf[q] : m;
-      if (m < kInf) atomicMin(&ctl->minfar[(R + 1) & 1][blockIdx.x % kCtrSlots].v, m);
-    }
-    __syncthreads();
-  }
-}
-
-// dist = INF, dirty = 0, fill = 0, control zero (minfar INF), split = delta.
-__global__ void ssspb_reset_kernel(BinArgs a) {
-  const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (size_t i = tid; i < a.nv; i += stride) a.dist[i] = kInf;
-  for (size_t i = tid; i < a.nw; i += stride) a.dirty[i] = 0u;
-  for (size_t i = tid; i < (size_t)a.nparts * kFillStride; i += stride) a.fill[i] = 0u;
-  uint32_t *c = reinterpret_cast<uint32_t *>(a.ctl);
-  for (size_t i = tid; i < sizeof(BinCtl) / 4; i += stride) c[i] = 0u;
-  if (tid == 0) a.ctl->split[0] = a.delta;
-}
-
-// One workgroup, after the reset: minfar = INF, then the k seeds.
-__global__ void ssspb_seed_kernel(const uint32_t *srcs, BinArgs a) {
-  if (threadIdx.x < kCtrSlots) {
-    a.ctl->minfar[0][threadIdx.x].v = kInf;
-    a.ctl->minfar[1][threadIdx.x].v = kInf;
-  }
-  auto claim = [&](uint32_t s) -> uint32_t {
-    const uint32_t x = s * a.n + srcs[s];
-    a.dist[x] = 0;
-    atomicOr(&a.dirty[x >> 5], 1u << (x & 31));
-    return x;
-  };
-  unsigned long long deg;
-  seed_frontier(srcs, a.k, a.row_ptr, a.hub_thr, a.queue[0], &a.ctl->qn[0], a.hubs[0], &a.ctl->hn[0], claim,
-                BinRow{a.n, a.k}, &deg);
-}
-
-// Capacity of each partition's bin: in-edges of its virtual vertices, i.e.
-// over the k instances, the edges whose target s*n + col[e] falls in it.
-__global__ void ssspb_cap_kernel(const uint32_t *col, uint32_t m, uint32_t n, uint32_t k, uint32_t sb,
-                                 uint32_t nparts, uint32_t *cap) {
-  __shared__ uint32_t s_h[kBinPartMax];
-  for (uint32_t p = threadIdx.x; p < nparts; p += blockDim.x) s_h[p] = 0;
-  __syncthreads();
-  const uint64_t total = (uint64_t)k * m;
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t s = (uint32_t)(i / m), e = (uint32_t)(i % m);
-    atomicAdd(&s_h[(s * n + col[e]) >> sb], 1u);
-  }
-  __syncthreads();
-  for (uint32_t p = threadIdx.x; p < nparts; p += blockDim.x)
-    if (s_h[p]) atomicAdd(&cap[p], s_h[p]);
-}
-
-// Rows with out-degree >= thr.
-__global__ void ssspb_hub_kernel(const uint32_t *rp, uint32_t n, uint32_t thr, uint32_t *bm) {
-  const uint32_t lane = lane_id();
-  for (uint32_t v0 = (blockIdx.x * blockDim.x + threadIdx.x) & ~63u; v0 < n; v0 += gridDim.x * blockDim.x) {
-    const uint32_t v = v0 + lane;
-    const bool h = v < n && rp[v + 1] - rp[v] >= thr;
-    const uint64_t b = ballot(h);
-    if (lane == 0) bm[v0 >> 5] = (uint32_t)b;
-    if (lane == 32 && v0 + 32 < n) bm[(v0 >> 5) + 1] = (uint32_t)(b >> 32);
-  }
-}
-
-// ------------------------------------------------------------ fused rounds
-// One kernel per round for graphs without hub vertices: workgroup q owns
+// ------------------------------------------------------------------ rounds
+// One kernel per round: workgroup q owns
 // partition q (2^14 virtual vertices) and, in launch R,
 //   1. applies the pairs that every partition sent it in launch R-1 (region
 //      p -> q of the pair store, one count per region) to its dist slice in
@@ -492,9 +56,7 @@ __global__ void ssspb_hub_kernel(const uint32_t *rp, uint32_t n, uint32_t thr, u
 //      the two slices, fixed per graph).
 // The split T of launch R comes from the previous launch's totals (striped
 // counters): frontier non-empty -> same split; empty -> re-split at the
-// smallest dirty far distance + delta; nothing dirty -> done.  Half the
-// kernel boundaries of the expand/apply pair above, and none of its
-// reservation atomics.
+// smallest dirty far distance + delta; nothing dirty -> done.
 // Slices of 2^14 vertices (64 KB of dist; ~135 KB of LDS, one workgroup per
 // CU) up to 16M virtual vertices.  (2^13-vertex slices fit two workgroups per
 // CU by LDS, but the second ones started up to 120 us late on MI355X and a
@@ -904,24 +466,16 @@ __global__ void ssspf_seed_kernel(const uint32_t *srcs, FusedArgs a) {
 
 // --------------------------------------------------------------------- host
 struct SsspBinWork {
-  bool fused = false;
-  uint32_t k = 0, hub_thr = 0, sb = 0, nparts = 0, nw = 0, nwp = 0;
+  uint32_t k = 0, sb = 0, nparts = 0, nw = 0, nwp = 0;
   uint64_t nv = 0;
-  uint32_t *pbase = nullptr, *fill = nullptr, *dirty = nullptr, *hub_bm = nullptr;
-  uint32_t *queue[2] = {nullptr, nullptr};
-  uint2 *hubs[2] = {nullptr, nullptr};
-  uint2 *bins = nullptr;
-  BinCtl *ctl = nullptr, *h_ctl = nullptr;
-  // fused rounds
+  uint32_t *dirty = nullptr;
   uint2 *pairs[2] = {nullptr, nullptr};
   uint32_t *base = nullptr, *cnt[2] = {nullptr, nullptr};
   FusedCtl *fctl = nullptr, *h_fctl = nullptr;
   ~SsspBinWork() {
-    void *ps[] = {pbase, fill, dirty, hub_bm, queue[0], queue[1], hubs[0], hubs[1], bins, ctl,
-                  pairs[0], pairs[1], base, cnt[0], cnt[1], fctl};
+    void *ps[] = {dirty, pairs[0], pairs[1], base, cnt[0], cnt[1], fctl};
     for (void *q : ps)
       if (q) (void)hipFree(q);
-    if (h_ctl) (void)hipHostFree(h_ctl);
     if (h_fctl) (void)hipHostFree(h_fctl);
   }
 };
@@ -936,109 +490,17 @@ static unsigned bgrid(size_t items, size_t per) {
   return (unsigned)std::max<size_t>(1, std::min(b, (size_t)cu_count() * 8));
 }
 
-template <uint32_t SB>
-constexpr size_t apply_lds() {
-  return ((size_t)1 << SB) * 4 + ((size_t)1 << SB) / 8;  // dist slice + dirty words
-}
-
-template <uint32_t SB>
-static void launch_apply(const BinArgs &a, unsigned grid, hipStream_t s) {
-  hipLaunchKernelGGL(ssspb_apply_kernel<SB>, dim3(grid), dim3(kBinB), apply_lds<SB>(), s, a);
-}
-
-// Allow the apply kernel's dynamic LDS (up to 132 KB) on the current device.
-static int allow_apply_lds(uint32_t sb) {
-  if (sb == 13)
-    OLV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ssspb_apply_kernel<13>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)apply_lds<13>()));
-  else if (sb == 14)
-    OLV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ssspb_apply_kernel<14>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)apply_lds<14>()));
-  else
-    OLV_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(ssspb_apply_kernel<15>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)apply_lds<15>()));
-  return OLV_OK;
-}
-
-// Work arrays for k instances on g (kept on the graph for the next call
-// with the same k and hub threshold).
-static int bin_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) {
-  SsspBinWork *w = g->sssp_bin;
-  const uint32_t hub_thr = g->tune.hub_thr;
-  if (w && !w->fused && w->k == k && w->hub_thr == hub_thr && w->sb == sb) {
-    *out = w;
-    return OLV_OK;
-  }
-  free_sssp_bin(g);
-  w = new SsspBinWork();
-  g->sssp_bin = w;
-  w->k = k;
-  w->hub_thr = hub_thr;
-  w->sb = sb;
-  w->nv = (uint64_t)k * g->n;
-  w->nparts = (uint32_t)((w->nv + (1ull << sb) - 1) >> sb);
-  w->nw = (uint32_t)((w->nv + 31) / 32);
-  w->nwp = (w->nw + 63) / 64 * 64;
-  auto fail_alloc = [&]() {
-    free_sssp_bin(g);
-    return fail(OLV_ENOMEM, "olv_sssp: device allocation for the binned relaxation failed");
-  };
-  const size_t hubcap = hub_capacity(g->m) * k;
-  if (hipMalloc(reinterpret_cast<void **>(&w->pbase), (size_t)(w->nparts + 1) * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->fill), (size_t)w->nparts * kFillStride * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->dirty), (size_t)w->nwp * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->queue[0]), w->nv * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->queue[1]), w->nv * 4) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->hubs[0]), hubcap * sizeof(uint2)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->hubs[1]), hubcap * sizeof(uint2)) != hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->bins), std::max<uint64_t>((uint64_t)k * g->m, 1) * sizeof(uint2)) !=
-          hipSuccess ||
-      hipMalloc(reinterpret_cast<void **>(&w->ctl), sizeof(BinCtl)) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void **>(&w->h_ctl), sizeof(BinCtl), hipHostMallocDefault) != hipSuccess)
-    return fail_alloc();
-  if (g->max_outdeg >= hub_thr) {
-    const uint32_t hw = (g->n + 31) / 32;
-    if (hipMalloc(reinterpret_cast<void **>(&w->hub_bm), (size_t)hw * 4) != hipSuccess) return fail_alloc();
-    hipLaunchKernelGGL(ssspb_hub_kernel, dim3(bgrid(g->n, 256)), dim3(256), 0, stream(), g->row_ptr, g->n, hub_thr,
-                       w->hub_bm);
-    OLV_HIP(hipGetLastError());
-  }
-  // bin offsets: exclusive scan of the partition capacities (host, <= 1024)
-  DevBuf cap;
-  OLV_TRY(cap.alloc((size_t)w->nparts * 4));
-  OLV_HIP(hipMemsetAsync(cap.p, 0, (size_t)w->nparts * 4, stream()));
-  hipLaunchKernelGGL(ssspb_cap_kernel, dim3(bgrid((size_t)k * g->m, 1024)), dim3(1024), 0, stream(), g->col, g->m,
-                     g->n, k, sb, w->nparts, cap.as<uint32_t>());
-  OLV_HIP(hipGetLastError());
-  std::vector<uint32_t> hc(w->nparts), hb(w->nparts + 1);
-  OLV_HIP(hipMemcpyAsync(hc.data(), cap.p, (size_t)w->nparts * 4, hipMemcpyDeviceToHost, stream()));
-  OLV_HIP(hipStreamSynchronize(stream()));
-  uint64_t run = 0;
-  for (uint32_t p = 0; p < w->nparts; ++p) {
-    hb[p] = (uint32_t)run;
-    run += hc[p];
-  }
-  hb[w->nparts] = (uint32_t)run;
-  if (run != (uint64_t)k * g->m) return fail(OLV_EINTERNAL, "olv_sssp: bin capacities %llu != %llu edges",
-                                              (unsigned long long)run, (unsigned long long)k * g->m);
-  OLV_HIP(hipMemcpy(w->pbase, hb.data(), (size_t)(w->nparts + 1) * 4, hipMemcpyHostToDevice));
-  OLV_TRY(allow_apply_lds(sb));
-  *out = w;
-  return OLV_OK;
-}
-
 // Work for the fused rounds: region capacities (edges between every pair of
 // slices), their offsets, two pair stores and two count matrices.
 static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) {
   SsspBinWork *w = g->sssp_bin;
-  if (w && w->fused && w->k == k && w->sb == sb) {
+  if (w && w->k == k && w->sb == sb) {
     *out = w;
     return OLV_OK;
   }
   free_sssp_bin(g);
   w = new SsspBinWork();
   g->sssp_bin = w;
-  w->fused = true;
   w->k = k;
   w->sb = sb;
   w->nv = (uint64_t)k * g->n;
@@ -1116,8 +578,9 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
   hipLaunchKernelGGL(ssspf_seed_kernel, dim3(1), dim3(256), 0, s, d_srcs, a);
   OLV_HIP(hipGetLastError());
   uint32_t hist = 8;
-  for (uint32_t r : gm->sssp_rounds) hist = std::max(hist, std::min(r + 1, 4096u));
+  for (uint32_t r : gm->sssp_rounds) hist = std::max(hist, std::min(r + 3, 4096u));
   uint32_t chunk = (flags & OLV_HOST_LOOP) ? 1u : hist;
+  uint32_t more = 4;
   uint64_t enq = 0;
   for (;;) {
     for (uint32_t i = 0; i < chunk; ++i)
@@ -1129,7 +592,7 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
     OLV_HIP(hipStreamSynchronize(s));
     if (w->h_fctl->done) break;
     if (enq > (uint64_t)a.max_rounds + 2) return fail(OLV_EINTERNAL, "olv_sssp: round loop did not terminate");
-    if (!(flags & OLV_HOST_LOOP)) chunk = std::min(chunk * 2, 256u);
+    if (!(flags & OLV_HOST_LOOP)) chunk = more = std::min(more * 2, 256u);
   }
   const FusedCtl &c = *w->h_fctl;
   for (int i = 3; i > 0; --i) gm->sssp_rounds[i] = gm->sssp_rounds[i - 1];
@@ -1145,113 +608,38 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
   return OLV_OK;
 }
 
-// Binned SSSP for k instances (sources d_srcs[0..k), on the device) with
-// near-far step delta > 0.  *used = false (and nothing run) when the graph
-// does not fit the scheme: more than 1024 partitions of 2^15 virtual
-// vertices, or k x m >= 2^32 bin entries.
-int sssp_bin_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, const int32_t *weights, int32_t *dist,
-                 int32_t delta, unsigned flags, olv_stats *st, bool *used) {
-  *used = false;
-  if (delta <= 0 || g->m == 0 || g->n == 0) return OLV_OK;
+// Virtual vertices from which binning beats direct relaxation on graphs
+// without hubs (8 edges a vertex, binned / direct: 250K vertices 995 / 570 us,
+// 1M 985 / 997, 2M 1075 / 1597, 4M 1455 / 2770).
+constexpr uint64_t kBinMinVertices = 1250000;
+
+// Whether k instances of g go through the binned rounds: no out-list long
+// enough to be split, slices for most of the chip, and at most 16M vertices
+// and 2^32 pairs.
+bool sssp_bin_fits(const olv_graph *g, uint32_t k) {
   const uint64_t nv = (uint64_t)k * g->n;
-  if ((uint64_t)k * g->m >= (1ull << 32) || nv >= (1ull << 32)) return OLV_OK;
-  // one kernel per round when no out-list needs splitting (hub items);
-  // more instances than the fused kernel's 16M virtual vertices run in
-  // groups of as many as fit
-  const uint64_t fmax = (uint64_t)kFParts << 14;
-  if (g->max_outdeg < g->tune.hub_thr && g->n <= fmax) {
-    *used = true;
-    const uint32_t gk = (uint32_t)std::min<uint64_t>(k, fmax / g->n);
-    if (gk == k) return fused_run(g, d_srcs, k, weights, dist, delta, flags, st);
-    olv_stats tot;
-    std::memset(&tot, 0, sizeof(tot));
-    for (uint32_t s0 = 0; s0 < k; s0 += gk) {
-      const uint32_t kk = std::min(gk, k - s0);
-      olv_stats one;
-      OLV_TRY(fused_run(g, d_srcs + s0, kk, weights, dist + (size_t)s0 * g->n, delta, flags, &one));
-      tot.elapsed_ms += one.elapsed_ms;
-      tot.iterations += one.iterations;
-      tot.edges_inspected += one.edges_inspected;
-    }
-    if (st) *st = tot;
-    return OLV_OK;
+  return g->m && (uint64_t)k * g->m < (1ull << 32) && nv < (1ull << 32) && nv >= kBinMinVertices &&
+         g->max_outdeg < g->tune.hub_thr && g->n <= ((uint64_t)kFParts << 14);
+}
+
+// Binned SSSP for k instances (sources d_srcs[0..k), on the device; the
+// graph fits) with near-far step delta > 0.  More instances than 16M virtual
+// vertices run in groups of as many as fit.
+int sssp_bin_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, const int32_t *weights, int32_t *dist,
+                 int32_t delta, unsigned flags, olv_stats *st) {
+  const uint32_t gk = (uint32_t)std::min<uint64_t>(k, ((uint64_t)kFParts << 14) / g->n);
+  if (gk == k) return fused_run(g, d_srcs, k, weights, dist, delta, flags, st);
+  olv_stats tot;
+  std::memset(&tot, 0, sizeof(tot));
+  for (uint32_t s0 = 0; s0 < k; s0 += gk) {
+    const uint32_t kk = std::min(gk, k - s0);
+    olv_stats one;
+    OLV_TRY(fused_run(g, d_srcs + s0, kk, weights, dist + (size_t)s0 * g->n, delta, flags, &one));
+    tot.elapsed_ms += one.elapsed_ms;
+    tot.iterations += one.iterations;
+    tot.edges_inspected += one.edges_inspected;
   }
-  uint32_t sb = kBinSbMin;
-  while (sb < kBinSbMax && ((nv + (1ull << sb) - 1) >> sb) > kBinPartMax) ++sb;
-  if (((nv + (1ull << sb) - 1) >> sb) > kBinPartMax) return OLV_OK;
-  olv_graph *gm = const_cast<olv_graph *>(g);
-  SsspBinWork *w = nullptr;
-  OLV_TRY(bin_work(gm, k, sb, &w));
-  *used = true;
-  BinArgs a;
-  a.row_ptr = g->row_ptr;
-  a.col = g->col;
-  a.w = weights;
-  a.dist = dist;
-  a.dirty = w->dirty;
-  a.hub_bm = w->hub_bm;
-  a.queue[0] = w->queue[0];
-  a.queue[1] = w->queue[1];
-  a.hubs[0] = w->hubs[0];
-  a.hubs[1] = w->hubs[1];
-  a.bins = w->bins;
-  a.pbase = w->pbase;
-  a.fill = w->fill;
-  a.ctl = w->ctl;
-  a.n = g->n;
-  a.k = k;
-  a.nv = (uint32_t)nv;
-  a.nw = w->nw;
-  a.nparts = w->nparts;
-  a.sb = sb;
-  a.hub_thr = w->hub_thr;
-  a.delta = delta;
-  a.max_rounds = (uint32_t)std::min<uint64_t>(4ull * g->n + 1024, 0xffffffffull);
-  hipStream_t s = stream();
-  const unsigned ga = (unsigned)cu_count() * 2;  // two expand workgroups per CU (VGPR-bound)
-  const unsigned gb = std::min<uint32_t>(w->nparts, (uint32_t)cu_count() * 2);
-  Timer t;
-  t.start();
-  hipLaunchKernelGGL(ssspb_reset_kernel, dim3(bgrid(std::max<uint64_t>(nv, w->nparts * kFillStride), 256)),
-                     dim3(256), 0, s, a);
-  hipLaunchKernelGGL(ssspb_seed_kernel, dim3(1), dim3(256), 0, s, d_srcs, a);
-  OLV_HIP(hipGetLastError());
-  // first chunk: the longest of the last runs (a run of r rounds takes r + 1
-  // launch pairs: the last one finds nothing left)
-  uint32_t hist = 8;
-  for (uint32_t r : gm->sssp_rounds) hist = std::max(hist, std::min(r + 1, 4096u));
-  uint32_t chunk = (flags & OLV_HOST_LOOP) ? 1u : hist;
-  uint64_t enq = 0;
-  for (;;) {
-    for (uint32_t i = 0; i < chunk; ++i) {
-      hipLaunchKernelGGL(ssspb_expand_kernel, dim3(ga), dim3(kBinA), 0, s, a);
-      if (sb == 13)
-        launch_apply<13>(a, gb, s);
-      else if (sb == 14)
-        launch_apply<14>(a, gb, s);
-      else
-        launch_apply<15>(a, gb, s);
-    }
-    OLV_HIP(hipGetLastError());
-    t.stop();
-    enq += chunk;
-    OLV_HIP(hipMemcpyAsync(w->h_ctl, w->ctl, sizeof(BinCtl), hipMemcpyDeviceToHost, s));
-    OLV_HIP(hipStreamSynchronize(s));
-    if (w->h_ctl->done) break;
-    if (enq > (uint64_t)a.max_rounds + 2) return fail(OLV_EINTERNAL, "olv_sssp: round loop did not terminate");
-    if (!(flags & OLV_HOST_LOOP)) chunk = std::min(chunk * 2, 256u);
-  }
-  const BinCtl &c = *w->h_ctl;
-  for (int i = 3; i > 0; --i) gm->sssp_rounds[i] = gm->sssp_rounds[i - 1];
-  gm->sssp_rounds[0] = c.rounds;
-  if (st) {
-    std::memset(st, 0, sizeof(*st));
-    st->elapsed_ms = t.ms();
-    st->iterations = c.rounds;
-    st->edges_inspected = c.relax;
-  }
-  if (c.err) return fail(OLV_EINTERNAL, "olv_sssp: a bin overflowed its capacity");
-  if (c.capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after %u rounds", c.rounds);
+  if (st) *st = tot;
   return OLV_OK;
 }
 

@@ -1,0 +1,43 @@
+"""SSSP by direct relaxation where its layout changes: vertex counts that do
+not fill the last word of mark bytes, hub rows cut into items, and both sides
+of the size up to which relaxations lower candidate copies instead of the
+distances.  Distances are whole numbers: equal to Dijkstra's."""
+import numpy as np
+import pytest
+
+import oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def graph(olv, n, m, hub, seed):
+    """m uniform edges plus `hub` out-edges of vertex n // 2, weights 1..64."""
+    rng = np.random.default_rng(seed)
+    src = np.concatenate([rng.integers(0, n, m), np.full(hub, n // 2)])
+    dst = rng.integers(0, n, src.size)
+    o = np.lexsort((dst, src))
+    rp = np.zeros(n + 1, np.int64)
+    np.add.at(rp, src + 1, 1)
+    return olv.CsrGraph(np.cumsum(rp).astype(np.uint32), dst[o].astype(np.uint32),
+                        rng.integers(1, 65, src.size).astype(np.int32))
+
+
+@pytest.mark.parametrize("n,m,hub", [(1, 2, 0), (2, 3, 0), (3, 7, 0), (5, 20, 1500), (1023, 4000, 1024),
+                                     (4097, 20000, 5000), ((1 << 20), 1 << 21, 3000), ((1 << 20) + 3, 1 << 21, 3000)])
+def test_direct_rounds(olv, n, m, hub):
+    print("sssp rounds", n, m, hub, flush=True)
+    csr = graph(olv, n, m, hub, n)
+    g = olv.Graph(csr, transpose=False)
+    for s in {0, n // 2, n - 1}:
+        ref = oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, s)
+        assert np.array_equal(g.sssp(s)[0].numpy(), ref), s
+
+
+def test_batched_rounds(olv):
+    # three instances of an odd graph: instance boundaries inside a mark word
+    csr = graph(olv, 333, 2000, 1100, 1)
+    g = olv.Graph(csr, transpose=False)
+    srcs = np.array([5, 166, 332], np.uint32)
+    out = g.sssp_batched(srcs)[0].numpy().reshape(3, -1)
+    for i, s in enumerate(srcs):
+        assert np.array_equal(out[i], oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, int(s))), s
