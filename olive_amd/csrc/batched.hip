@@ -30,12 +30,13 @@ namespace olv {
 int bfs_multisource(const olv_graph *g, const uint32_t *seeds, uint32_t k, bool seeds_host, int32_t *levels,
                     unsigned flags, olv_stats *st);
 int bfs_prepare(const olv_graph *g, bool can_bu, BfsWork **w);
-int bfs_enqueue_init(const olv_graph *g, BfsWork *w, const uint32_t *d_seeds, uint32_t k, int32_t *levels,
-                     bool can_bu);
-int bfs_enqueue_levels(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t count);
+int bfs_enqueue_init(const olv_graph *g, BfsWork *w, const uint32_t *d_seeds, uint32_t k, uint32_t seed1,
+                     int32_t *levels, bool can_bu);
+int bfs_enqueue_levels(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t count, bool narrow);
 int bfs_result(BfsWork *w, uint32_t *levels_run, uint32_t *bu_levels);
 bool bfs_done(BfsWork *w);
-uint32_t bfs_depth_hint(BfsWork *w);
+uint32_t bfs_pairs_hint(const BfsWork *w);
+bool bfs_deep_hint(const BfsWork *w);
 int reach_stats(const olv_graph *g, const int32_t *d, uint32_t k, olv_stats *st);
 
 constexpr int kMB = 256;          // workgroup size
@@ -764,6 +765,7 @@ struct olv_plan {
   uint32_t k = 0;
   int32_t *levels = nullptr;
   bool can_bu = true;
+  bool narrow = false;  // BFS: with narrow launches
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   olv::BfsWork *bw = nullptr;
@@ -1013,10 +1015,10 @@ int olv_bfs_multigraph(olv_graph *const *gs, uint32_t k, const uint32_t *srcs, i
   return s;
 }
 
-// A plan captures init + `depth` levels.  The depth comes from one eager
-// run at plan time (levels are deterministic for fixed sources); a replay
-// that still reports work left continues eagerly, so results never depend
-// on the captured depth.
+// A plan captures init + the launch pairs (and narrow launches) of an eager
+// run at plan time (levels are deterministic for fixed sources); a replay that
+// still reports work left continues eagerly, so results never depend on what
+// was captured.
 int olv_plan_bfs(const olv_graph *g, const uint32_t *srcs, uint32_t k, int32_t *levels, unsigned flags,
                  olv_plan **out) {
   if (!g || !srcs || !levels || !out || k == 0) return fail(OLV_EINVAL, "olv_plan_bfs: bad arguments");
@@ -1036,11 +1038,15 @@ int olv_plan_bfs(const olv_graph *g, const uint32_t *srcs, uint32_t k, int32_t *
   if (s == OLV_OK) s = p->seeds.alloc((size_t)k * 4);
   if (s == OLV_OK && hipMemcpy(p->seeds.p, srcs, (size_t)k * 4, hipMemcpyHostToDevice) != hipSuccess)
     s = fail(OLV_EHIP, "olv_plan_bfs: seed copy failed");
-  const uint32_t depth = bfs_depth_hint(p->bw);
+  uint32_t pairs = 0;
+  if (s == OLV_OK) {
+    pairs = bfs_pairs_hint(p->bw);
+    p->narrow = bfs_deep_hint(p->bw);
+  }
   if (s == OLV_OK)
     s = capture(p, [&]() -> int {
-      OLV_TRY(bfs_enqueue_init(g, p->bw, p->seeds.as<uint32_t>(), k, levels, p->can_bu));
-      return bfs_enqueue_levels(g, p->bw, levels, p->can_bu, depth);
+      OLV_TRY(bfs_enqueue_init(g, p->bw, p->seeds.as<uint32_t>(), k, srcs[0], levels, p->can_bu));
+      return bfs_enqueue_levels(g, p->bw, levels, p->can_bu, pairs, p->narrow);
     });
   if (s != OLV_OK) {
     delete p;
@@ -1115,7 +1121,7 @@ int olv_plan_launch(olv_plan *p, olv_stats *st) {
       Timer t2;
       t2.start();
       for (uint32_t chunk = 8; !bfs_done(p->bw); chunk = std::min(chunk * 2, 256u)) {
-        OLV_TRY(bfs_enqueue_levels(p->g, p->bw, p->levels, p->can_bu, chunk));
+        OLV_TRY(bfs_enqueue_levels(p->g, p->bw, p->levels, p->can_bu, chunk, p->narrow));
         OLV_TRY(bfs_result(p->bw, &levels, &nbu));
       }
       t2.stop();

@@ -17,12 +17,21 @@
 // about 3 us on MI355X (1.8 us inside a hipGraph), less than a grid barrier
 // (6-34 us), so this beats one persistent kernel; the persistent variant is
 // kept behind OLV_PERSISTENT for comparison.
+//
+// A graph of many small levels (meshes, road networks) is bound by those two
+// launches, about 7.7 us a level whatever the level holds.  For such graphs a
+// third kernel precedes every few pairs: one workgroup that keeps the frontier
+// in LDS and runs level after level until the frontier outgrows it
+// (bfs_narrow_kernel; 1.5 us a level of 150 vertices, 2.4 us of 340).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
+#include <cstddef>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "bfs_core.hpp"
@@ -45,19 +54,23 @@ struct BfsState {              // per level parity
 };
 
 struct BfsCtl {
+  uint32_t done;       // traversal finished
+  uint32_t skip;       // the narrow kernel has expanded the level: the next expand launch passes
   uint32_t level;      // next level to expand (written by compact)
   uint32_t level_e;    // level being compacted (written by expand)
-  uint32_t done;       // traversal finished
+  uint32_t pairs;      // result: expand/compact launch pairs that had work
+  uint32_t nlevels;    // result: levels run by the narrow kernel
   uint32_t levels;     // result: levels run, the final empty one included
   uint32_t nbu;        // result: bottom-up levels
   uint32_t overflow;   // result: level cap (n + 1) reached
   uint32_t qfill[2];   // frontier queue length of level L, slot L & 1
   uint32_t hfill[2];   // hub items of level L, slot L & 1
-  uint32_t pad[2];
+  uint32_t pad;
   unsigned long long inspected;  // result: edges read
   BfsState st[2];
   CtrSet cnt[3];       // level counters, slot L % 3
 };
+constexpr size_t kBfsCtlHead = offsetof(BfsCtl, st);  // what the host reads back
 
 struct BfsWork {
   uint32_t n = 0, nw = 0, nwp = 0;  // vertices, bitmap words, padded words
@@ -70,8 +83,8 @@ struct BfsWork {
   BfsCtl *h_ctl = nullptr;          // pinned mirror
   GridBar *bar = nullptr;           // persistent mode
   unsigned long long *stat = nullptr;
-  uint32_t last_levels = 0;         // depth of the previous run (plan capture depth)
-  uint32_t recent[4] = {0, 0, 0, 0};  // depths of the last runs (first chunk = their maximum)
+  uint32_t recent[4] = {0, 0, 0, 0};  // launch pairs of the last runs (first chunk = their maximum)
+  bool deep = false;                // the last run had many small levels: narrow launches from the start
   bool force_bu = false;            // OLV_FORCE_BOTTOM_UP of the current run
 };
 
@@ -127,20 +140,20 @@ static int get_work(const olv_graph *cg, BfsWork **out) {
 // are pre-claimed (visited byte and snapshot bit) when bottom-up steps may
 // run -- no parent can claim them, so bottom-up steps skip them;
 // bfs_seed_kernel releases the seeds among them -- else nothing is.
-// With a single seed (`seed1`, device) the seeding is done here as well:
+// With a single seed (seed1; ~0: none) the seeding is done here as well:
 // the seed's level, visited byte and snapshot bit are written by the lanes
 // that own them, and workgroup 0 builds the level-0 frontier after clearing
-// the control block -- one launch instead of two.
+// the control block -- one launch instead of two, and no copy of the seed.
 __global__ void bfs_reset_kernel(int32_t *__restrict__ levels, uint32_t n, uint8_t *__restrict__ visited,
                                  uint32_t *__restrict__ snap, const uint32_t *__restrict__ no_in,
                                  uint32_t *__restrict__ bms, uint32_t nwp, BfsCtl *__restrict__ ctl,
-                                 GridBar *__restrict__ bar, const uint32_t *__restrict__ seed1, BfsArgs a,
+                                 GridBar *__restrict__ bar, uint32_t seed1, BfsArgs a,
                                  unsigned long long m) {
   const size_t tid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   const size_t nw = ((size_t)n + 31) / 32;
-  const uint32_t s = seed1 ? *seed1 : 0xffffffffu;
-  const uint32_t so = (seed1 && a.omap) ? a.omap[s] : s;  // the seed's levels index
+  const uint32_t s = seed1;
+  const uint32_t so = (s != 0xffffffffu && a.omap) ? a.omap[s] : s;  // the seed's levels index
   for (size_t i = tid; i < n; i += stride) levels[i] = i == so ? 0 : kInf;
   for (size_t i = tid; i < nwp; i += stride) {
     uint32_t d = (no_in && i < nw) ? no_in[i] : 0u;
@@ -160,10 +173,10 @@ __global__ void bfs_reset_kernel(int32_t *__restrict__ levels, uint32_t n, uint8
   if (blockIdx.x != 0) return;
   for (uint32_t i = threadIdx.x; i < sizeof(BfsCtl) / 4; i += blockDim.x) reinterpret_cast<uint32_t *>(ctl)[i] = 0u;
   for (uint32_t i = threadIdx.x; i < sizeof(GridBar) / 4; i += blockDim.x) reinterpret_cast<uint32_t *>(bar)[i] = 0u;
-  if (!seed1) return;
+  if (s == 0xffffffffu) return;
   __syncthreads();
   unsigned long long deg = 0;
-  seed_frontier(seed1, 1u, a.row_ptr, a.hub_thr, a.queue, &ctl->qfill[0], a.hubs, &ctl->hfill[0],
+  seed_frontier(nullptr, 1u, a.row_ptr, a.hub_thr, a.queue, &ctl->qfill[0], a.hubs, &ctl->hfill[0],
                 [&](uint32_t) -> uint32_t { return s; }, IdRow(), &deg);
   if (threadIdx.x == 0) {
     ctl->st[0].mu = m > deg ? m - deg : 0ull;
@@ -213,6 +226,7 @@ struct BfsDir {
 template <bool Mapped>
 __global__ void __launch_bounds__(kBlock) bfs_expand_kernel(BfsArgs a, BfsCtl *ctl, uint32_t *bms, uint32_t nwp) {
   if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  if (ctl->skip) return;
   const uint32_t L = ctl->level;
   const BfsState st = ctl->st[L & 1];
   const uint32_t qsize = ctl->qfill[L & 1], nhubs = ctl->hfill[L & 1];
@@ -247,7 +261,11 @@ __global__ void __launch_bounds__(kBlock) bfs_compact_kernel(BfsArgs a, BfsCtl *
   const BfsState st = ctl->st[L & 1];
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   const uint32_t nbu = st.nbu + st.mode;
-  if (lead) ctl->inspected += c.inspected;
+  if (lead) {
+    ctl->inspected += c.inspected;
+    ctl->pairs += 1;
+    ctl->skip = 0;
+  }
   if (c.nf == 0 || L + 1 > a.n) {
     if (lead) {
       ctl->levels = L + 1;
@@ -270,6 +288,258 @@ __global__ void __launch_bounds__(kBlock) bfs_compact_kernel(BfsArgs a, BfsCtl *
   }
   frontier_words<kBlock>(a, bms + (size_t)((L + 1) & 1) * nwp, nw, !next_bu, &ctl->qfill[(L + 1) & 1],
                          &ctl->hfill[(L + 1) & 1], blockIdx.x, gridDim.x, pre);
+}
+
+// Top-down levels of a small frontier, one after another, in one workgroup.
+// Returns at once unless the level's frontier is a queue of at most kNarrowQ
+// vertices with at most kNarrowEdges out-edges.  A level is bound by its chain:
+// the column loads, the claims in LDS, the claimed vertices' rows, a barrier.
+// So a row is dealt to a group of lanes about as wide as the frontier's mean
+// degree (a lane holds one edge where the level has few: four claims one after
+// another by a lane cost more than the loads), and what the claims go by
+// depends on the vertex count:
+//   Bits   a bitmap of the visited vertices in LDS, read from the visited
+//          bytes on entry (up to kNarrowBitsN vertices).  Nothing that a level
+//          stores to memory is read by the next, so the barrier waits for LDS
+//          only.
+//   else   the visited bytes, read beside the rows; a hash set of the level's
+//          claims in LDS, at most half full, tells apart lanes that find a
+//          vertex unvisited at once.  The barrier waits for the stores.
+// A vertex whose level the kernel expands itself gets visited byte 3, not 1:
+// frontier_words takes it for an old claim (setting its snapshot bit here would
+// take an atomic, about 1 us of the level's chain).
+// The direction rule is not asked: a bottom-up level reads every unvisited
+// vertex's state in two launches, so at these sizes it costs several times a
+// level here (the last 38 levels of a 200 x 150 grid: 10 us each).
+// The level whose claims no longer fit ends as the expand kernel would leave
+// it, its claims in the visited bytes and its totals in the counters, and
+// `skip` makes the next expand launch pass: the compact launch then takes the
+// direction decision and extracts the frontier.
+// Traversals of grids from an inner vertex, before and with it: 200 x 150 2.14
+// and 0.31 ms, 601 x 389 7.6 and 1.65 ms, 1200 x 900 (more than kNarrowBitsN
+// vertices) 22.1 and 11.6 ms, 30 x 8000 (6134 levels) 63.7 and 9.6 ms.
+constexpr int kNarrowBlock = 1024;
+constexpr uint32_t kNarrowQ = 2048;
+constexpr uint32_t kNarrowEdges = 4096;
+constexpr uint32_t kNarrowHashBits = 13;  // twice kNarrowEdges slots
+constexpr uint32_t kNarrowBitsN = 24576 * 32;  // 96 KB of bitmap
+constexpr uint32_t kNarrowLevels = 8192;  // levels per launch, at most
+constexpr uint32_t kNarrowEvery = 16;     // launch pairs between narrow launches
+
+template <bool Mapped, bool Bits>
+__global__ void __launch_bounds__(kNarrowBlock) bfs_narrow_kernel(BfsArgs a, BfsCtl *ctl) {
+  constexpr uint32_t kSlots = 1u << kNarrowHashBits;
+  __shared__ uint32_t s_v[2][kNarrowQ], s_beg[2][kNarrowQ], s_deg[2][kNarrowQ];  // frontier L in [L & 1]
+  __shared__ uint32_t s_claim[Bits ? kNarrowBitsN / 32 : 2 * kSlots];  // bitmap, or two hash sets (~0 = free)
+  __shared__ uint16_t s_slot[2][Bits ? 1 : kNarrowQ];                  // the frontier's places in its hash set
+  __shared__ uint32_t s_cnt[3], s_mf[3];  // level L's claims and their out-degrees, slot L % 3
+  __shared__ unsigned long long s_red[kNarrowBlock / kWave];
+  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+  const uint32_t t = threadIdx.x, lane = lane_id();
+  const uint32_t L0 = ctl->level;
+  uint32_t L = L0, qs = ctl->qfill[L & 1];
+  const BfsState st = ctl->st[L & 1];
+  if (st.mode != 0 || ctl->hfill[L & 1] != 0 || qs == 0 || qs > kNarrowQ) return;
+  unsigned long long insp = 0;
+  for (uint32_t i = t; i < qs; i += kNarrowBlock) {
+    const uint32_t v = a.queue[i], b = a.row_ptr[v], d = a.row_ptr[v + 1] - b;
+    s_v[L & 1][i] = v;
+    s_beg[L & 1][i] = b;
+    s_deg[L & 1][i] = d;
+    if (!Bits) s_slot[L & 1][i] = 0;
+    insp += d;
+  }
+  if (t < 3) s_cnt[t] = s_mf[t] = 0;
+  insp = block_sum<kNarrowBlock, unsigned long long>(insp, s_red);
+  if (insp > kNarrowEdges) return;
+  uint32_t qe = (uint32_t)insp;  // edges of the frontier
+  if (Bits) {
+    const uint32_t nw = (a.n + 31) / 32;
+    for (uint32_t i = t; i < nw; i += kNarrowBlock) {
+      const uint4 *p = reinterpret_cast<const uint4 *>(a.visited + (size_t)i * 32u);
+      s_claim[i] = byte_flags(p[0], p[1], 0);
+    }
+  } else {
+    for (uint32_t i = t; i < 2 * kSlots; i += kNarrowBlock) s_claim[i] = 0xffffffffu;
+  }
+  __syncthreads();
+  unsigned long long mu = st.mu;
+  uint32_t nf = 0, mf = 0;
+  insp = 0;
+  for (;;) {
+    const uint32_t cur = L & 1, nxt = cur ^ 1, c3 = L % 3;
+    if (t == 0) s_cnt[(L + 1) % 3] = s_mf[(L + 1) % 3] = 0;  // last read before the previous level's barrier
+    uint32_t lmf = 0;
+    // the unvisited targets among U edges of a lane
+    auto visit = [&](const auto &e, const auto &in) {
+      constexpr int U = sizeof(in);
+      uint32_t v[U], h[U];
+      uint2 r[U];
+      bool mine[U];
+#pragma unroll
+      for (int j = 0; j < U; ++j) v[j] = in[j] ? a.col[e[j]] : 0u;
+      if (Bits) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          const uint32_t bit = 1u << (v[j] & 31);
+          mine[j] = in[j] && !(atomicOr(&s_claim[v[j] >> 5], bit) & bit);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < U; ++j) mine[j] = in[j] && a.visited[v[j]] == 0;
+      }
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const bool ld = Bits ? mine[j] : in[j];
+        r[j] = make_uint2(0u, 0u);
+        if (ld) __builtin_memcpy(&r[j], a.row_ptr + v[j], 8);  // begin and end in one load
+      }
+      if (!Bits) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+          if (!mine[j]) continue;
+          uint32_t *set = s_claim + nxt * kSlots, old;
+          h[j] = (v[j] * 2654435761u) >> (32 - kNarrowHashBits);
+          while ((old = atomicCAS(&set[h[j]], 0xffffffffu, v[j])) != 0xffffffffu && old != v[j])
+            h[j] = (h[j] + 1) & (kSlots - 1);
+          mine[j] = old != v[j];  // else another edge's claim
+        }
+      }
+      uint32_t before[U], total = 0;  // the wave's claims, counted by one atomic
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const uint64_t w = ballot(mine[j]);
+        before[j] = total + lane_rank(w);
+        total += (uint32_t)__popcll(w);
+      }
+      if (total == 0) return;
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&s_cnt[c3], total);
+      base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        if (!mine[j]) continue;
+        const uint32_t pos = base + before[j];
+        lmf += r[j].y - r[j].x;
+        if (!Bits) a.visited[v[j]] = 1;
+        if (pos < kNarrowQ) {
+          s_v[nxt][pos] = v[j];
+          s_beg[nxt][pos] = r[j].x;
+          s_deg[nxt][pos] = r[j].y - r[j].x;
+          if (!Bits) s_slot[nxt][pos] = (uint16_t)h[j];
+        } else {
+          if (Bits) a.visited[v[j]] = 1;
+          a.template set_level<Mapped>(v[j], (int32_t)(L + 1));
+        }
+      }
+    };
+    // lanes per row: the mean degree rounded up to a power of two, a lane
+    // visiting one edge at a time; where the frontier has more rows than that
+    // allows at once, fewer lanes, each visiting two edges at a time (four:
+    // 601 x 389 grid 1.70 ms, two 1.65; one, in more rounds: 1.78)
+    uint32_t lg = 0;
+    while (lg < 6 && (qs << lg) < qe) ++lg;
+    const bool one = (qs << lg) <= kNarrowBlock;
+    while (lg > 0 && (qs << lg) > kNarrowBlock) --lg;
+    const uint32_t gl = 1u << lg, sub = t & (gl - 1);
+    auto edges = [&](uint32_t first, uint32_t count, uint32_t sub_, uint32_t gl_, auto U) {
+      for (uint32_t q = 0; ballot(q < count); q += U * gl_) {
+        uint32_t e[U];
+        bool in[U];
+#pragma unroll
+        for (uint32_t j = 0; j < U; ++j) {
+          e[j] = first + q + j * gl_ + sub_;
+          in[j] = q + j * gl_ + sub_ < count;
+        }
+        visit(e, in);
+      }
+    };
+    for (uint32_t i = t >> lg; i - (lane >> lg) < qs; i += kNarrowBlock >> lg) {  // the same rounds for the whole wave
+      uint32_t beg = 0, deg = 0, u = 0, o = 0;
+      const bool put = L != L0 && sub == 0 && i < qs;  // the vertex's level is stored beside the visits
+      if (i < qs) {
+        beg = s_beg[cur][i];
+        deg = s_deg[cur][i];
+        if (put) {
+          u = s_v[cur][i];
+          o = Mapped ? a.omap[u] : u;
+        }
+        if (sub == 0) {
+          insp += deg;
+          if (!Bits) s_claim[cur * kSlots + s_slot[cur][i]] = 0xffffffffu;  // free for the claims of the next level
+        }
+      }
+      const bool wide = deg > 8 * gl;
+      if (one)
+        edges(beg, wide ? 0u : deg, sub, gl, std::integral_constant<uint32_t, 1>());
+      else
+        edges(beg, wide ? 0u : deg, sub, gl, std::integral_constant<uint32_t, 2>());
+      for (uint64_t w = ballot(wide && sub == 0); w; w &= w - 1) {  // rows of many edges: the wave's lanes on each
+        const int from = __ffsll((unsigned long long)w) - 1;
+        edges(__shfl(beg, from, kWave), __shfl(deg, from, kWave), lane, kWave, std::integral_constant<uint32_t, 4>());
+      }
+      if (put) {
+        a.levels[o] = (int32_t)L;
+        a.visited[u] = 3;
+      }
+    }
+    lmf = wave_sum_last(lmf);  // 64 lanes' atomics on one word would take longer than the loads
+    if (lane == kWave - 1 && lmf) atomicAdd(&s_mf[c3], lmf);
+    if (Bits) {
+      lds_barrier();
+    } else {
+      __syncthreads();
+    }
+    nf = s_cnt[c3];
+    mf = s_mf[c3];
+    if (nf == 0 || L + 1 > a.n || nf > kNarrowQ || mf > kNarrowEdges) break;
+    mu = mu > mf ? mu - mf : 0ull;
+    qs = nf;
+    qe = mf;
+    nf = 0;
+    ++L;
+    if (L - L0 == kNarrowLevels) break;
+  }
+  const bool more = L - L0 == kNarrowLevels;  // level L's frontier is whole and has its row in LDS
+  const uint32_t last = more ? L : L + 1;     // the frontier not expanded here
+  for (uint32_t i = t; i < min(more ? qs : nf, kNarrowQ); i += kNarrowBlock) {
+    const uint32_t v = s_v[last & 1][i];
+    a.template set_level<Mapped>(v, (int32_t)last);
+    a.visited[v] = more ? 3 : 1;
+    if (more) a.queue[i] = v;
+  }
+  ctr_clear(&ctl->cnt[L % 3]);
+  ctr_clear(&ctl->cnt[(L + 1) % 3]);
+  insp = block_sum<kNarrowBlock, unsigned long long>(insp, s_red);  // (and a barrier)
+  if (t != 0) return;
+  ctl->nlevels += L - L0 + (more ? 0u : 1u);
+  if (!more && nf == 0) {
+    ctl->levels = L + 1;
+    ctl->nbu = st.nbu;
+    ctl->inspected += insp;
+    ctl->done = 1u;
+    return;
+  }
+  BfsState ns;
+  ns.mu = mu;
+  ns.mode = 0;
+  ns.nbu = st.nbu;
+  ctl->st[L & 1] = ns;
+  ctl->level = L;
+  if (more) {
+    ctl->inspected += insp;
+    ctl->qfill[L & 1] = qs;
+    ctl->hfill[L & 1] = 0;
+    return;
+  }
+  ctl->level_e = L;
+  ctl->qfill[(L + 1) & 1] = 0;
+  ctl->hfill[(L + 1) & 1] = 0;
+  BfsCtr &c = ctl->cnt[L % 3].s[0];
+  c.nf = nf;
+  c.mf = mf;
+  c.inspected = insp;
+  ctl->skip = 1;
 }
 
 // All levels in one cooperative launch with the XCD-aware grid barrier
@@ -391,14 +661,15 @@ int bfs_prepare(const olv_graph *g, bool can_bu, BfsWork **w) {
   return get_work(g, w);
 }
 
-// Stream-ordered, capturable: reset and seeding.
-int bfs_enqueue_init(const olv_graph *g, BfsWork *w, const uint32_t *d_seeds, uint32_t k, int32_t *levels,
-                     bool can_bu) {
+// Stream-ordered, capturable: reset and seeding from k seeds d_seeds
+// (device), or from the one seed `seed1` by value (k == 1).
+int bfs_enqueue_init(const olv_graph *g, BfsWork *w, const uint32_t *d_seeds, uint32_t k, uint32_t seed1,
+                     int32_t *levels, bool can_bu) {
   const uint32_t *no_in = can_bu ? g->no_in_bm : nullptr;
   const BfsArgs a = make_args(g, w, levels);
   hipLaunchKernelGGL(bfs_reset_kernel, dim3(grid_for(std::max<size_t>(g->n, (size_t)w->nwp * 2), 256, 8)), dim3(256),
                      0, stream(), levels, g->n, w->visited, w->snap, no_in, w->bms, w->nwp, w->ctl, w->bar,
-                     k == 1 ? d_seeds : nullptr, a, (unsigned long long)g->m);
+                     k == 1 ? seed1 : 0xffffffffu, a, (unsigned long long)g->m);
   if (k != 1)
     hipLaunchKernelGGL(bfs_seed_kernel, dim3(1), dim3(256), 0, stream(), d_seeds, k, a, (unsigned long long)g->m,
                        w->ctl);
@@ -406,13 +677,20 @@ int bfs_enqueue_init(const olv_graph *g, BfsWork *w, const uint32_t *d_seeds, ui
   return OLV_OK;
 }
 
-// Stream-ordered, capturable: `count` levels (expand + compact each).
-int bfs_enqueue_levels(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t count) {
+// Stream-ordered, capturable: `count` launch pairs (expand + compact, a level
+// each), with a narrow launch ahead of every kNarrowEvery of them if `narrow`.
+int bfs_enqueue_levels(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t count, bool narrow) {
   const BfsArgs a = make_args(g, w, levels);
   const BfsDir dir = make_dir(g, w, can_bu);
   const unsigned ge = (unsigned)cu_count() * (a.omap ? g->tune.bfs_expand_per_cu_twin : g->tune.bfs_expand_per_cu);
   const unsigned gc = grid_for(w->nw, kBlock, g->tune.bfs_compact_per_cu);
   for (uint32_t i = 0; i < count; ++i) {
+    if (narrow && !dir.force_bu && i % kNarrowEvery == 0) {
+      const bool bits = g->n <= kNarrowBitsN;
+      auto *kern = a.omap ? (bits ? bfs_narrow_kernel<true, true> : bfs_narrow_kernel<true, false>)
+                          : (bits ? bfs_narrow_kernel<false, true> : bfs_narrow_kernel<false, false>);
+      hipLaunchKernelGGL(kern, dim3(1), dim3(kNarrowBlock), 0, stream(), a, w->ctl);
+    }
     if (a.omap)
       hipLaunchKernelGGL(bfs_expand_kernel<true>, dim3(ge), dim3(kBlock), 0, stream(), a, w->ctl, w->bms, w->nwp);
     else
@@ -442,9 +720,9 @@ static int enqueue_persistent(const olv_graph *g, BfsWork *w, int32_t *levels, b
   return OLV_OK;
 }
 
-// Wait for the stream, then read the control block.
+// Wait for the stream, then read the head of the control block.
 int bfs_result(BfsWork *w, uint32_t *levels_run, uint32_t *bu_levels) {
-  OLV_HIP(hipMemcpyAsync(w->h_ctl, w->ctl, sizeof(BfsCtl), hipMemcpyDeviceToHost, stream()));
+  OLV_HIP(hipMemcpyAsync(w->h_ctl, w->ctl, kBfsCtlHead, hipMemcpyDeviceToHost, stream()));
   OLV_HIP(hipStreamSynchronize(stream()));
   if (levels_run) *levels_run = w->h_ctl->levels;
   if (bu_levels) *bu_levels = w->h_ctl->nbu;
@@ -452,28 +730,41 @@ int bfs_result(BfsWork *w, uint32_t *levels_run, uint32_t *bu_levels) {
 }
 
 bool bfs_done(BfsWork *w) { return w->h_ctl->done != 0; }
-uint32_t bfs_depth_hint(BfsWork *w) { return w->last_levels; }
-void bfs_set_depth_hint(BfsWork *w, uint32_t d) { w->last_levels = d; }
-uint32_t *bfs_ctl_words(BfsWork *w) { return reinterpret_cast<uint32_t *>(w->ctl); }
-GridBar *bfs_bar(BfsWork *w) { return w->bar; }
+// Launch pairs that a run like the last one takes, and whether it begins with
+// a narrow launch (so it does where no run went through launch pairs: a graph
+// for bfs_small).
+uint32_t bfs_pairs_hint(const BfsWork *w) { return std::max(1u, w->recent[0]); }
+bool bfs_deep_hint(const BfsWork *w) { return w->deep || w->recent[0] == 0; }
 
-// Enqueue levels in growing chunks until the device reports done.
-// chunk0 == 1 gives one host round trip per level (OLV_HOST_LOOP).  The
-// stop event of `t` follows the last enqueued level, ahead of the control
-// block read-back, so host latency after the last kernel is not timed (the
-// gaps between chunks are).
-static int run_pipeline(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t chunk0, Timer *t) {
-  uint32_t chunk = std::max(1u, chunk0);
+// Enqueue launch pairs in growing chunks until the device reports done; one
+// host round trip per level if `host_loop`.  The narrow kernel joins from the
+// second chunk on, or from the first where the last run on this graph ran
+// kDeepLevels levels in it: on a shallow graph a launch that finds a wide
+// frontier costs 2 us for nothing.  The stop event of `t` follows the last
+// enqueued level, ahead of the control block read-back, so host latency after
+// the last kernel is not timed (the gaps between chunks are).
+constexpr uint32_t kDeepLevels = 8;
+
+static int run_pipeline(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t chunk0, bool host_loop,
+                        Timer *t) {
+  uint32_t chunk = host_loop ? 1u : chunk0;
+  bool narrow = !host_loop && w->deep;
   uint64_t enq = 0;
   for (;;) {
-    OLV_TRY(bfs_enqueue_levels(g, w, levels, can_bu, chunk));
+    OLV_TRY(bfs_enqueue_levels(g, w, levels, can_bu, chunk, narrow));
     if (t) t->stop();
     enq += chunk;
     OLV_TRY(bfs_result(w, nullptr, nullptr));
     if (w->h_ctl->done) break;
     if (enq > (uint64_t)g->n + 2) return fail(OLV_EINTERNAL, "olv_bfs: level loop did not terminate");
-    if (chunk0 > 1) chunk = std::min(chunk * 2, 256u);
+    if (!host_loop) chunk = std::min(std::max(chunk, 2u) * 2, 256u);
+    narrow = !host_loop;
   }
+  if (!host_loop && !w->force_bu) w->deep = w->h_ctl->nlevels >= kDeepLevels;
+  w->recent[3] = w->recent[2];
+  w->recent[2] = w->recent[1];
+  w->recent[1] = w->recent[0];
+  w->recent[0] = w->h_ctl->pairs;
   return OLV_OK;
 }
 
@@ -643,41 +934,36 @@ int bfs_multisource(const olv_graph *g0, const uint32_t *seeds, uint32_t k, bool
   OLV_TRY(bfs_prepare(g, can_bu, &w));
   w->force_bu = (flags & OLV_FORCE_BOTTOM_UP) != 0;
   DevBuf d_seeds, d_levels;
-  OLV_TRY(d_seeds.alloc((size_t)k * 4));
-  OLV_HIP(hipMemcpyAsync(d_seeds.p, h_seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice, stream()));
+  if (k > 1) {
+    OLV_TRY(d_seeds.alloc((size_t)k * 4));
+    OLV_HIP(hipMemcpyAsync(d_seeds.p, h_seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice, stream()));
+  }
   int32_t *out = levels;
   if (host) {
     OLV_TRY(d_levels.alloc((size_t)g->n * 4));
     out = d_levels.as<int32_t>();
   }
-  Timer t;
-  t.start();
-  OLV_TRY(bfs_enqueue_init(g, w, d_seeds.as<uint32_t>(), k, out, can_bu));
+  std::unique_ptr<Timer> t(st ? new Timer() : nullptr);
+  if (t) t->start();
+  OLV_TRY(bfs_enqueue_init(g, w, d_seeds.as<uint32_t>(), k, h_seeds[0], out, can_bu));
   if (flags & OLV_PERSISTENT) {
     OLV_TRY(enqueue_persistent(g, w, out, can_bu));
-    t.stop();
-  } else {
-    // first chunk: the deepest of the last few runs (traversals of one graph
-    // from different sources have similar depths); deeper runs continue in
-    // doubling chunks after one host check
-    const uint32_t recent_max = std::max(std::max(w->recent[0], w->recent[1]), std::max(w->recent[2], w->recent[3]));
-    const uint32_t chunk0 = (flags & OLV_HOST_LOOP) ? 1u : std::max(4u, recent_max);
-    OLV_TRY(run_pipeline(g, w, out, can_bu, chunk0, &t));
-  }
-  const double ms = t.ms();
-  uint32_t levels_run = 0, bu_levels = 0;
-  OLV_TRY(bfs_result(w, &levels_run, &bu_levels));
-  if (flags & OLV_PERSISTENT) {
+    if (t) t->stop();
+    OLV_TRY(bfs_result(w, nullptr, nullptr));
     GridBar hb;
     OLV_HIP(hipMemcpy(&hb, w->bar, sizeof(hb), hipMemcpyDeviceToHost));
     if (hb.err || !w->h_ctl->done) return fail(OLV_EINTERNAL, "olv_bfs: grid barrier timed out (co-residency lost)");
+  } else {
+    // first chunk: the most launch pairs of the last few runs (traversals of
+    // one graph from different sources have similar depths); longer runs
+    // continue in doubling chunks after one host check
+    const uint32_t recent_max = std::max(std::max(w->recent[0], w->recent[1]), std::max(w->recent[2], w->recent[3]));
+    OLV_TRY(run_pipeline(g, w, out, can_bu, std::max(w->deep ? 1u : 4u, recent_max), (flags & OLV_HOST_LOOP) != 0,
+                         t.get()));
   }
+  const uint32_t levels_run = w->h_ctl->levels, bu_levels = w->h_ctl->nbu;
+  const double ms = t ? t->ms() : 0.0;
   if (w->h_ctl->overflow) return fail(OLV_EINTERNAL, "olv_bfs: more than n levels");
-  w->last_levels = levels_run;
-  w->recent[3] = w->recent[2];
-  w->recent[2] = w->recent[1];
-  w->recent[1] = w->recent[0];
-  w->recent[0] = levels_run;
   if (host) OLV_HIP(hipMemcpy(levels, out, (size_t)g->n * 4, hipMemcpyDeviceToHost));
   if (st) {
     std::memset(st, 0, sizeof(*st));
@@ -703,7 +989,7 @@ extern "C" int olv_bfs(const olv_graph *g, uint32_t src, int32_t *levels, unsign
 // ------------------------------------------------ allocation-free entry point
 // olv_bfs_noalloc keeps every work buffer of a traversal (visited bytes,
 // snapshot and frontier bitmaps, queue, hub items, control block, barrier,
-// statistics, the seed) in one static device array per GPU instead of
+// statistics) in one static device array per GPU instead of
 // buffers allocated with the graph.  The host code only ever uses the array's
 // device address, obtained once per device with hipGetSymbolAddress.
 namespace olv {
@@ -719,7 +1005,7 @@ std::mutex g_scratch_mu;
 unsigned char *g_scratch_ptr[kMaxDevices] = {};
 
 struct NoAllocLayout {
-  size_t visited, snap, bms, queue, hubs, ctl, bar, stat, seed, total;
+  size_t visited, snap, bms, queue, hubs, ctl, bar, stat, total;
   uint32_t nw, nwp;
 };
 
@@ -745,13 +1031,9 @@ NoAllocLayout noalloc_layout(uint32_t n, uint64_t m) {
   o += al(sizeof(GridBar));
   L.stat = o;
   o += al(2 * sizeof(unsigned long long));
-  L.seed = o;
-  o += al(sizeof(uint32_t));
   L.total = o;
   return L;
 }
-
-__global__ void store_word_kernel(uint32_t *__restrict__ p, uint32_t v) { *p = v; }
 }  // namespace
 
 // The current device's copy of `scratch` (its address looked up once per
@@ -809,13 +1091,10 @@ extern "C" int olv_bfs_noalloc(const olv_graph *g, uint32_t src, int32_t *levels
   w.stat = reinterpret_cast<unsigned long long *>(base + L.stat);
   w.h_ctl = &hctl;
   w.force_bu = (flags & OLV_FORCE_BOTTOM_UP) != 0;
-  uint32_t *seed = reinterpret_cast<uint32_t *>(base + L.seed);
   const auto t0 = std::chrono::steady_clock::now();
-  hipLaunchKernelGGL(store_word_kernel, dim3(1), dim3(1), 0, stream(), seed, src);
-  OLV_TRY(bfs_enqueue_init(g, &w, seed, 1, levels, can_bu));
-  OLV_TRY(run_pipeline(g, &w, levels, can_bu, (flags & OLV_HOST_LOOP) ? 1u : 8u, nullptr));
-  uint32_t levels_run = 0, bu_levels = 0;
-  OLV_TRY(bfs_result(&w, &levels_run, &bu_levels));
+  OLV_TRY(bfs_enqueue_init(g, &w, nullptr, 1, src, levels, can_bu));
+  OLV_TRY(run_pipeline(g, &w, levels, can_bu, 8u, (flags & OLV_HOST_LOOP) != 0, nullptr));
+  const uint32_t levels_run = hctl.levels, bu_levels = hctl.nbu;
   const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
   if (hctl.overflow) return fail(OLV_EINTERNAL, "olv_bfs_noalloc: more than n levels");
   if (st) {

@@ -77,7 +77,7 @@ struct BfsArgs {
   const uint2 *in_head;  // first two in-neighbours (0xffffffff where absent)
   int32_t *levels;
   const uint32_t *omap;  // levels index of each vertex (renumbered twin), or nullptr: the vertex id
-  uint8_t *visited;    // one byte per vertex: nonzero = claimed (padded to 32-vertex words)
+  uint8_t *visited;    // one byte per vertex: bit 0 = claimed, bit 1 = and expanded (padded to 32-vertex words)
   uint32_t *snap;      // bitmap of the claims as of the last frontier extraction
   uint32_t *queue;
   uint2 *hubs;
@@ -470,13 +470,23 @@ struct WordLoad {
   uint32_t snap;
 };
 
+// Bit `bit` of 32 bytes side by side: four bytes per multiplication, which
+// moves their flags next to each other without a carry.
+__device__ __forceinline__ uint32_t byte_flags(const uint4 &q0, const uint4 &q1, int bit) {
+  const uint32_t parts[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+  uint32_t f = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) f |= ((((parts[i] >> bit) & 0x01010101u) * 0x10204080u) >> 28) << (4 * i);
+  return f;
+}
+
 __device__ __forceinline__ WordLoad load_word(const BfsArgs &a, uint32_t w) {
   const uint4 *p = reinterpret_cast<const uint4 *>(a.visited + (size_t)w * 32u);  // 32-byte aligned
   return WordLoad{p[0], p[1], a.snap[w]};
 }
 
-// Next frontier = visited bytes set since the last extraction: written to
-// `front` (for a bottom-up step) and, if `to_queue`, compacted into the
+// Next frontier = visited bytes set since the last extraction, those that say
+// "expanded already" (bit 1, bfs_narrow_kernel) excepted: written to `front` (for a bottom-up step) and, if `to_queue`, compacted into the
 // queue and hub items (for a top-down step); `snap` catches up.  `pre` is
 // this lane's first word (index vb * BLOCK + threadIdx.x), already loaded.
 template <int BLOCK>
@@ -485,14 +495,9 @@ __device__ void frontier_words(const BfsArgs &a, uint32_t *front, uint32_t nw, b
   const uint32_t wpre = vb * BLOCK + threadIdx.x;
   auto word_of = [&](uint32_t w) -> uint32_t {
     const WordLoad x = w == wpre ? pre : load_word(a, w);
-    const uint32_t parts[8] = {x.q0.x, x.q0.y, x.q0.z, x.q0.w, x.q1.x, x.q1.y, x.q1.z, x.q1.w};
-    uint32_t v = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) v |= ((parts[i] >> (8 * b)) & 0xffu ? 1u : 0u) << (4 * i + b);
-    const uint32_t nb = v & ~x.snap;
-    if (nb) a.snap[w] = x.snap | nb;
+    const uint32_t v = byte_flags(x.q0, x.q1, 0), old = byte_flags(x.q0, x.q1, 1);
+    const uint32_t nb = v & ~(x.snap | old);
+    if (v & ~x.snap) a.snap[w] = x.snap | v;
     front[w] = nb;
     return nb;
   };
