@@ -786,71 +786,105 @@ static int collect_stats(const olv_graph *g, BfsWork *w, const int32_t *levels, 
 // whole traversal in one workgroup: the row offsets, the visited bits and
 // both frontier queues sit in LDS (~130 KB), so a level costs the column
 // loads (L2 hits after the first level), LDS claims and one barrier -- not
-// two kernel launches.  The 128 x 128 grid (255 levels of at most 128
-// vertices) was launch-bound at ~11 us per level in the pipeline.
+// two kernel launches.  A small frontier is dealt to lanes by edges (2^lg
+// lanes a row, lg from the graph's mean degree), a large one by rows, four
+// edges of a lane in flight; a wave counts its claims by one LDS atomic.  The
+// 128 x 128 grid (from an inner vertex, 200 levels of at most 128 vertices):
+// 254 us by rows with a lane's claims one by one and two barriers a level,
+// 174 us so.
 constexpr uint32_t kSmallN = 16384;
 constexpr uint32_t kSmallMaxDeg = 256;
 constexpr int kSmallBlock = 1024;
 
-// out[0] = levels run (the deepest level + 1), out[1] = edges read (= the
-// out-degree sum of reached vertices), out[2] = vertices reached.
+// Seeds: k of them at `seeds` (device), or the one seed `seed1` (k == 1).
+// out (nullptr: not wanted): [0] = levels run (the deepest level + 1), [1] =
+// edges read (= the out-degree sum of reached vertices), [2] = vertices reached.
 __global__ void __launch_bounds__(kSmallBlock) bfs_small_kernel(const uint32_t *__restrict__ rp,
                                                                 const uint32_t *__restrict__ col, uint32_t n,
-                                                                const uint32_t *__restrict__ seeds, uint32_t k,
+                                                                uint32_t lg, const uint32_t *__restrict__ seeds,
+                                                                uint32_t k, uint32_t seed1,
                                                                 int32_t *__restrict__ levels,
                                                                 unsigned long long *__restrict__ out) {
   __shared__ uint32_t s_rp[kSmallN + 1];
   __shared__ uint32_t s_vis[kSmallN / 32];
   __shared__ uint16_t s_q[2][kSmallN];
-  __shared__ uint32_t s_cnt[2];
+  __shared__ uint32_t s_cnt[3];  // frontier L's size, slot L % 3
   __shared__ unsigned long long s_red[kSmallBlock / kWave];
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = threadIdx.x, lane = lane_id();
   for (uint32_t i = t; i <= n; i += kSmallBlock) s_rp[i] = rp[i];
   for (uint32_t i = t; i < kSmallN / 32; i += kSmallBlock) s_vis[i] = 0u;
   for (uint32_t v = t; v < n; v += kSmallBlock) levels[v] = kInf;
-  if (t < 2) s_cnt[t] = 0u;
+  if (t < 3) s_cnt[t] = 0u;
   __syncthreads();
   for (uint32_t i = t; i < k; i += kSmallBlock) {
-    const uint32_t v = seeds[i], bit = 1u << (v & 31);
+    const uint32_t v = k == 1 ? seed1 : seeds[i], bit = 1u << (v & 31);
     if (!(atomicOr(&s_vis[v >> 5], bit) & bit)) {
       s_q[0][atomicAdd(&s_cnt[0], 1u)] = (uint16_t)v;
       levels[v] = 0;
     }
   }
   __syncthreads();
-  uint32_t cur = 0, L = 0;
+  uint32_t L = 0;
   unsigned long long insp = 0, reached = 0;
-  for (;;) {
-    const uint32_t qs = s_cnt[cur];
+  for (;; ++L) {
+    const uint32_t qs = s_cnt[L % 3], cur = L & 1, nxt = cur ^ 1, c3 = (L + 1) % 3;
     if (qs == 0 || L > n) break;
+    if (t == 0) s_cnt[(L + 2) % 3] = 0u;  // last read before the previous level's barrier
     reached += t < qs ? (qs - t + kSmallBlock - 1) / kSmallBlock : 0u;
-    if (t == 0) s_cnt[cur ^ 1] = 0u;
-    __syncthreads();
-    const uint32_t nxt = cur ^ 1;
-    for (uint32_t i = t; i < qs; i += kSmallBlock) {
-      const uint32_t u = s_q[cur][i];
-      const uint32_t b = s_rp[u], e = s_rp[u + 1];
-      insp += e - b;
-      for (uint32_t x = b; x < e; x += 4) {
-        uint32_t v[4];
+    // the unvisited among U targets of a lane (~0: none)
+    auto visit = [&](const auto &v) {
+      constexpr int U = sizeof(v) / 4;
+      bool mine[U];
+      uint32_t before[U], total = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = x + j < e ? col[x + j] : 0xffffffffu;
+      for (int j = 0; j < U; ++j) {
+        const uint32_t bit = 1u << (v[j] & 31);
+        mine[j] = v[j] != 0xffffffffu && !(s_vis[v[j] >> 5] & bit) && !(atomicOr(&s_vis[v[j] >> 5], bit) & bit);
+      }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (v[j] == 0xffffffffu) continue;
-          const uint32_t bit = 1u << (v[j] & 31);
-          if (s_vis[v[j] >> 5] & bit) continue;
-          if (!(atomicOr(&s_vis[v[j] >> 5], bit) & bit)) {
-            levels[v[j]] = (int32_t)(L + 1);
-            s_q[nxt][atomicAdd(&s_cnt[nxt], 1u)] = (uint16_t)v[j];
-          }
+      for (int j = 0; j < U; ++j) {
+        const uint64_t w = ballot(mine[j]);
+        before[j] = total + lane_rank(w);
+        total += (uint32_t)__popcll(w);
+      }
+      if (total == 0) return;
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&s_cnt[c3], total);
+      base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+      for (int j = 0; j < U; ++j)
+        if (mine[j]) {
+          levels[v[j]] = (int32_t)(L + 1);
+          s_q[nxt][base + before[j]] = (uint16_t)v[j];
+        }
+    };
+    const bool by_edge = (qs << lg) <= kSmallBlock;
+    const uint32_t g = by_edge ? lg : 0u;
+    for (uint32_t i = t >> g; i - (lane >> g) < qs; i += kSmallBlock >> g) {  // the same rounds for the whole wave
+      uint32_t x = 0, e = 0;
+      if (i < qs) {
+        const uint32_t u = s_q[cur][i];
+        x = s_rp[u] + (t & ((1u << g) - 1));
+        e = s_rp[u + 1];
+        if ((t & ((1u << g) - 1)) == 0) insp += e - x;
+      }
+      if (by_edge) {
+        for (; ballot(x < e); x += 1u << g) {
+          const uint32_t v[1] = {x < e ? col[x] : 0xffffffffu};
+          visit(v);
+        }
+      } else {
+        for (; ballot(x < e); x += 4) {
+          uint32_t v[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[j] = x + j < e ? col[x + j] : 0xffffffffu;
+          visit(v);
         }
       }
     }
-    __syncthreads();
-    cur = nxt;
-    ++L;
+    lds_barrier();
   }
+  if (!out) return;
   const unsigned long long ti = block_sum<kSmallBlock, unsigned long long>(insp, s_red);
   const unsigned long long tr = block_sum<kSmallBlock, unsigned long long>(reached, s_red);
   if (t == 0) {
@@ -869,28 +903,31 @@ static int bfs_small(const olv_graph *g, const std::vector<uint32_t> &seeds, int
                      olv_stats *st) {
   const uint32_t k = (uint32_t)seeds.size();
   DevBuf d_seeds, d_out, d_levels;
-  OLV_TRY(d_seeds.alloc((size_t)k * 4));
-  OLV_TRY(d_out.alloc(3 * sizeof(unsigned long long)));
-  OLV_HIP(hipMemcpyAsync(d_seeds.p, seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice, stream()));
+  if (k > 1) {
+    OLV_TRY(d_seeds.alloc((size_t)k * 4));
+    OLV_HIP(hipMemcpyAsync(d_seeds.p, seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice, stream()));
+  }
+  if (st) OLV_TRY(d_out.alloc(3 * sizeof(unsigned long long)));
   int32_t *outl = levels;
   if (host) {
     OLV_TRY(d_levels.alloc((size_t)g->n * 4));
     outl = d_levels.as<int32_t>();
   }
-  Timer t;
-  t.start();
-  hipLaunchKernelGGL(bfs_small_kernel, dim3(1), dim3(kSmallBlock), 0, stream(), g->row_ptr, g->col, g->n,
-                     d_seeds.as<uint32_t>(), k, outl, d_out.as<unsigned long long>());
+  uint32_t lg = 0;  // lanes per row: the mean degree rounded up to a power of two
+  while (lg < 6 && ((uint64_t)g->n << lg) < g->m) ++lg;
+  std::unique_ptr<Timer> t(st ? new Timer() : nullptr);
+  if (t) t->start();
+  hipLaunchKernelGGL(bfs_small_kernel, dim3(1), dim3(kSmallBlock), 0, stream(), g->row_ptr, g->col, g->n, lg,
+                     d_seeds.as<uint32_t>(), k, seeds[0], outl, d_out.as<unsigned long long>());
   OLV_HIP(hipGetLastError());
-  t.stop();
+  if (t) t->stop();
   unsigned long long h[3];
-  OLV_HIP(hipMemcpyAsync(h, d_out.p, sizeof(h), hipMemcpyDeviceToHost, stream()));
+  if (st) OLV_HIP(hipMemcpyAsync(h, d_out.p, sizeof(h), hipMemcpyDeviceToHost, stream()));
   OLV_HIP(hipStreamSynchronize(stream()));
-  if (h[0] > g->n) return fail(OLV_EINTERNAL, "olv_bfs: more than n levels");
   if (host) OLV_HIP(hipMemcpy(levels, outl, (size_t)g->n * 4, hipMemcpyDeviceToHost));
   if (st) {
     std::memset(st, 0, sizeof(*st));
-    st->elapsed_ms = t.ms();
+    st->elapsed_ms = t->ms();
     st->iterations = (uint32_t)h[0];
     st->edges_inspected = h[1];
     st->edges_traversed = h[1];

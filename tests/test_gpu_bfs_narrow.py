@@ -71,3 +71,19 @@ def test_narrow_levels(olv, name):
             _lib.check(_lib.lib().olv_plan_launch(plan, None), "launch")
             assert np.array_equal(lv.numpy(), ref), flags
         _lib.lib().olv_plan_destroy(plan)
+
+
+@pytest.mark.parametrize("extra", [0, 9000, 40000])  # mean degrees 2, 4 and 8: lanes per row 2, 4 and 8
+def test_small_graph_levels(olv, extra):
+    widths = [1, 3, 127, 128, 129, 255, 256, 257, 60, 511, 512, 513, 1023, 1024, 1025, 40, 64, 63, 65]
+    csr, src = layered(olv, widths, extra, seed=extra + 1)
+    assert csr.n <= 16384 and np.diff(csr.row_ptr.astype(np.int64)).max() <= 256  # for the small-graph kernel
+    ref = oracle.bfs(csr.row_ptr, csr.col, src)
+    g = olv.Graph(csr, transpose=False)
+    print("bfs small", extra, flush=True)
+    lv, st = g.bfs(src)
+    assert np.array_equal(lv.numpy(), ref)
+    assert (st.iterations, st.edges_inspected, st.vertices_reached) == (ref.max() + 1, csr.m, csr.n)
+    seeds = np.flatnonzero(ref == 5).astype(np.uint32)
+    want = np.min([oracle.bfs(csr.row_ptr, csr.col, int(s)) for s in seeds[:9]], axis=0)
+    assert np.array_equal(g.bfs_multisource(seeds[:9])[0].numpy(), want)
