@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
 #include <vector>
 
 #include "error.hpp"
@@ -70,6 +71,7 @@ constexpr uint32_t kHubThrMin = 256;  // smallest hub item (sizes the hub item b
 struct BfsWork;   // bfs.hip
 struct PrWork;    // pagerank.hip
 struct SsspWork;     // sssp.hip
+struct MbfsWork;     // batched.hip
 struct SsspBinWork;  // sssp_bin.hip
 
 }  // namespace olv
@@ -95,7 +97,8 @@ struct olv_graph {
   bool plan_in_ready = false, plan_out_ready = false;
   olv::BfsWork *bfs = nullptr;
   olv::PrWork *pr = nullptr;
-  olv::SsspWork *sssp = nullptr;         // direct SSSP work (for the last k sources)
+  std::atomic<olv::SsspWork *> sssp{nullptr};   // direct SSSP work (for the last k sources), while no call has it
+  std::atomic<olv::MbfsWork *> mbfs{nullptr};   // batched BFS work (for up to its k sources), while no call has it
   olv::SsspBinWork *sssp_bin = nullptr;  // binned SSSP work (for the last k sources)
   // In-degree numbering: vertices by descending in-degree, ties by id
   // (built on first use; shared by the PageRank pull and the BFS twin).
@@ -137,6 +140,7 @@ int noalloc_scratch(unsigned char **out);
 void free_pr_work(olv_graph *g);
 void free_sssp_bin(olv_graph *g);
 void free_sssp_work(olv_graph *g);
+void free_mbfs_work(olv_graph *g);
 // Binned SSSP (sssp_bin.hip): whether k instances of g take it, and its run
 // from device sources.
 bool sssp_bin_fits(const olv_graph *g, uint32_t k);
@@ -172,6 +176,28 @@ struct DevBuf {
 // olv_free_cached_memory() returns the cached blocks to the device.
 void *scratch_get(size_t bytes);
 void scratch_put(void *p);
+
+// A call's work buffers, kept with the graph between calls: taken out of the
+// graph's slot for the call's duration (a second thread's call on the graph
+// finds the slot empty and makes its own) and put back by keep() once the
+// call's stream has finished with them; freed if the call fails.
+template <class W>
+struct WorkLease {
+  std::atomic<W *> &slot;
+  W *w;
+  explicit WorkLease(std::atomic<W *> &s) : slot(s), w(s.exchange(nullptr)) {}
+  WorkLease(const WorkLease &) = delete;
+  WorkLease &operator=(const WorkLease &) = delete;
+  ~WorkLease() { delete w; }
+  void renew() {
+    delete w;
+    w = new W();
+  }
+  void keep() {
+    delete slot.exchange(w);
+    w = nullptr;
+  }
+};
 
 // RAII scratch buffer from the pool (for temporaries inside entry points).
 struct ScratchBuf {

@@ -400,6 +400,7 @@ static void graph_free(olv_graph *g) {
   free_bfs_work(g);
   free_pr_work(g);
   free_sssp_work(g);
+  free_mbfs_work(g);
   free_sssp_bin(g);
   g->plan_in.release();
   g->plan_out.release();

@@ -392,26 +392,7 @@ struct SsspWork {
   }
 };
 
-void free_sssp_work(olv_graph *g) {
-  delete g->sssp;
-  g->sssp = nullptr;
-}
-
-// The graph's work for k instances, published once complete.
-static int get_sssp_work(olv_graph *g, uint32_t k, SsspWork **out) {
-  if (!g->sssp || g->sssp->k != k) {
-    free_sssp_work(g);
-    SsspWork *w = new SsspWork();
-    const int rc = w->alloc((uint64_t)k * g->n, k, g->m);
-    if (rc != OLV_OK) {
-      delete w;
-      return rc;
-    }
-    g->sssp = w;
-  }
-  *out = g->sssp;
-  return OLV_OK;
-}
+void free_sssp_work(olv_graph *g) { delete g->sssp.exchange(nullptr); }
 
 static unsigned sgrid(size_t items, size_t per) {
   size_t b = (items + per - 1) / per;
@@ -505,8 +486,12 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   }
   // destination binning (sssp_bin.hip) unless asked to relax directly
   if (binned) return sssp_bin_run(g, ds.as<uint32_t>(), k, weights, dist, delta, flags, st);
-  SsspWork *w = nullptr;
-  OLV_TRY(get_sssp_work(gm, k, &w));
+  WorkLease<SsspWork> lease(gm->sssp);
+  if (!lease.w || lease.w->k != k) {
+    lease.renew();
+    OLV_TRY(lease.w->alloc(nv, k, g->m));
+  }
+  SsspWork *w = lease.w;
   SsspParams p;
   p.row_ptr = g->row_ptr;
   p.col = g->col;
@@ -589,7 +574,9 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
     st->iterations = w->h_ctl->rounds;
     st->edges_inspected = w->h_ctl->relax;
   }
-  if (w->h_ctl->capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after n=%u rounds (negative cycle)", g->n);
+  const bool capped = w->h_ctl->capped != 0;
+  lease.keep();  // the stream is idle: the control block has been read back
+  if (capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after n=%u rounds (negative cycle)", g->n);
   return OLV_OK;
 }
 
