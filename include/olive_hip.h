@@ -72,13 +72,15 @@ enum {
                                         the solver's slot order (ignored for
                                         host pointers or when no such copy is
                                         kept)                                    */
-#define OLV_SSSP_DIRECT      0x0800u /* olv_sssp, olv_sssp_batched: relax with a
-                                        dist probe and device-scope atomics per
-                                        edge instead of binning the candidates
-                                        by destination partition (kept to
-                                        compare; also taken when the binned
-                                        scheme does not fit: more than 2^25
-                                        virtual vertices or 2^32 bin entries) */
+#define OLV_SSSP_DIRECT      0x0800u /* olv_sssp, olv_sssp_batched: relax with
+                                        device-scope atomics per edge instead of
+                                        binning the candidates by destination
+                                        partition, also where the bins would be
+                                        used: from 1.25 M virtual vertices up,
+                                        on graphs without hubs (the direct
+                                        rounds also run what the bins cannot:
+                                        more than 2^25 virtual vertices or 2^32
+                                        bin entries) */
 
 /* weight dtypes for olv_graph_create */
 enum { OLV_W_NONE = 0, OLV_W_I32 = 1, OLV_W_F32 = 2 };
@@ -275,10 +277,11 @@ int olv_bfs_noalloc(const olv_graph *g, uint32_t src, int32_t *levels,
 /* SSSP distances over int32 weights (graph weights, or `weights` if not
  * NULL), INF = 0x7fffffff.  Frontier relaxation as SSSP.cu:146-163 with
  * cond(v, acc[v]) (SSSP.cu:72-75), run to the same fixed point in near-far
- * order; with non-negative weights each round's candidates are binned by
- * destination partition and min-reduced in LDS (OLV_SSSP_DIRECT: per-edge
- * probe and atomics instead).  The first binned call on a graph keeps its
- * bins (k x m pairs of 8 bytes) on the graph until olv_graph_destroy. */
+ * order; with non-negative weights the rounds of a large graph without hubs
+ * bin their candidates by destination partition and min-reduce them in LDS,
+ * the others relax with atomics (OLV_SSSP_DIRECT: all do).  The first binned
+ * call on a graph keeps its bins (k x m pairs of 8 bytes) on the graph until
+ * olv_graph_destroy, a direct call its queue, marks and candidate copies. */
 int olv_sssp(const olv_graph *g, uint32_t src, const int32_t *weights,
              int32_t *dist, unsigned flags, olv_stats *st);
 
@@ -385,8 +388,7 @@ typedef struct olv_tuning {
   uint32_t seg_bounds[3];           /* row pulls: 1 lane per row up to seg_bounds[0]
                                        entries, 8 lanes up to [1], a wave up to [2],
                                        then a workgroup                                  */
-  uint32_t sssp_relax_per_cu;       /* SSSP direct relaxation (OLV_SSSP_DIRECT)
-                                       workgroups per CU                                 */
+  uint32_t sssp_relax_per_cu;       /* SSSP direct relaxation: workgroups per CU         */
   uint32_t sssp_delta_num;          /* SSSP near-far step = mean weight x this / mean
                                        out-degree (1..1024; distances do not change)    */
   uint32_t source;                  /* 0 defaults, 1 measured by olv_autotune_ex, 2 read
