@@ -83,7 +83,7 @@ struct BfsWork {
   BfsCtl *h_ctl = nullptr;          // pinned mirror
   GridBar *bar = nullptr;           // persistent mode
   unsigned long long *stat = nullptr;
-  uint32_t recent[4] = {0, 0, 0, 0};  // launch pairs of the last runs (first chunk = their maximum)
+  uint32_t recent[4] = {0, 0, 0, 0};  // launch pairs that the last runs take (first chunk = their maximum)
   bool deep = false;                // the last run had many small levels: narrow launches from the start
   bool force_bu = false;            // OLV_FORCE_BOTTOM_UP of the current run
 };
@@ -764,7 +764,8 @@ static int run_pipeline(const olv_graph *g, BfsWork *w, int32_t *levels, bool ca
   w->recent[3] = w->recent[2];
   w->recent[2] = w->recent[1];
   w->recent[1] = w->recent[0];
-  w->recent[0] = w->h_ctl->pairs;
+  // a run that begins without the narrow kernel needs a pair for every level
+  w->recent[0] = w->deep ? w->h_ctl->pairs : w->h_ctl->levels;
   return OLV_OK;
 }
 
