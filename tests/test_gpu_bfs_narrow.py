@@ -87,3 +87,24 @@ def test_small_graph_levels(olv, extra):
     seeds = np.flatnonzero(ref == 5).astype(np.uint32)
     want = np.min([oracle.bfs(csr.row_ptr, csr.col, int(s)) for s in seeds[:9]], axis=0)
     assert np.array_equal(g.bfs_multisource(seeds[:9])[0].numpy(), want)
+
+
+@pytest.mark.parametrize("name", ["narrow", "queue_limit", "edge_limit", "hubs"])
+def test_narrow_levels_many_vertices(olv, name):
+    # more vertices than the bitmap in LDS holds: isolated ones between the others
+    from olive_amd import _lib
+
+    small, src = layered(olv, *CASES[name], seed=len(name))
+    step = 800_000 // small.n + 1
+    deg = np.zeros(small.n * step, np.int64)
+    deg[::step] = np.diff(small.row_ptr.astype(np.int64))
+    rp = np.concatenate([[0], np.cumsum(deg)]).astype(np.uint32)
+    csr = olv.CsrGraph(rp, small.col * np.uint32(step))
+    ref = oracle.bfs(csr.row_ptr, csr.col, src * step)
+    for flags in (0, _lib.OLV_GRAPH_ORDER, _lib.OLV_NO_DIRECTION_OPT):
+        g = olv.Graph(csr, transpose=True)
+        for run in range(3):
+            print("bfs narrow, many vertices", name, flags, run, flush=True)
+            lv, st = g.bfs(src * step, flags=flags)
+            assert np.array_equal(lv.numpy(), ref), (flags, run)
+            assert st.iterations == ref[ref < 0x7FFFFFFF].max() + 1
