@@ -33,6 +33,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 #include "bfs_core.hpp"
@@ -491,16 +492,16 @@ static unsigned bgrid(size_t items, size_t per) {
 }
 
 // Work for the fused rounds: region capacities (edges between every pair of
-// slices), their offsets, two pair stores and two count matrices.
+// slices), their offsets, two pair stores and two count matrices.  Published to
+// the graph only once the offsets are on the device: the rounds store pairs by
+// them.
 static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) {
-  SsspBinWork *w = g->sssp_bin;
-  if (w && w->k == k && w->sb == sb) {
-    *out = w;
+  if (g->sssp_bin && g->sssp_bin->k == k && g->sssp_bin->sb == sb) {
+    *out = g->sssp_bin;
     return OLV_OK;
   }
   free_sssp_bin(g);
-  w = new SsspBinWork();
-  g->sssp_bin = w;
+  std::unique_ptr<SsspBinWork> w(new SsspBinWork());
   w->k = k;
   w->sb = sb;
   w->nv = (uint64_t)k * g->n;
@@ -516,10 +517,8 @@ static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) 
       hipMalloc(reinterpret_cast<void **>(&w->cnt[0]), P2 * 4) != hipSuccess ||
       hipMalloc(reinterpret_cast<void **>(&w->cnt[1]), P2 * 4) != hipSuccess ||
       hipMalloc(reinterpret_cast<void **>(&w->fctl), sizeof(FusedCtl)) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void **>(&w->h_fctl), sizeof(FusedCtl), hipHostMallocDefault) != hipSuccess) {
-    free_sssp_bin(g);
+      hipHostMalloc(reinterpret_cast<void **>(&w->h_fctl), sizeof(FusedCtl), hipHostMallocDefault) != hipSuccess)
     return fail(OLV_ENOMEM, "olv_sssp: device allocation for the fused rounds failed");
-  }
   DevBuf cap;
   OLV_TRY(cap.alloc(P2 * 4));
   OLV_HIP(hipMemsetAsync(cap.p, 0, P2 * 4, stream()));
@@ -539,7 +538,7 @@ static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) 
     return fail(OLV_EINTERNAL, "olv_sssp: region capacities %llu != %llu edges", (unsigned long long)run,
                 (unsigned long long)k * g->m);
   OLV_HIP(hipMemcpy(w->base, hb.data(), (P2 + 1) * 4, hipMemcpyHostToDevice));
-  *out = w;
+  *out = g->sssp_bin = w.release();
   return OLV_OK;
 }
 

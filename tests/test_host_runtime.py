@@ -1,0 +1,120 @@
+"""Host code of the library on a runtime that keeps "device" memory on the heap
+and reports launches instead of running them (host_runtime.cpp): what a call
+leaves behind when an allocation fails, which kernels it launches and how many,
+and what memory stays with a graph.  CPU only; each test body runs in a child
+process with that runtime preloaded, its launch hook standing in for the kernels
+whose results the host reads."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes, struct, sys
+import numpy as np
+sys.path.insert(0, {root!r})
+rt = ctypes.CDLL({rt!r})
+rt.rt_live.restype = ctypes.c_size_t
+rt.rt_fail_at.argtypes = [ctypes.c_long]
+HOOK = ctypes.CFUNCTYPE(None, ctypes.c_char_p, ctypes.c_uint, ctypes.POINTER(ctypes.c_void_p))
+launched = []   # kernel names of the launches so far
+effects = {{}}    # substring of a kernel's name -> function(args)
+
+@HOOK
+def hook(name, grid, args):
+    name = name.decode()
+    launched.append(name)
+    for key, f in effects.items():
+        if key in name:
+            f(args)
+
+def count(key):
+    return sum(key in x for x in launched)
+
+def u64(p):
+    return ctypes.c_uint64.from_address(p)
+
+def u32(p):
+    return ctypes.c_uint32.from_address(p)
+
+rt.rt_hook(hook)
+import olive_amd
+from olive_amd import _lib
+from olive_amd._lib import lib
+olive_amd.init()
+
+def graph(n, m, weighted=True, transpose=False):
+    # all edges leave and enter vertex 0; no kernel looks at them here
+    rp = np.full(n + 1, m, np.uint32)
+    rp[0] = 0
+    w = np.ones(m, np.int32) if weighted else None
+    return olive_amd.Graph(olive_amd.CsrGraph(rp, np.zeros(m, np.uint32), w), transpose=transpose)
+
+def weights_of_one(args):  # wstat_kernel: minimum and sum of the weights
+    out, m = u64(args[2]).value, u32(args[1]).value
+    u64(out).value, u64(out + 8).value = 1, m
+effects["wstat_kernel"] = weights_of_one
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    rt = str(tmp_path_factory.mktemp("rt") / "libhostrt.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "host_runtime.cpp"), "-o", rt], check=True, timeout=120)
+
+    def go(body):
+        env = dict(os.environ)
+        env["LD_PRELOAD"] = " ".join(x for x in (rt, env.get("LD_PRELOAD")) if x)
+        code = PRELUDE.format(root=ROOT, rt=rt) + textwrap.dedent(body)
+        r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-4000:]
+        return r.stdout
+
+    return go
+
+
+# The binned SSSP rounds: their launch arguments are read back as the kernels
+# would (FusedArgs: base at byte 56, ctl at 80, nparts at 104; ctl: done first).
+BINNED = """
+n, m = 1_300_000, 40
+def caps(args):   # ssspf_cap_kernel: all edges go from the first slice to itself
+    u32(u64(args[7]).value).value = u32(args[3]).value * m
+bases = []
+def round_(args):
+    a = args[0]
+    base, ctl, nparts = u64(a + 56).value, u64(a + 80).value, u32(a + 104).value
+    bases.append((u32(base).value, u32(base + 4).value, u32(base + 4 * nparts * nparts).value))
+    u32(ctl).value = 1
+effects["ssspf_cap_kernel"] = caps
+effects["ssspf_round_kernel"] = round_
+out = olive_amd.DeviceBuffer(n, np.int32)
+def call(g, flags=0):
+    return lib().olv_sssp(g.h, 0, None, out.c, flags, None)
+"""
+
+
+def test_failed_sssp_bins_are_not_kept(run):
+    """Whichever allocation of a first binned call fails, the call says so and
+    the next one builds the bins anew: its rounds get the region offsets."""
+    run(BINNED + """
+g = graph(n, m)
+rt.rt_fail_at(0)
+assert call(g) == 0 and bases and set(bases) == {(0, m, m)}
+allocs = rt.rt_allocs()
+assert allocs > 8
+for i in range(1, allocs + 1):
+    g = graph(n, m)
+    live = rt.rt_live()
+    rt.rt_fail_at(i)
+    del bases[:]
+    assert call(g) != 0 and not bases, i
+    rt.rt_fail_at(0)
+    assert call(g) == 0 and bases and set(bases) == {(0, m, m)}, (i, bases[:1])
+    g.close()
+""")
