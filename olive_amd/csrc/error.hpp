@@ -8,9 +8,14 @@
 #include <cstdarg>
 #include <cstdio>
 
+#include "olive_hip.h"
+
 namespace olv {
 
 char *error_buffer();
+// Take the HIP error that a failed call left: hipGetLastError() keeps it until
+// asked, and the next entry point that checks its launches would report it.
+void clear_hip_error();
 
 // Record a formatted message and return `code`.
 inline int fail(int code, const char *fmt, ...) {
@@ -18,6 +23,7 @@ inline int fail(int code, const char *fmt, ...) {
   va_start(ap, fmt);
   std::vsnprintf(error_buffer(), 1024, fmt, ap);
   va_end(ap);
+  if (code == OLV_ENOMEM || code == OLV_EHIP) clear_hip_error();
   return code;
 }
 

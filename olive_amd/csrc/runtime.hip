@@ -20,6 +20,7 @@ namespace olv {
 
 static thread_local char g_err[1024] = "";
 char *error_buffer() { return g_err; }
+void clear_hip_error() { (void)hipGetLastError(); }
 
 static thread_local hipStream_t g_stream = nullptr;
 hipStream_t stream() { return g_stream; }

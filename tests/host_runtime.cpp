@@ -27,11 +27,12 @@ std::map<void *, size_t> &blocks() {
 std::vector<Config> g_config;
 void (*g_hook)(const char *name, unsigned grid, void **args) = nullptr;
 long g_allocs = 0, g_fail_at = 0;  // allocations so far; the one to fail (0: none)
+hipError_t g_last = hipSuccess;    // kept until hipGetLastError reports it
 size_t g_live = 0;
 
 hipError_t allocate(void **p, size_t bytes) {
   *p = nullptr;
-  if (++g_allocs == g_fail_at) return hipErrorOutOfMemory;
+  if (++g_allocs == g_fail_at) return g_last = hipErrorOutOfMemory;
   *p = std::calloc(1, bytes ? bytes : 1);
   if (!*p) return hipErrorOutOfMemory;
   blocks()[*p] = bytes;
@@ -96,7 +97,10 @@ hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { return *ms = 0.f, hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  return g_last = hipSuccess, e;
+}
 const char *hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipGetDevice(int *d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }

@@ -118,3 +118,22 @@ for i in range(1, allocs + 1):
     assert call(g) == 0 and bases and set(bases) == {(0, m, m)}, (i, bases[:1])
     g.close()
 """)
+
+
+def test_failed_allocation_is_reported_once(run):
+    """The runtime keeps a failed allocation as its last error until asked; the
+    call that failed takes it along, so the next call's launches are not blamed."""
+    run(BINNED + """
+g = graph(3000, 40)
+def done(args):   # SSSP by direct relaxation: the control block says done
+    u32(u64(args[0] + 64).value).value = 1
+effects["sssp_compact_kernel"] = done
+rt.rt_fail_at(0)
+assert call(g) == 0
+for i in range(1, rt.rt_allocs() + 1):
+    g = graph(3000, 40)
+    rt.rt_fail_at(i)
+    assert call(g) in (2, 3), i   # OLV_ENOMEM, OLV_EHIP
+    rt.rt_fail_at(0)
+    assert call(g) == 0, lib().olv_last_error()
+""")
