@@ -85,6 +85,13 @@ struct PrWork {
   float *wpiece[2] = {nullptr, nullptr};  // rl.blk_w[side].nweights floats each
   const float *wpiece_src[2] = {nullptr, nullptr};
   const uint32_t *wpiece_eid[2] = {nullptr, nullptr};
+  // The rows of the out-CSR that have entries, where fewer than half do (n = 0:
+  // not so): their ids and row offsets (n + 1).  For passes over tiles of edges.
+  struct {
+    uint32_t n = 0;
+    uint32_t *row = nullptr, *rp = nullptr;
+    bool ready = false;
+  } full;
   IterCtl *ctl = nullptr;
   IterCtl *h_ctl = nullptr;
   double *part = nullptr;  // per-workgroup partial sums (kPartials)
@@ -101,6 +108,8 @@ void free_pr_work(olv_graph *g) {
     if (p) (void)hipFree(p);
   for (float *p : w->wpiece)
     if (p) (void)hipFree(p);
+  if (w->full.row) (void)hipFree(w->full.row);
+  if (w->full.rp) (void)hipFree(w->full.rp);
   if (w->ctl) (void)hipFree(w->ctl);
   if (w->h_ctl) (void)hipHostFree(w->h_ctl);
   if (w->part) (void)hipFree(w->part);
@@ -213,6 +222,52 @@ static int ensure_side(olv_graph *g, PrWork *w, bool in_edges, bool with_eid) {
   OLV_HIP(hipGetLastError());
   OLV_HIP(hipStreamSynchronize(stream()));
   sd.ready = true;
+  return OLV_OK;
+}
+
+__global__ void row_full_kernel(const uint32_t *__restrict__ rp, uint32_t n, uint32_t *__restrict__ flag) {
+  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x)
+    flag[v] = rp[v + 1] > rp[v];
+}
+
+// row[i], out_rp[i] = id and first slot of the i-th row with entries (scan:
+// the exclusive sums of their flags).
+__global__ void full_rows_kernel(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ scan, uint32_t n,
+                                 uint32_t *__restrict__ row, uint32_t *__restrict__ out_rp) {
+  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (size_t)gridDim.x * blockDim.x) {
+    const uint32_t i = scan[v];
+    if (scan[v + 1] == i) continue;
+    row[i] = (uint32_t)v;
+    out_rp[i] = rp[v];
+    if (rp[v + 1] == rp[n]) out_rp[i + 1] = rp[n];
+  }
+}
+
+// w->full (built once): a tile of edges over many empty rows would have to
+// step over them in every backward pass.
+static int ensure_full_rows(const olv_graph *g, PrWork *w) {
+  if (w->full.ready || !g->m) return OLV_OK;
+  ScratchBuf scan;
+  OLV_TRY(scan.alloc(((size_t)g->n + 1) * 4));
+  uint32_t *sc = scan.as<uint32_t>(), count = 0;
+  hipLaunchKernelGGL(row_full_kernel, dim3(ew_grid(g->n)), dim3(256), 0, stream(), g->row_ptr, g->n, sc);
+  OLV_TRY(exclusive_scan(sc, sc, g->n));
+  OLV_HIP(hipMemcpyAsync(&count, sc + g->n, 4, hipMemcpyDeviceToHost, stream()));
+  OLV_HIP(hipStreamSynchronize(stream()));
+  if (count < g->n / 2) {
+    DevBuf row, rp;  // published once complete
+    OLV_TRY(row.alloc((size_t)count * 4));
+    OLV_TRY(rp.alloc(((size_t)count + 1) * 4));
+    hipLaunchKernelGGL(full_rows_kernel, dim3(ew_grid(g->n)), dim3(256), 0, stream(), g->row_ptr, sc, g->n,
+                       row.as<uint32_t>(), rp.as<uint32_t>());
+    OLV_HIP(hipGetLastError());
+    OLV_HIP(hipStreamSynchronize(stream()));
+    w->full.n = count;
+    w->full.row = row.as<uint32_t>();
+    w->full.rp = rp.as<uint32_t>();
+    row.p = rp.p = nullptr;
+  }
+  w->full.ready = true;
   return OLV_OK;
 }
 
@@ -357,10 +412,12 @@ struct AdjOp {
 // lambda in its numbering: a workgroup takes a tile of consecutive edges, so
 // the column reads and the gradient stores are whole lines: 132 us on RMAT-20,
 // bound by the gathers of lambda (walking the renumbered rows and storing
-// through each slot's edge id took 180).
+// through each slot's edge id took 180).  rp: offsets of the n rows row[0..n),
+// or (row null) of rows 0..n.
 __global__ void __launch_bounds__(kIB)
-    edge_grad_kernel(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col, uint32_t n, uint32_t m,
-                     const float *__restrict__ r, const float *__restrict__ lam, float d, float *__restrict__ grad_w) {
+    edge_grad_kernel(const uint32_t *__restrict__ rp, const uint32_t *__restrict__ row,
+                     const uint32_t *__restrict__ col, uint32_t n, uint32_t m, const float *__restrict__ r,
+                     const float *__restrict__ lam, float d, float *__restrict__ grad_w) {
   __shared__ uint32_t s_row[kITile];
   const uint32_t base = blockIdx.x * kITile, cnt = min(kITile, m - base);
   uint32_t v[kIItems];
@@ -376,7 +433,9 @@ __global__ void __launch_bounds__(kIB)
 #pragma unroll
   for (int i = 0; i < kIItems; ++i) {
     const uint32_t j = threadIdx.x + i * kIB;
-    if (j < cnt) grad_w[base + j] = d * r[first + s_row[j]] * lv[i];
+    if (j >= cnt) continue;
+    const uint32_t u = first + s_row[j];
+    grad_w[base + j] = d * r[row ? row[u] : u] * lv[i];
   }
 }
 
@@ -907,6 +966,7 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
   else OLV_TRY(ensure_plan(g, false));
   if (blocked) OLV_TRY(ensure_wblocked(g, w, 1));
   else if (relabel) OLV_TRY(ensure_side_plan(g, w->rl.out));
+  if (grad_w) OLV_TRY(ensure_full_rows(g, w));
   const SegDev d = make_seg_dev(relabel ? w->rl.out.plan : g->plan_out, g->tune);
   const uint32_t *rp = relabel ? w->rl.out.rp : g->row_ptr;
   const uint32_t *ci = relabel ? w->rl.out.col : g->col;
@@ -974,8 +1034,10 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
       gather_f32(lf, g->rl_pi, g->n, gb.as<float>());
       lo = gb.as<float>();
     }
+    const bool few = w->full.n != 0;
     hipLaunchKernelGGL(edge_grad_kernel, dim3((unsigned)(((size_t)g->m + kITile - 1) / kITile)), dim3(kIB), 0, stream(),
-                       g->row_ptr, g->col, g->n, g->m, dr, lo, damping, dgw);
+                       few ? w->full.rp : g->row_ptr, w->full.row, g->col, few ? w->full.n : g->n, g->m, dr, lo, damping,
+                       dgw);
   }
   if (dgt) {
     if (relabel) {

@@ -55,9 +55,15 @@ __device__ __forceinline__ uint32_t wave_row_of(const uint32_t *__restrict__ rp,
 }
 
 // Rows of the slots base .. base + cnt - 1 (0 < cnt <= kITile) of a CSR for a
-// workgroup of kIB lanes: slot base + j lies in row first + s_row[j].  Row
-// starts are marked in LDS and spread by a running maximum, so hub rows and
-// runs of empty rows cost no more than any others.  Returns `first`.
+// workgroup of kIB lanes: slot base + j lies in row first + s_row[j].  Returns
+// `first`.  Rows that start in the tile are marked in LDS -- the empty ones
+// aside, so no two at one slot -- and spread by a running maximum, so hub rows
+// cost no more than any others.  A tile over a long run of empty rows (a block
+// of ids without edges) does not walk it: every lane searches the row of the
+// first of its kIItems consecutive slots, then those of the others up to the
+// next lane's.
+constexpr uint32_t kIWalk = 8;           // rows in flight per lane
+constexpr uint32_t kIWalkRows = 1u << 16;  // rows between a tile's first and last that are walked, at most
 __device__ __forceinline__ uint32_t tile_rows(const uint32_t *__restrict__ rp, uint32_t n, uint32_t base, uint32_t cnt,
                                               uint32_t *s_row) {
   __shared__ uint32_t s_ends[2], s_w[kIWaves];
@@ -69,7 +75,38 @@ __device__ __forceinline__ uint32_t tile_rows(const uint32_t *__restrict__ rp, u
   for (uint32_t j = t; j < kITile; j += kIB) s_row[j] = 0u;
   __syncthreads();
   const uint32_t first = s_ends[0], last = s_ends[1];
-  for (uint64_t r = (uint64_t)first + 1 + t; r <= last; r += kIB) atomicMax(&s_row[rp[r] - base], (uint32_t)r - first);
+  if (last - first > kIWalkRows) {
+    const uint32_t j0 = t * kIItems;
+    uint32_t r0 = first;
+    for (uint32_t len = last - first + 1; len > 1; len -= len / 2)  // the row is in r0 .. r0 + len - 1
+      if (rp[r0 + len / 2] <= base + min(j0, cnt - 1)) r0 += len / 2;
+    s_row[j0] = r0 - first;
+    __syncthreads();
+    uint32_t r[kIItems];
+#pragma unroll
+    for (int i = 1; i < kIItems; ++i) r[i] = r0;
+    for (uint32_t len = (j0 + kIItems < kITile ? first + s_row[j0 + kIItems] : last) - r0 + 1; len > 1; len -= len / 2) {
+#pragma unroll
+      for (int i = 1; i < kIItems; ++i)
+        if (rp[r[i] + len / 2] <= base + min(j0 + i, cnt - 1)) r[i] += len / 2;
+    }
+#pragma unroll
+    for (int i = 1; i < kIItems; ++i) s_row[j0 + i] = r[i] - first;
+    __syncthreads();
+    return first;
+  }
+  for (uint32_t q = first + 1 + t; q <= last; q += kIWalk * kIB) {
+    uint32_t at[kIWalk], end[kIWalk];
+#pragma unroll
+    for (uint32_t i = 0; i < kIWalk; ++i) {
+      const uint32_t r = min(q + i * kIB, last);
+      at[i] = rp[r];
+      end[i] = rp[r + 1];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kIWalk; ++i)
+      if (end[i] > at[i] && q + i * kIB <= last) s_row[at[i] - base] = q + i * kIB - first;
+  }
   __syncthreads();
   uint32_t v[kIItems], run = 0;
 #pragma unroll
