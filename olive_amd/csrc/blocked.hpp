@@ -382,29 +382,33 @@ __global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, con
   const uint32_t nv = k >= 2 ? d.n_live : d.n;
   float err = 0.f;
   const uint32_t lane = threadIdx.x % kWave;
-  // U terms of a range from q on, `stride` apart, all in flight; 0 past end
-  auto terms = [&](auto u, uint32_t q, uint32_t stride, uint32_t end, float *p) {
+  // U terms, all in flight: term t at cmb_pos[at(t)] where in(t), else 0
+  auto gather = [&](auto u, auto at, auto in, float *p) {
     constexpr uint32_t U = decltype(u)::value;
     uint32_t ix[U];
     float w[kW ? U : 1];
 #pragma unroll
-    for (uint32_t t = 0; t < U; ++t) ix[t] = q + t * stride < end ? d.cmb_pos[q + t * stride] : 0u;
+    for (uint32_t t = 0; t < U; ++t) ix[t] = in(t) ? d.cmb_pos[at(t)] : 0u;
     if constexpr (kW) {  // beside a segment pass nearly every term is a partial: no weight to load
 #pragma unroll
       for (uint32_t t = 0; t < U; ++t) {
-        const bool has = kSolo ? q + t * stride < end : (q + t * stride < end && !(ix[t] & kIsPartial));
-        w[t] = has ? d.wcmb[q + t * stride] : 1.f;
+        const bool has = kSolo ? in(t) : (in(t) && !(ix[t] & kIsPartial));
+        w[t] = has ? d.wcmb[at(t)] : 1.f;
       }
     }
 #pragma unroll
     for (uint32_t t = 0; t < U; ++t) {
       const float *b = (ix[t] & kIsPartial) ? d.partial : src;
-      p[t] = q + t * stride < end ? b[ix[t] & ~kIsPartial] : 0.f;
+      p[t] = in(t) ? b[ix[t] & ~kIsPartial] : 0.f;
     }
     if constexpr (kW) {
 #pragma unroll
       for (uint32_t t = 0; t < U; ++t) p[t] *= w[t];
     }
+  };
+  // those of a range from q on, `stride` apart
+  auto terms = [&](auto u, uint32_t q, uint32_t stride, uint32_t end, float *p) {
+    gather(u, [&](uint32_t t) { return q + t * stride; }, [&](uint32_t t) { return q + t * stride < end; }, p);
   };
   using Per = std::integral_constant<uint32_t, kCmbPer>;
   uint32_t blk = blockIdx.x;
@@ -454,9 +458,9 @@ __global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, con
   } else {
     blk -= mid_blocks;
     const uint32_t nlb = gridDim.x - huge_blocks - big_blocks - mid_blocks;
-    for (uint32_t v = blk * 256 + threadIdx.x; v < nv; v += nlb * 256) {
+    auto one = [&](uint32_t v) {
       const uint32_t a = d.cmb_rp[v], b = d.cmb_rp[v + 1];
-      if (b - a > kCmbLight) continue;  // a listed row
+      if (b - a > kCmbLight) return;  // a listed row
       const auto pre = fin.pre(v);
       // the wave takes 4, 8 or 16 terms a lane by its longest row
       const bool over4 = ballot(b - a > 4) != 0, over8 = ballot(b - a > 8) != 0;
@@ -472,7 +476,49 @@ __global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, con
       else if (over4) run(std::integral_constant<uint32_t, 8>{});
       else run(std::integral_constant<uint32_t, 4>{});
       fin.finish(v, s, err, pre);
+    };
+    // R rows of the lane, `step` apart, of at most T terms each, all in flight.
+    // Where a lane has many short rows (millions of vertices of low degree) its
+    // rows one after another are a chain of offsets, places, terms and stores
+    // that does not keep HBM busy: an iteration on a path of 10 M vertices 109
+    // us row by row, 94 so; a 3000 x 3000 grid 111 and 98; the adjoint on 40 M
+    // vertices with 1 M edges 83 and 58.
+    const uint32_t step = nlb * 256;
+    auto rows = [&](auto r, auto per, uint32_t v, const uint32_t *a, const uint32_t *b) {
+      constexpr uint32_t R = decltype(r)::value, T = decltype(per)::value;
+      typename Fin::Pre pre[R];
+#pragma unroll
+      for (uint32_t i = 0; i < R; ++i) pre[i] = fin.pre(v + i * step);
+      float p[R * T];
+      gather(std::integral_constant<uint32_t, R * T>{}, [&](uint32_t t) { return a[t / T] + t % T; },
+             [&](uint32_t t) { return a[t / T] + t % T < b[t / T]; }, p);
+#pragma unroll
+      for (uint32_t i = 0; i < R; ++i) {
+        float s = 0.f;
+#pragma unroll
+        for (uint32_t t = 0; t < T; ++t) s += p[i * T + t];
+        fin.finish(v + i * step, s, err, pre[i]);
+      }
+    };
+    using R2 = std::integral_constant<uint32_t, 2>;
+    using R4 = std::integral_constant<uint32_t, 4>;
+    uint32_t v = blk * 256 + threadIdx.x;
+    for (; nv > 3 * step && v < nv - 3 * step; v += 4 * step) {
+      uint32_t a[4], b[4], most = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) a[i] = d.cmb_rp[v + i * step], b[i] = d.cmb_rp[v + i * step + 1];
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) most = max(most, b[i] - a[i]);
+      if (!ballot(most > 2)) {
+        rows(R4{}, R2{}, v, a, b);
+      } else if (!ballot(most > 4)) {
+        rows(R2{}, R4{}, v, a, b);
+        rows(R2{}, R4{}, v + 2 * step, a + 2, b + 2);
+      } else {
+        for (uint32_t i = 0; i < 4; ++i) one(v + i * step);
+      }
     }
+    for (; v < nv; v += step) one(v);
   }
   err = block_sum<256, float>(err, s_red);
   if (threadIdx.x == 0 && err != 0.f) atomicAdd(&ctl->errs[k % 3][blockIdx.x % kErrSlots].v, (double)err);

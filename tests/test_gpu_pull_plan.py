@@ -60,6 +60,9 @@ CASES = {
     "segment_plus_one": (32769, 520000, 20000),
     "single_launch": (100003, 300000, 16384),
     "few_edges_long_row": (100003, 1000, 70000),
+    # lanes with four short rows and more: groups of them of at most two, at
+    # most four and more terms
+    "many_short_rows": (2200003, 3000000, 50000),
 }
 
 
