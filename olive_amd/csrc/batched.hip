@@ -1111,7 +1111,8 @@ int olv_plan_bfs(const olv_graph *g, const uint32_t *srcs, uint32_t k, int32_t *
   p->can_bu = !(flags & OLV_NO_DIRECTION_OPT);
   int s = bfs_prepare(g, p->can_bu, &p->bw);
   if (s == OLV_OK)  // on g itself: its work buffers keep the depth the capture uses
-    s = bfs_multisource(g, srcs, k, true, levels, (flags & ~(OLV_PTR_HOST | OLV_PERSISTENT)) | OLV_GRAPH_ORDER, nullptr);
+    s = bfs_multisource(g, srcs, k, true, levels, (flags & ~(OLV_PTR_HOST | OLV_PERSISTENT | OLV_HOST_LOOP)) | OLV_GRAPH_ORDER,
+                        nullptr);
   if (s == OLV_OK) s = p->seeds.alloc((size_t)k * 4);
   if (s == OLV_OK && hipMemcpy(p->seeds.p, srcs, (size_t)k * 4, hipMemcpyHostToDevice) != hipSuccess)
     s = fail(OLV_EHIP, "olv_plan_bfs: seed copy failed");

@@ -83,8 +83,14 @@ struct BfsWork {
   BfsCtl *h_ctl = nullptr;          // pinned mirror
   GridBar *bar = nullptr;           // persistent mode
   unsigned long long *stat = nullptr;
-  uint32_t recent[4] = {0, 0, 0, 0};  // launch pairs that the last runs take (first chunk = their maximum)
-  bool deep = false;                // the last run had many small levels: narrow launches from the start
+  // launch pairs that the last runs take (first chunk = their maximum) and
+  // whether the last one had many small levels: narrow launches from the start.
+  // Of runs that could launch the narrow kernel only
+  uint32_t recent[4] = {0, 0, 0, 0};
+  bool deep = false;
+  // the same of the last run, whatever its flags (for a plan's capture)
+  uint32_t last_pairs = 0;
+  bool last_narrow = true;
   bool force_bu = false;            // OLV_FORCE_BOTTOM_UP of the current run
 };
 
@@ -733,22 +739,28 @@ bool bfs_done(BfsWork *w) { return w->h_ctl->done != 0; }
 // Launch pairs that a run like the last one takes, and whether it begins with
 // a narrow launch (so it does where no run went through launch pairs: a graph
 // for bfs_small).
-uint32_t bfs_pairs_hint(const BfsWork *w) { return std::max(1u, w->recent[0]); }
-bool bfs_deep_hint(const BfsWork *w) { return w->deep || w->recent[0] == 0; }
+uint32_t bfs_pairs_hint(const BfsWork *w) { return std::max(1u, w->last_pairs); }
+bool bfs_deep_hint(const BfsWork *w) { return w->last_narrow; }
 
 // Enqueue launch pairs in growing chunks until the device reports done; one
 // host round trip per level if `host_loop`.  The narrow kernel joins from the
 // second chunk on, or from the first where the last run on this graph ran
 // kDeepLevels levels in it: on a shallow graph a launch that finds a wide
-// frontier costs 2 us for nothing.  The stop event of `t` follows the last
-// enqueued level, ahead of the control block read-back, so host latency after
-// the last kernel is not timed (the gaps between chunks are).
+// frontier costs 2 us for nothing.  A first chunk without it has kShallowPairs
+// pairs at most, so that no run of many levels ends before the kernel has been
+// asked: one that did would leave the next run without it as well.  The stop
+// event of `t` follows the last enqueued level, ahead of the control block
+// read-back, so host latency after the last kernel is not timed (the gaps
+// between chunks are).
 constexpr uint32_t kDeepLevels = 8;
+constexpr uint32_t kShallowPairs = 32;
 
 static int run_pipeline(const olv_graph *g, BfsWork *w, int32_t *levels, bool can_bu, uint32_t chunk0, bool host_loop,
                         Timer *t) {
-  uint32_t chunk = host_loop ? 1u : chunk0;
-  bool narrow = !host_loop && w->deep;
+  const bool may_narrow = !host_loop && !w->force_bu;
+  bool narrow = may_narrow && w->deep;
+  uint32_t chunk = host_loop ? 1u : (narrow || !may_narrow ? chunk0 : std::min(chunk0, kShallowPairs));
+  uint32_t rest = host_loop ? 0u : chunk0 - chunk, more = 4;
   uint64_t enq = 0;
   for (;;) {
     OLV_TRY(bfs_enqueue_levels(g, w, levels, can_bu, chunk, narrow));
@@ -757,15 +769,17 @@ static int run_pipeline(const olv_graph *g, BfsWork *w, int32_t *levels, bool ca
     OLV_TRY(bfs_result(w, nullptr, nullptr));
     if (w->h_ctl->done) break;
     if (enq > (uint64_t)g->n + 2) return fail(OLV_EINTERNAL, "olv_bfs: level loop did not terminate");
-    if (!host_loop) chunk = std::min(std::max(chunk, 2u) * 2, 256u);
-    narrow = !host_loop;
+    if (rest) chunk = rest, rest = 0;
+    else if (!host_loop) chunk = more = std::min(more * 2, 256u);
+    narrow = may_narrow;
   }
-  if (!host_loop && !w->force_bu) w->deep = w->h_ctl->nlevels >= kDeepLevels;
-  w->recent[3] = w->recent[2];
-  w->recent[2] = w->recent[1];
-  w->recent[1] = w->recent[0];
+  w->last_narrow = may_narrow && w->h_ctl->nlevels >= kDeepLevels;
   // a run that begins without the narrow kernel needs a pair for every level
-  w->recent[0] = w->deep ? w->h_ctl->pairs : w->h_ctl->levels;
+  w->last_pairs = w->last_narrow ? w->h_ctl->pairs : w->h_ctl->levels;
+  if (!may_narrow) return OLV_OK;
+  w->deep = w->last_narrow;
+  for (int i = 3; i > 0; --i) w->recent[i] = w->recent[i - 1];
+  w->recent[0] = w->last_pairs;
   return OLV_OK;
 }
 

@@ -137,3 +137,67 @@ for i in range(1, rt.rt_allocs() + 1):
     rt.rt_fail_at(0)
     assert call(g) == 0, lib().olv_last_error()
 """)
+
+
+# BFS: a traversal of `depth` levels.  A narrow launch runs what is left of it,
+# a launch pair one level (BfsCtl: done, skip, level, level_e, pairs, nlevels,
+# levels).
+BFS = """
+FLAGS = _lib.OLV_GRAPH_ORDER | _lib.OLV_NO_DIRECTION_OPT
+n = 20_000
+depth = 300
+def ctl_of(args, at):
+    return u64(args[at]).value
+def reset(args):
+    for i in range(7):
+        u32(ctl_of(args, 7) + 4 * i).value = 0
+def finish(c):
+    u32(c + 24).value, u32(c).value = depth, 1
+def narrow(args):
+    c = ctl_of(args, 1)
+    if not u32(c).value:
+        u32(c + 20).value += depth - u32(c + 8).value
+        finish(c)
+def compact(args):
+    c = ctl_of(args, 1)
+    if u32(c).value:
+        return
+    u32(c + 8).value += 1
+    u32(c + 16).value += 1
+    if u32(c + 8).value == depth:
+        finish(c)
+effects.update(bfs_reset_kernel=reset, bfs_narrow_kernel=narrow, bfs_compact_kernel=compact)
+out = olive_amd.DeviceBuffer(n, np.int32)
+def call(g, flags=0):
+    del launched[:]
+    assert lib().olv_bfs(g.h, 0, out.c, FLAGS | flags, None) == 0, lib().olv_last_error()
+    return count("bfs_compact"), count("bfs_narrow")
+"""
+
+
+@pytest.mark.parametrize("flags", [0, 0x8, 0x4])  # OLV_HOST_LOOP, OLV_FORCE_BOTTOM_UP
+def test_history_leads_to_the_narrow_kernel(run, flags):
+    """Whatever kind of call comes first on a graph of many small levels, plain
+    calls run it in the narrow kernel, and enqueue no pairs for the others."""
+    run(BFS + f"flags = {flags}" + """
+if flags & _lib.OLV_FORCE_BOTTOM_UP:
+    FLAGS = _lib.OLV_GRAPH_ORDER
+g = graph(n, 40, weighted=False, transpose=True)
+for _ in range(2):
+    if flags:
+        pairs, launches = call(g, flags)
+        assert pairs >= depth and launches == 0
+    for _ in range(3):
+        pairs, launches = call(g)
+        assert pairs <= 12 and launches, (pairs, launches)
+# levels too wide for the narrow kernel, then the first again
+effects["bfs_narrow_kernel"] = lambda args: None
+for _ in range(5):
+    call(g)
+pairs, launches = call(g)
+assert pairs == depth and launches   # no surplus
+effects["bfs_narrow_kernel"] = narrow
+for _ in range(5):
+    call(g)
+assert call(g)[0] <= 4
+""")
