@@ -231,8 +231,9 @@ struct BfsDir {
 // L & 1; reset the next level's fill counters.
 template <bool Mapped>
 __global__ void __launch_bounds__(kBlock) bfs_expand_kernel(BfsArgs a, BfsCtl *ctl, uint32_t *bms, uint32_t nwp) {
-  if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
-  if (ctl->skip) return;
+  // (both written by earlier launches; loaded together, one after the other
+  // would cost a level another trip to the cache)
+  if ((ctl->done | ctl->skip) != 0) return;
   const uint32_t L = ctl->level;
   const BfsState st = ctl->st[L & 1];
   const uint32_t qsize = ctl->qfill[L & 1], nhubs = ctl->hfill[L & 1];

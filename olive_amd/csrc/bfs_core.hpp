@@ -165,7 +165,8 @@ __device__ void push_expand(const uint32_t *queue, uint32_t qsize, const uint2 *
   const uint32_t lg = qsize >= 16 * nvb ? 4u : (qsize >= 4 * nvb ? 2u : 0u);
   const uint32_t runs = (qsize + (1u << lg) - 1) >> lg;
   const uint32_t per = ((runs + nvb - 1) / nvb) << lg;  // entries of a workgroup
-  for (uint32_t base = 0; base < per; base += BLOCK) {
+  // (a workgroup without entries leaves before the barriers)
+  for (uint32_t base = 0; base < per && (vb << lg) < qsize; base += BLOCK) {
     const uint32_t j = base + threadIdx.x;
     const uint64_t i = (((uint64_t)(j >> lg) * nvb + vb) << lg) + (j & ((1u << lg) - 1));
     uint32_t beg = 0, end = 0;
