@@ -806,10 +806,12 @@ static int mbfs_pull_plan(olv_graph *g, unsigned flags, SegDev *d) {
   return OLV_OK;
 }
 
-// Run one group to completion (levels enqueued in growing chunks).
+// Run one group to completion: levels enqueued in chunks, the first as long as
+// the last group was deep (of this call or the one before), those after it 8,
+// 16, ...: groups of one graph differ by a few levels.
 static int mbfs_run_group(const MbfsParams &p, const SegDev &d, MbfsWork &w, const uint32_t *d_srcs) {
   OLV_TRY(mbfs_enqueue_init(p, d_srcs));
-  uint32_t chunk = std::max(4u, w.last_levels);
+  uint32_t chunk = std::max(4u, w.last_levels), more = 4;
   uint64_t enq = 0;
   for (;;) {
     OLV_TRY(mbfs_enqueue_levels(p, d, chunk));
@@ -817,7 +819,7 @@ static int mbfs_run_group(const MbfsParams &p, const SegDev &d, MbfsWork &w, con
     OLV_TRY(mbfs_read(w));
     if (w.h_ctl->done) break;
     if (enq > (uint64_t)p.n + 2) return fail(OLV_EINTERNAL, "olv_bfs_batched: level loop did not terminate");
-    chunk = std::min(chunk * 2, 256u);
+    chunk = more = std::min(more * 2, 256u);
   }
   if (w.h_ctl->overflow) return fail(OLV_EINTERNAL, "olv_bfs_batched: more than n levels");
   w.last_levels = w.h_ctl->levels;

@@ -201,3 +201,34 @@ for _ in range(5):
     call(g)
 assert call(g)[0] <= 4
 """)
+
+
+def test_batched_groups_of_unlike_depth(run):
+    """Groups of a batched BFS whose depths differ by a few levels: no group
+    enqueues many launches past its end (MbfsParams: k at byte 44, ctl at 184;
+    MbfsCtl: level, -, done, levels)."""
+    run("""
+depth = {256: 130, 44: 128}
+def reset(args):
+    c = u64(args[0] + 184).value
+    for i in range(4):
+        u32(c + 4 * i).value = 0
+def compact(args):
+    c, d = u64(args[0] + 184).value, depth[u32(args[0] + 44).value]
+    if u32(c + 8).value:
+        return
+    u32(c).value += 1
+    if u32(c).value == d:
+        u32(c + 12).value, u32(c + 8).value = d, 1
+effects.update(mbfs_reset_kernel=reset, mbfs_compact_kernel=compact)
+n = 500
+g = graph(n, 40, weighted=False, transpose=True)
+srcs = np.zeros(300, np.uint32)
+out = olive_amd.DeviceBuffer(300 * n, np.int32)
+for i in range(4):
+    del launched[:]
+    assert lib().olv_bfs_batched(g.h, srcs.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), 300, out.c,
+                                 _lib.OLV_GRAPH_ORDER | _lib.OLV_NO_DIRECTION_OPT, None) == 0, lib().olv_last_error()
+    if i:
+        assert 258 <= count("mbfs_compact") <= 258 + 20, (i, count("mbfs_compact"))
+""")
