@@ -59,11 +59,17 @@ constexpr uint8_t kMarkNew = 1, kMarkFar = 2;
 // graph many relaxations improve on the same hub, so workgroup b lowers copy
 // b % kCopies; the compaction, a launch later, takes the smallest of a marked
 // vertex's copies.  RMAT 250K x 4M: 601 us lowering dist itself, 502, 474, 452,
-// 455 with 1, 2, 4, 8 copies; RMAT 1M x 16M: 1095 and 959.  Past 1M vertices
-// the copies no longer stay cached (2M x 16M: 1458 and 1418; 4M x 32M: 1532
-// and 2040), so relaxations lower dist there.
+// 455 with 1, 2, 4, 8 copies; RMAT 1M x 8M 605 and 582.  Past 1M vertices the
+// copies no longer stay cached (RMAT 2M x 16M: 1458 and 1418; 4M x 32M: 1532 and
+// 2040), and without hubs they gain nothing from 600K on (uniform, 8 edges a
+// vertex: 500K 743 and 674 us, 700K 780 and 765, 800K 769 and 788, 1M 882 and
+// 947), so relaxations lower dist there.
 constexpr uint32_t kCopies = 4;
-constexpr uint64_t kCopiesMaxVertices = 1u << 20;
+constexpr uint64_t kCopiesHubs = 1u << 20, kCopiesNoHubs = 600000;  // vertices, at most
+constexpr uint32_t kWideWords = 4;  // words of mark bytes a lane compacts without copies
+static bool with_copies(const olv_graph *g, uint64_t nv) {
+  return nv <= (g->max_outdeg >= g->tune.hub_thr ? kCopiesHubs : kCopiesNoHubs);
+}
 
 template <bool Multi, bool Copies>
 struct SsspVisitor {
@@ -111,7 +117,10 @@ struct SsspVisitor {
 enum : uint32_t { kModeNear = 0, kModeResplit = 1, kModeDone = 2 };
 
 // Smallest marked distance at or above the split, one copy per 128-byte line
-// (workgroup b updates copy b % kCtrSlots).
+// (workgroup b updates copy b % kCtrSlots).  Exact after a round that moved the
+// split; until the next one it may stand for a vertex that has since been
+// lowered below the split, and a re-split from it then promotes less, at worst
+// nothing, and leaves the exact one.
 struct alignas(128) MinSlot {
   int32_t v;
   uint32_t pad[31];
@@ -167,11 +176,31 @@ __device__ __forceinline__ void sssp_round(const SsspParams &p, uint32_t qsize, 
 }
 
 // Marked vertices with a distance below `split` -> queue and hub items (their
-// marks cleared); the smallest other marked distance -> *minfar.  A lane
-// takes the mark bytes of four vertices.
-template <int BLOCK>
-__device__ void sssp_take(const SsspParams &p, int32_t split, uint32_t *qcount, uint32_t *hcount, int32_t *minfar,
-                          uint32_t vb, uint32_t nvb) {
+// marks cleared); the smallest other marked distance -> *minfar.  Where the
+// split has not moved (`all` false) vertices marked far stay so, and only those
+// lowered since are looked at.  A lane takes W consecutive words of four mark
+// bytes.  W = 1 with candidate copies, where a vertex costs five loads and lanes
+// are few; else W = kWideWords, and a workgroup collects its vertices in LDS: its place in the queue comes from an atomic, and one for every 1024
+// vertices, 12 ns each after another, made a compaction of 16.7M vertices 195
+// us whatever it found (85 to 110 with W = 4, 25 to 50 collected and without the
+// far ones).  Relaxed directly, 16.7M vertices with 67M edges 8.4 -> 4.8 ms a
+// call, 5M with 40M 3.33 -> 2.46.
+template <int BLOCK, uint32_t W>
+__device__ void sssp_take(const SsspParams &p, int32_t split, bool all, uint32_t *qcount, uint32_t *hcount,
+                          int32_t *minfar, uint32_t vb, uint32_t nvb) {
+  const uint32_t look = all ? 0xffffffffu : 0x01010101u * kMarkNew;
+  constexpr uint32_t kHold = W > 1 ? BLOCK * 4 * W : 1;
+  __shared__ uint32_t s_hold[kHold];
+  uint32_t held = 0;  // entries in s_hold
+  auto flush = [&]() {
+    __shared__ uint32_t s_at;
+    __syncthreads();
+    if (threadIdx.x == 0) s_at = atomicAdd(qcount, held);
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < held; i += BLOCK) p.queue[s_at + i] = s_hold[i];
+    __syncthreads();
+    held = 0;
+  };
   __shared__ uint32_t s_scan[BLOCK / kWave + 1];
   __shared__ uint32_t s_base;
   __shared__ int32_t s_mf[BLOCK / kWave];
@@ -179,18 +208,24 @@ __device__ void sssp_take(const SsspParams &p, int32_t split, uint32_t *qcount, 
   const uint32_t nw = (p.nv + 3) / 4;
   uint32_t *words = reinterpret_cast<uint32_t *>(p.mark);
   int32_t mf = kInf;
-  for (uint32_t w0 = vb * BLOCK; w0 < nw; w0 += nvb * BLOCK) {
-    const uint32_t w = w0 + threadIdx.x;
-    const uint32_t word = w < nw ? words[w] : 0u;
-    uint32_t keep = word, take = 0;  // take: bit b, vertex 4 w + b goes to the queue
-    if (word) {
+  for (uint64_t w0 = (uint64_t)vb * BLOCK * W; w0 < nw; w0 += (uint64_t)nvb * BLOCK * W) {
+    const uint32_t wl = (uint32_t)w0 + threadIdx.x * W;  // this lane's first word
+    uint32_t word[W], take = 0;  // take: bit b, vertex 4 wl + b goes to the queue
+#pragma unroll
+    for (uint32_t i = 0; i < W; ++i) word[i] = wl + i < nw ? words[wl + i] : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < W; ++i) {
+      const uint32_t seen = word[i] & look;
+      if (!seen) continue;
+      const uint32_t w = wl + i;
+      uint32_t keep = word[i];
       int32_t d[4];
 #pragma unroll
-      for (int b = 0; b < 4; ++b) d[b] = (word >> (8 * b)) & 0xffu ? p.dist[w * 4u + b] : kInf;
+      for (int b = 0; b < 4; ++b) d[b] = (seen >> (8 * b)) & 0xffu ? p.dist[w * 4u + b] : kInf;
       if (p.cand) {
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
-          if (((word >> (8 * b)) & 0xffu) != kMarkNew) continue;
+          if (!((seen >> (8 * b)) & kMarkNew)) continue;
           int32_t c[kCopies], m = d[b];
 #pragma unroll
           for (uint32_t x = 0; x < kCopies; ++x) c[x] = p.cand[(size_t)x * p.nv + w * 4u + b];
@@ -201,7 +236,7 @@ __device__ void sssp_take(const SsspParams &p, int32_t split, uint32_t *qcount, 
       }
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        if (!((word >> (8 * b)) & 0xffu)) continue;
+        if (!((seen >> (8 * b)) & 0xffu)) continue;
         keep &= ~(0xffu << (8 * b));
         if (d[b] >= split) {
           mf = d[b] < mf ? d[b] : mf;
@@ -215,19 +250,27 @@ __device__ void sssp_take(const SsspParams &p, int32_t split, uint32_t *qcount, 
           const uint32_t hb = atomicAdd(hcount, k);
           for (uint32_t j = 0; j < k; ++j) p.hubs[hb + j] = make_uint2(x, j);
         } else {
-          take |= 1u << b;
+          take |= 1u << (4 * i + b);
         }
       }
-      if (keep != word) words[w] = keep;
+      if (keep != word[i]) words[w] = keep;
     }
     uint32_t total;
     const uint32_t off = block_exclusive_scan<BLOCK>((uint32_t)__popc(take), s_scan, &total);
-    if (threadIdx.x == 0) s_base = total ? atomicAdd(qcount, total) : 0u;
-    __syncthreads();
-    uint32_t pos = s_base + off;
-    for (uint32_t x = take; x; x &= x - 1) p.queue[pos++] = w * 4u + __ffs(x) - 1;
-    __syncthreads();
+    if constexpr (W > 1) {
+      if (held + total > kHold) flush();
+      uint32_t pos = held + off;
+      for (uint32_t x = take; x; x &= x - 1) s_hold[pos++] = wl * 4u + __ffs(x) - 1;
+      held += total;
+    } else {
+      if (threadIdx.x == 0) s_base = total ? atomicAdd(qcount, total) : 0u;
+      __syncthreads();
+      uint32_t pos = s_base + off;
+      for (uint32_t x = take; x; x &= x - 1) p.queue[pos++] = wl * 4u + __ffs(x) - 1;
+      __syncthreads();
+    }
   }
+  if (held) flush();
   mf = wave_min(mf);
   if (lane_id() == 0) s_mf[threadIdx.x / kWave] = mf;
   __syncthreads();
@@ -248,13 +291,14 @@ __global__ void __launch_bounds__(kSBlock) sssp_relax_kernel(SsspParams p) {
   const uint32_t qsize = ctl->qfill[R & 1], nhubs = ctl->hfill[R & 1];
   if (blockIdx.x == 0) {
     __shared__ int32_t s_mf;
+    const int32_t far = t < kCtrSlots ? ctl->minfar[R & 1][t].v : kInf;
     if (t < kWave) {
-      const int32_t mf = wave_min(t < kCtrSlots ? ctl->minfar[R & 1][t].v : kInf);
+      const int32_t mf = wave_min(far);
       if (t == 0) s_mf = mf;
     }
     __syncthreads();
+    const uint32_t mode = (qsize + nhubs) ? kModeNear : (s_mf < kInf ? kModeResplit : kModeDone);
     if (t == 0) {
-      const uint32_t mode = (qsize + nhubs) ? kModeNear : (s_mf < kInf ? kModeResplit : kModeDone);
       const int32_t split = ctl->split[R & 1];
       ctl->round_e = R;
       ctl->mode[R & 1] = mode;
@@ -267,7 +311,7 @@ __global__ void __launch_bounds__(kSBlock) sssp_relax_kernel(SsspParams p) {
         ctl->done = 1u;
       }
     }
-    if (t < kCtrSlots) ctl->minfar[(R + 1) & 1][t].v = kInf;
+    if (t < kCtrSlots) ctl->minfar[(R + 1) & 1][t].v = mode == kModeNear ? far : kInf;
   }
   if (qsize + nhubs == 0 || R >= p.max_rounds) return;
   unsigned long long insp = 0;
@@ -275,6 +319,7 @@ __global__ void __launch_bounds__(kSBlock) sssp_relax_kernel(SsspParams p) {
   flush_counters<kSBlock>(&ctl->cnt[R & 1], 0u, 0ull, insp);
 }
 
+template <uint32_t W>
 __global__ void __launch_bounds__(kSBlock) sssp_compact_kernel(SsspParams p) {
   SsspCtl *ctl = p.ctl;
   if (__hip_atomic_load(&ctl->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
@@ -287,8 +332,9 @@ __global__ void __launch_bounds__(kSBlock) sssp_compact_kernel(SsspParams p) {
     }
     ctr_clear(&ctl->cnt[(R + 1) & 1]);
   }
-  sssp_take<kSBlock>(p, ctl->split[(R + 1) & 1], &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1],
-                     &ctl->minfar[(R + 1) & 1][blockIdx.x % kCtrSlots].v, blockIdx.x, gridDim.x);
+  sssp_take<kSBlock, W>(p, ctl->split[(R + 1) & 1], ctl->mode[R & 1] != kModeNear, &ctl->qfill[(R + 1) & 1],
+                        &ctl->hfill[(R + 1) & 1], &ctl->minfar[(R + 1) & 1][blockIdx.x % kCtrSlots].v, blockIdx.x,
+                        gridDim.x);
 }
 
 // All rounds (plain: every marked vertex is expanded) in one cooperative
@@ -318,7 +364,7 @@ __global__ void __launch_bounds__(kSBlock) sssp_persistent_kernel(SsspParams p) 
     }
     sssp_round<Multi, false>(p, qsize, nhubs, vb, nvb, insp);
     if (!grid_barrier(p.bar, gb, kSSpin)) break;
-    sssp_take<kSBlock>(p, kInf, &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1], &ctl->minfar[0][vb % kCtrSlots].v, vb,
+    sssp_take<kSBlock, 1>(p, kInf, true, &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1], &ctl->minfar[0][vb % kCtrSlots].v, vb,
                        nvb);
     if (!grid_barrier(p.bar, gb, kSSpin)) break;
   }
@@ -379,11 +425,11 @@ struct SsspWork {
       if (p) (void)hipFree(p);
     if (h_ctl) (void)hipHostFree(h_ctl);
   }
-  int alloc(uint64_t nv, uint32_t kk, uint64_t m) {
+  int alloc(uint64_t nv, uint32_t kk, uint64_t m, bool copies) {
     k = kk;
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&queue), (size_t)nv * 4));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&mark), ((size_t)nv + 3) / 4 * 4));
-    if (nv <= kCopiesMaxVertices) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&cand), (size_t)nv * kCopies * 4));
+    if (copies) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&cand), (size_t)nv * kCopies * 4));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&hubs), hub_capacity(m) * k * sizeof(uint2)));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&ctl), sizeof(SsspCtl)));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&bar), sizeof(GridBar)));
@@ -487,9 +533,10 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   // destination binning (sssp_bin.hip) unless asked to relax directly
   if (binned) return sssp_bin_run(g, ds.as<uint32_t>(), k, weights, dist, delta, flags, st);
   WorkLease<SsspWork> lease(gm->sssp);
-  if (!lease.w || lease.w->k != k) {
+  const bool copies = with_copies(g, nv);
+  if (!lease.w || lease.w->k != k || (copies && !lease.w->cand)) {
     lease.renew();
-    OLV_TRY(lease.w->alloc(nv, k, g->m));
+    OLV_TRY(lease.w->alloc(nv, k, g->m, copies));
   }
   SsspWork *w = lease.w;
   SsspParams p;
@@ -500,7 +547,7 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   p.queue = w->queue;
   p.hubs = w->hubs;
   p.mark = w->mark;
-  p.cand = (flags & OLV_PERSISTENT) ? nullptr : w->cand;
+  p.cand = copies && !(flags & OLV_PERSISTENT) ? w->cand : nullptr;
   p.ctl = w->ctl;
   p.bar = w->bar;
   p.n = g->n;
@@ -534,7 +581,8 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   } else {
     // relax workgroups per CU: the graph's tuning
     const unsigned gr = (unsigned)cu_count() * g->tune.sssp_relax_per_cu;
-    const unsigned gc = sgrid(((size_t)nv + 3) / 4, kSBlock);
+    const bool wide = !p.cand;
+    const unsigned gc = sgrid(((size_t)nv + 3) / 4, (size_t)kSBlock * (wide ? kWideWords : 1));
     // first chunk: the longest of the last few runs on this graph (8 at
     // first; a run of r rounds takes r + 1 launch pairs, and two runs may
     // differ by a round or two); longer runs continue in chunks of 8, 16, ...
@@ -554,7 +602,10 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
           hipLaunchKernelGGL((sssp_relax_kernel<true, false>), dim3(gr), dim3(kSBlock), 0, s, p);
         else
           hipLaunchKernelGGL((sssp_relax_kernel<false, false>), dim3(gr), dim3(kSBlock), 0, s, p);
-        hipLaunchKernelGGL(sssp_compact_kernel, dim3(gc), dim3(kSBlock), 0, s, p);
+        if (wide)
+          hipLaunchKernelGGL(sssp_compact_kernel<kWideWords>, dim3(gc), dim3(kSBlock), 0, s, p);
+        else
+          hipLaunchKernelGGL(sssp_compact_kernel<1>, dim3(gc), dim3(kSBlock), 0, s, p);
       }
       OLV_HIP(hipGetLastError());
       t.stop();  // ahead of the read-back: host latency after the last round is not timed

@@ -607,18 +607,33 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
   return OLV_OK;
 }
 
-// Virtual vertices from which binning beats direct relaxation on graphs
-// without hubs (8 edges a vertex, binned / direct: 250K vertices 995 / 570 us,
-// 1M 985 / 997, 2M 1075 / 1597, 4M 1455 / 2770).
-constexpr uint64_t kBinMinVertices = 1250000;
+// Where binning beats direct relaxation on graphs without hubs: from
+// kBinMinVertices virtual vertices, or from kBinMinSparse where a vertex has at
+// most kBinSparse edges.  In between, the direct rounds have the cheaper edges
+// and the binned ones, whose slices leave CUs idle, the cheaper vertices (us,
+// binned / direct; d: edges a vertex):
+//   vertices  d 2.5      d 4        d 8         d 16
+//   800K      785/774    777/747    902/769    1203/841
+//   1M        755/797    825/845    962/882    1256/942
+//   1.2M      881/913    857/885    940/885    1286/1059
+//   1.5M      824/908    894/920   1006/1012   1391/1202
+//   4.2M                           1640/2200
+//   16.7M                5150/4800 7350/7480  11330/11910
+// Past 16M vertices (two slices per lane of a workgroup) direct is the faster
+// one up to 8 edges a vertex and, beyond, slower by up to a fifth than binning
+// with a launch of its own for the apply step was, which went by queues in
+// memory (17M vertices: d 4 7.5 ms binned, 5.1 direct; d 8 8.65 and 7.4; d 16
+// 11.7 and 12.4; d 24 16.5 and 20.0).
+constexpr uint64_t kBinMinVertices = 1250000, kBinMinSparse = 900000, kBinSparse = 5;
 
 // Whether k instances of g go through the binned rounds: no out-list long
 // enough to be split, slices for most of the chip, and at most 16M vertices
 // and 2^32 pairs.
 bool sssp_bin_fits(const olv_graph *g, uint32_t k) {
   const uint64_t nv = (uint64_t)k * g->n;
-  return g->m && (uint64_t)k * g->m < (1ull << 32) && nv < (1ull << 32) && nv >= kBinMinVertices &&
-         g->max_outdeg < g->tune.hub_thr && g->n <= ((uint64_t)kFParts << 14);
+  if (!g->m || (uint64_t)k * g->m >= (1ull << 32) || nv >= (1ull << 32)) return false;
+  if (g->max_outdeg >= g->tune.hub_thr || g->n > ((uint64_t)kFParts << 14)) return false;
+  return nv >= kBinMinVertices || (nv >= kBinMinSparse && g->m <= kBinSparse * g->n);
 }
 
 // Binned SSSP for k instances (sources d_srcs[0..k), on the device; the
