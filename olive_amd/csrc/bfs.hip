@@ -989,8 +989,7 @@ int bfs_multisource(const olv_graph *g0, const uint32_t *seeds, uint32_t k, bool
   DevBuf d_seeds, d_levels;
   if (k > 1) {
     OLV_TRY(d_seeds.alloc((size_t)k * 4));
-    // (complete on return: launches behind a copy in the stream start 10 us late)
-    OLV_HIP(hipMemcpy(d_seeds.p, h_seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice));
+    OLV_HIP(hipMemcpyAsync(d_seeds.p, h_seeds.data(), (size_t)k * 4, hipMemcpyHostToDevice, stream()));
   }
   int32_t *out = levels;
   if (host) {
