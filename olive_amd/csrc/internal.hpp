@@ -97,7 +97,7 @@ struct olv_graph {
   bool plan_in_ready = false, plan_out_ready = false;
   olv::BfsWork *bfs = nullptr;
   olv::PrWork *pr = nullptr;
-  std::atomic<olv::SsspWork *> sssp{nullptr};   // direct SSSP work (for the last k sources), while no call has it
+  std::atomic<olv::SsspWork *> sssp{nullptr};   // direct SSSP work (for up to its k sources), while no call has it
   std::atomic<olv::MbfsWork *> mbfs{nullptr};   // batched BFS work (for up to its k sources), while no call has it
   olv::SsspBinWork *sssp_bin = nullptr;  // binned SSSP work (for the last k sources)
   // In-degree numbering: vertices by descending in-degree, ties by id

@@ -409,10 +409,12 @@ __global__ void sssp_seed_kernel(const uint32_t *__restrict__ srcs, uint32_t k, 
                 ModRow{p.n}, &deg);
 }
 
-// Work arrays for k instances, kept on the graph for the next call with the
-// same k (allocating them took 0.35 ms of every call).
+// Work arrays for up to k instances, kept on the graph for the next call
+// (allocating them took 0.35 ms of every call).
 struct SsspWork {
   uint32_t k = 0;
+  uint64_t cand_nv = 0;  // virtual vertices that the candidate copies have room for
+  size_t bytes = 0;      // of queue, marks and hub items
   uint32_t *queue = nullptr;
   uint8_t *mark = nullptr;
   int32_t *cand = nullptr;
@@ -425,18 +427,31 @@ struct SsspWork {
       if (p) (void)hipFree(p);
     if (h_ctl) (void)hipHostFree(h_ctl);
   }
-  int alloc(uint64_t nv, uint32_t kk, uint64_t m, bool copies) {
+  int alloc(uint64_t nv, uint32_t kk, uint64_t m) {
     k = kk;
+    const size_t hb = hub_capacity(m) * k * sizeof(uint2);
+    bytes = (size_t)nv * 5 + hb;
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&queue), (size_t)nv * 4));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&mark), ((size_t)nv + 3) / 4 * 4));
-    if (copies) OLV_HIP(hipMalloc(reinterpret_cast<void **>(&cand), (size_t)nv * kCopies * 4));
-    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&hubs), hub_capacity(m) * k * sizeof(uint2)));
+    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&hubs), hb));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&ctl), sizeof(SsspCtl)));
     OLV_HIP(hipMalloc(reinterpret_cast<void **>(&bar), sizeof(GridBar)));
     OLV_HIP(hipHostMalloc(reinterpret_cast<void **>(&h_ctl), sizeof(SsspCtl), hipHostMallocDefault));
     return OLV_OK;
   }
+  int alloc_copies(uint64_t nv) {
+    if (nv <= cand_nv) return OLV_OK;
+    if (cand) (void)hipFree(cand);
+    cand = nullptr;
+    cand_nv = 0;
+    OLV_HIP(hipMalloc(reinterpret_cast<void **>(&cand), (size_t)nv * kCopies * 4));
+    cand_nv = nv;
+    return OLV_OK;
+  }
 };
+// Larger work is freed after the call: its allocation is little beside
+// relaxing that many vertices.
+constexpr size_t kSsspKeepBytes = size_t(4) << 30;
 
 void free_sssp_work(olv_graph *g) { delete g->sssp.exchange(nullptr); }
 
@@ -534,10 +549,11 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   if (binned) return sssp_bin_run(g, ds.as<uint32_t>(), k, weights, dist, delta, flags, st);
   WorkLease<SsspWork> lease(gm->sssp);
   const bool copies = with_copies(g, nv);
-  if (!lease.w || lease.w->k != k || (copies && !lease.w->cand)) {
+  if (!lease.w || lease.w->k < k) {
     lease.renew();
-    OLV_TRY(lease.w->alloc(nv, k, g->m, copies));
+    OLV_TRY(lease.w->alloc(nv, k, g->m));
   }
+  if (copies) OLV_TRY(lease.w->alloc_copies(nv));
   SsspWork *w = lease.w;
   SsspParams p;
   p.row_ptr = g->row_ptr;
@@ -626,7 +642,8 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
     st->edges_inspected = w->h_ctl->relax;
   }
   const bool capped = w->h_ctl->capped != 0;
-  lease.keep();  // the stream is idle: the control block has been read back
+  // (the stream is idle: the control block has been read back)
+  if (w->bytes <= kSsspKeepBytes) lease.keep();
   if (capped) return fail(OLV_ENOCONV, "olv_sssp: still relaxing after n=%u rounds (negative cycle)", g->n);
   return OLV_OK;
 }

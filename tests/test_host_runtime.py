@@ -232,3 +232,31 @@ for i in range(4):
     if i:
         assert 258 <= count("mbfs_compact") <= 258 + 20, (i, count("mbfs_compact"))
 """)
+
+
+def test_sssp_work_kept(run):
+    """Directly relaxed SSSP keeps its work for calls of as many sources or
+    fewer, and only up to 4 GiB (SsspParams: ctl at byte 64)."""
+    run("""
+def done(args):
+    u32(u64(args[0] + 64).value).value = 1
+effects["sssp_compact_kernel"] = done
+def call(g, k, out):
+    srcs = np.zeros(k, np.uint32)
+    rt.rt_fail_at(0)
+    assert lib().olv_sssp_batched(g.h, srcs.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), k, None, out.c,
+                                  _lib.OLV_SSSP_DIRECT, None) == 0, lib().olv_last_error()
+    return rt.rt_allocs()
+g = graph(50_000, 40)
+out = olive_amd.DeviceBuffer(64 * g.n, np.int32)
+for k in (64, 1, 5):   # without candidate copies and with them
+    call(g, k, out)
+for k in (5, 64, 3, 1, 17):
+    assert call(g, k, out) <= 1, (k, rt.rt_allocs())   # the copy of the sources
+g = graph(9_000_000, 40)
+out = olive_amd.DeviceBuffer(100 * g.n, np.int32)
+call(g, 1, out)
+live = rt.rt_live()
+call(g, 100, out)   # 4.5 GB of queue and marks
+assert rt.rt_live() < live + (1 << 20)
+""")
