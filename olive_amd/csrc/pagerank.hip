@@ -985,7 +985,7 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
   OLV_TRY(s);
   float *dl = sl.out(lambda_out, g->n, host, &s);
   OLV_TRY(s);
-  ScratchBuf gb;  // gbar in the new numbering
+  ScratchBuf gb, rb;  // gbar in the new numbering; the ranks, where the gradient overwrites them
   if (relabel) OLV_TRY(gb.alloc(std::max<size_t>(g->n, 1) * 4));
   Timer t;
   t.start();
@@ -1033,6 +1033,12 @@ int olv_pagerank_vjp_f32(const olv_graph *cg, const float *wts, const float *ran
     if (relabel) {  // into the scratch of the renumbered gbar, which is done with
       gather_f32(lf, g->rl_pi, g->n, gb.as<float>());
       lo = gb.as<float>();
+    }
+    const auto at = [](const float *p) { return reinterpret_cast<uintptr_t>(p); };
+    if (at(dgw) < at(dr + g->n) && at(dr) < at(dgw + g->m)) {  // the ranks where the gradient goes
+      OLV_TRY(rb.alloc((size_t)g->n * 4));
+      OLV_HIP(hipMemcpyAsync(rb.p, dr, (size_t)g->n * 4, hipMemcpyDeviceToDevice, stream()));
+      dr = rb.as<float>();
     }
     const bool few = w->full.n != 0;
     hipLaunchKernelGGL(edge_grad_kernel, dim3((unsigned)(((size_t)g->m + kITile - 1) / kITile)), dim3(kIB), 0, stream(),

@@ -172,3 +172,25 @@ def test_autograd_weights_updated_in_place(olv):
             assert torch.equal(gw, w2.grad), step
         with torch.no_grad():
             w.mul_(1.0 + 0.1 * torch.rand_like(w))
+
+
+def test_vjp_gradient_over_the_ranks(olv):
+    """grad_w may be written where the ranks are: the same bits as apart."""
+    import ctypes
+
+    from olive_amd import _lib
+    csr = olv.with_weights_f32_normalized(olv.gen_uniform(800_000, 8_000_000, seed=4), seed=1)
+    g = olv.Graph(csr)
+    B = olv.DeviceBuffer.from_numpy
+    w, gbar = B(csr.weights), B(np.random.default_rng(1).standard_normal(csr.n).astype(np.float32))
+    ranks = np.random.default_rng(2).random(csr.n).astype(np.float32)
+    for flags in (0, _lib.OLV_GRAPH_ORDER):
+        want = g.pagerank_vjp(w, B(ranks), gbar, flags=flags)[0].numpy()
+        for off in (0, 3_000_001):  # entries into the gradient
+            both = np.zeros(csr.m, np.float32)
+            both[off:off + csr.n] = ranks
+            buf = B(both)
+            p = ctypes.c_void_p(buf.c.value + 4 * off)
+            _lib.check(_lib.lib().olv_pagerank_vjp_f32(g.h, w.c, p, gbar.c, 0.85, 1e-6, 1000, buf.c, None, None, flags,
+                                                       None), "vjp")
+            assert np.array_equal(buf.numpy(), want), (flags, off)
