@@ -202,21 +202,27 @@ def test_sssp_negative_weights_without_cycle(olv):
 
 
 def test_sssp_zero_and_large_weights(olv):
-    """Near-far split with zero weights (step 1) and with weights up to 2^20."""
+    """Near-far split with zero weights (step 1) and with weights up to 2^20:
+    relaxed directly, and binned (80 instances, 1.3M virtual vertices)."""
     base = olv.gen_uniform(1 << 14, 1 << 17, seed=4)
+    srcs = sources(base, 80, 3)
     for lo, hi in ((0, 1), (0, 3), (1, 1 << 20)):
         csr = olv.with_weights_i32(base, lo, hi, seed=lo + hi)
         g = olv.Graph(csr, transpose=False)
-        ref = oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, 0)
-        assert np.array_equal(g.sssp(0)[0].numpy(), ref), (lo, hi)
+        ref = {int(s): oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, int(s)) for s in (0, *srcs[[0, 41, 79]])}
+        assert np.array_equal(g.sssp(0)[0].numpy(), ref[0]), (lo, hi)
+        for flags in (0, 0x8, 0x800):
+            got = g.sssp_batched(srcs, flags=flags)[0].numpy().reshape(80, csr.n)
+            for i in (0, 41, 79):
+                assert np.array_equal(got[i], ref[int(srcs[i])]), (lo, hi, flags, i)
 
 
+@pytest.mark.parametrize("k", [1, 1300])  # relaxed directly, and (without 0x800) binned: 1.3M virtual vertices
 @pytest.mark.parametrize("flags", [0, 0x8, 0x800, 0x808])
-def test_sssp_chain_with_one_heavy_edge(olv, flags):
-    """A 1000-vertex chain with unit weights and one weight-1e6 edge: with
-    direct relaxation (0x800) the near-far step (~32k) needs ~31 promotions
-    with nothing to relax, so the run takes more rounds than the chain has
-    vertices; the binned path re-splits past the heavy edge at once."""
+def test_sssp_chain_with_one_heavy_edge(olv, flags, k):
+    """A 1000-vertex chain with unit weights and one weight-1e6 edge: the split
+    moves past the heavy edge at once, not in steps of the near-far distance
+    (32), so a run takes a round per hop and one or two more."""
     n = 1000
     rp = np.arange(n + 1, dtype=np.uint32)
     rp[n] = n - 1
@@ -225,14 +231,24 @@ def test_sssp_chain_with_one_heavy_edge(olv, flags):
     w[500] = 1_000_000
     csr = olv.CsrGraph(rp, col, w)
     g = olv.Graph(csr, transpose=False)
-    out, st = g.sssp(0, flags=flags)
+    out, st = g.sssp_batched(np.zeros(k, np.uint32), flags=flags) if k > 1 else g.sssp(0, flags=flags)
     ref = oracle.dijkstra(rp, col, w, 0)
     assert ref[-1] == n - 2 + 1_000_000
-    assert np.array_equal(out.numpy(), ref)
+    assert np.array_equal(out.numpy().reshape(k, n), np.broadcast_to(ref, (k, n)))
     say(f"  chain: {st.iterations} rounds")
-    if not flags & 0x800:
-        assert st.iterations <= n + 2  # one round per hop, plus one re-split
-    assert st.edges_inspected == n - 1  # every edge relaxed exactly once
+    assert st.iterations <= n + 3
+    assert st.edges_inspected == k * (n - 1)  # every edge relaxed exactly once
+
+
+@pytest.mark.parametrize("n,m,k", [(9973, 5 * 9973, 90), (9973, 5 * 9973, 91),  # 900K vertices, 5 edges each
+                                   (9973, 6 * 9973, 125), (9973, 6 * 9973, 126)])  # 1.25M, more edges
+def test_sssp_both_sides_of_the_bins(olv, n, m, k):
+    csr = olv.with_weights_i32(olv.gen_uniform(n, m, seed=k), 1, 64, seed=k)
+    g = olv.Graph(csr, transpose=False)
+    srcs = sources(csr, k, k)
+    got = g.sssp_batched(srcs)[0].numpy().reshape(k, n)
+    for i in (0, k // 2, k - 1):
+        assert np.array_equal(got[i], oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, int(srcs[i]))), i
 
 
 def test_sssp_negative_cycle_reports_enoconv(olv):
@@ -265,11 +281,12 @@ def sources(csr, k, seed):
     return rng.choice(nz, size=k, replace=k > nz.size).astype(np.uint32)
 
 
-def test_sssp_binned_hubs_and_instances(olv):
-    """Binned relaxation with hub items (RMAT, out-degree >= hub_thr) and k
-    instances whose virtual ranges straddle partitions (n not a multiple of
-    the 8192-vertex slice), against Dijkstra; zero-weight edges included."""
-    say("sssp binned: rmat hubs, 6 instances")
+def test_sssp_hubs_and_instances(olv):
+    """Hub items (RMAT, out-degree >= hub_thr) with k instances, whose virtual
+    ids pass the sizes of the candidate copies and of the bins: a graph with
+    hubs is relaxed directly at any.  Against Dijkstra; zero-weight edges
+    included."""
+    say("sssp: rmat hubs, 6 instances")
     csr = olv.with_weights_i32(olv.gen_rmat(16, 16, seed=5), 0, 9, seed=5)
     assert int(csr.outdeg().max()) >= 1024
     g = olv.Graph(csr, transpose=False)
@@ -280,9 +297,7 @@ def test_sssp_binned_hubs_and_instances(olv):
         assert np.array_equal(got[i], oracle.dijkstra(csr.row_ptr, csr.col, csr.weights, int(s_))), i
     one, _ = g.sssp(int(srcs[3]))
     assert np.array_equal(one.numpy(), got[3])
-    # 260 instances: 17.0M virtual vertices, the expand/apply pair on
-    # 32K-vertex slices
-    say("sssp binned: rmat hubs, 260 instances")
+    say("sssp: rmat hubs, 260 instances")  # 17.0M virtual vertices
     srcs = sources(csr, 260, 12)
     out, st = g.sssp_batched(srcs)
     got = out.numpy().reshape(len(srcs), csr.n)

@@ -49,9 +49,8 @@ from olive_amd._lib import lib
 olive_amd.init()
 
 def graph(n, m, weighted=True, transpose=False):
-    # all edges leave and enter vertex 0; no kernel looks at them here
-    rp = np.full(n + 1, m, np.uint32)
-    rp[0] = 0
+    # edges spread over the vertices, all to vertex 0; no kernel looks at them here
+    rp = (np.arange(n + 1, dtype=np.uint64) * m // n).astype(np.uint32)
     w = np.ones(m, np.int32) if weighted else None
     return olive_amd.Graph(olive_amd.CsrGraph(rp, np.zeros(m, np.uint32), w), transpose=transpose)
 
@@ -259,4 +258,31 @@ call(g, 1, out)
 live = rt.rt_live()
 call(g, 100, out)   # 4.5 GB of queue and marks
 assert rt.rt_live() < live + (1 << 20)
+""")
+
+
+@pytest.mark.parametrize("n,m,k,binned", [
+    (1000, 5000, 899, 0), (1000, 5000, 900, 1), (1000, 5001, 900, 0),  # 900K vertices of at most 5 edges
+    (1000, 6000, 1249, 0), (1000, 6000, 1250, 1),                      # 1.25M of any
+    (1 << 24, 40, 1, 1), ((1 << 24) + 1, 40, 1, 0),                    # 1024 slices of 16K
+    (1000, 6000, 20_000, 2)])                                          # 20M: in groups of as many as fit
+def test_sssp_route(run, n, m, k, binned):
+    """Graphs without hubs that go through the binned rounds."""
+    run(f"n, m, k, binned = {n}, {m}, {k}, {binned}" + """
+groups = []
+def caps(args):   # (k at 3)
+    groups.append(u32(args[3]).value)
+    u32(u64(args[7]).value).value = u32(args[3]).value * m
+def round_(args):
+    u32(u64(args[0] + 80).value).value = 1
+def done(args):
+    u32(u64(args[0] + 64).value).value = 1
+effects.update(ssspf_cap_kernel=caps, ssspf_round_kernel=round_, sssp_compact_kernel=done)
+g = graph(n, m)
+out = olive_amd.DeviceBuffer(k * n, np.int32)
+srcs = np.zeros(k, np.uint32)
+assert lib().olv_sssp_batched(g.h, srcs.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), k, None, out.c, 0, None) == 0
+assert len(groups) == binned and bool(count("ssspf_round")) == bool(binned), groups
+assert bool(count("sssp_relax")) == (not binned)
+assert not groups or sum(groups) == k
 """)
