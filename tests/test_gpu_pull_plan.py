@@ -103,3 +103,33 @@ def test_weighted_against_row_pull(olv, name):
         assert rel(x, y) <= 1e-4
     j0 = g.pagerank_jvp(w, r0, dw, dt, flags=_lib.OLV_PR_ROW_PULL)[0]
     assert rel(g.pagerank_jvp(w, r0, dw, dt)[0], j0) <= 1e-4
+
+
+@pytest.mark.parametrize("name", ["segmented", "single_launch"])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_not_finite_stays_in_its_rows(olv, name, bad):
+    """Weights and teleports that are not finite reach the rows that the per-row
+    pull says and no others, whatever pieces share a task with theirs."""
+    print("pull plan not finite", name, bad, flush=True)
+    n, fill, hub = CASES[name]
+    csr = olv.with_weights_f32_normalized(ladder(olv, n, fill, hub, 4), seed=2)
+    rng = np.random.default_rng(8)
+    w, t = csr.weights.copy(), olv.gen_dirichlet(n, 7)
+    w[rng.integers(0, csr.m, 12)] = bad
+    t[rng.integers(0, n, 3)] = bad
+    g = olv.Graph(csr)
+    B = olv.DeviceBuffer.from_numpy
+    dw, dt = B(w), B(t)
+    for iters in (1, 2):
+        out = []
+        for flags in (0, _lib.OLV_PR_ROW_PULL):
+            r = olv.DeviceBuffer(n, np.float32)
+            rc = _lib.lib().olv_pagerank_weighted_f32(g.h, dw.c, dt.c, 0.85, 1e-6, iters, r.c, flags, None)
+            assert rc == _lib.OLV_ENOCONV
+            out.append(r.numpy())
+        a, b = out
+        assert np.array_equal(np.isnan(a), np.isnan(b)) and not np.isfinite(a).all()
+        fin = np.isfinite(b)
+        assert fin.sum() > n // 4  # the rows that nothing of it reaches
+        assert np.array_equal(a[~fin], b[~fin], equal_nan=True)
+        assert np.linalg.norm(a[fin].astype(np.float64) - b[fin]) <= 1e-5 * np.linalg.norm(b[fin].astype(np.float64))

@@ -59,3 +59,16 @@ def test_frontiers_larger_than_a_workgroup_holds(olv):
     g = olv.Graph(csr, transpose=False)
     for s in (0, int(src[-1])):
         assert np.array_equal(g.sssp(s)[0].numpy(), oracle.bfs(rp, csr.col, s)), s
+
+
+def test_more_vertices_than_the_bins_take(olv):
+    n, m = (1 << 24) + 5, 1 << 25
+    rng = np.random.default_rng(9)
+    src = np.sort(rng.integers(0, n, m, dtype=np.int64))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(src, minlength=n))]).astype(np.uint32)
+    csr = olv.CsrGraph(rp, rng.integers(0, n, m).astype(np.uint32), np.ones(m, np.int32))
+    print("sssp rounds, 2^24 + 5 vertices", flush=True)
+    s = int(src[m // 2])
+    ref = oracle.bfs(rp, csr.col, s)
+    assert (ref < 0x7FFFFFFF).sum() > n // 2
+    assert np.array_equal(olv.Graph(csr, transpose=False).sssp(s)[0].numpy(), ref)
