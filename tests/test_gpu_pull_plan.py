@@ -58,6 +58,7 @@ CASES = {
     "segmented": (100003, 600000, 50000),
     "one_segment": (32768, 520000, 20000),
     "segment_plus_one": (32769, 520000, 20000),
+    "segment_plus_six": (32774, 520000, 20000),
     "single_launch": (100003, 300000, 16384),
     "few_edges_long_row": (100003, 1000, 70000),
     # lanes with four short rows and more: groups of them of at most two, at
