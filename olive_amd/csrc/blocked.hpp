@@ -71,10 +71,13 @@ static_assert(kPieceMax == kTask, "the longest piece fills one task");
 template <bool kW>
 constexpr int kBlkRing = kW ? 2 : 4;
 constexpr uint32_t kSegMinEntries = 2048;      // entries of a staged segment, at least
-// Edges of a CSR with a segment pass, at least: one launch of m random
-// gathers (4.5 us + m / 180 G/s) against two launches (about 8.6 us on 1 M
-// edges, where the single launch takes 10.8; on 65 K edges it takes 5.5).
-constexpr uint32_t kPassMinEntries = 500000;
+// Edges of a CSR with a segment pass, at least: one launch of m random gathers
+// against two launches.  20 iterations, one launch / two (us), uniform edges at
+// 6, 16, 32 a vertex, then RMAT: 500K edges 197/232, 197/220, 180/218 and
+// 200/231, 220/228, 215/227; 850K 228/247, 231/228, 192/228 and 219/238,
+// 242/228, 251/240; 1.2M 268/279, 252/242, 214/241 and 256/256, 267/243,
+// 268/242.  Weighted solves cross at the same sizes.
+constexpr uint32_t kPassMinEntries = 700000;
 constexpr uint32_t kDirectRowMax = 16384;      // without a segment pass: entries per row, at most
 constexpr uint32_t kIsPartial = 0x80000000u;   // combine term: a partial's index, else a source
 constexpr uint32_t kEidZero = 0xffffffffu;     // weight source of a padding entry: 0
