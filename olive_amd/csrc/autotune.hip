@@ -507,8 +507,8 @@ int olv_autotune_ex(olv_graph *g, unsigned what, const char *cache_path, olv_tun
                       {}, [&](double *ms) { return S.time_pull(ms); }));
   }
   if ((what & OLV_TUNE_SSSP) && g->wdtype == OLV_W_I32) {
-    // the step on the default (binned) path; the grid on the direct path,
-    // the only one it shapes
+    // the step on the path that the graph's calls take (binned or direct); the
+    // grid on the direct path, the only one it shapes
     double warm;
     OLV_TRY(S.time_sssp(&warm, 0u));
     OLV_TRY(S.descend({{&T.sssp_delta_num, {16, 24, 32, 48, 64}}}, {},

@@ -487,9 +487,10 @@ __device__ __forceinline__ WordLoad load_word(const BfsArgs &a, uint32_t w) {
 }
 
 // Next frontier = visited bytes set since the last extraction, those that say
-// "expanded already" (bit 1, bfs_narrow_kernel) excepted: written to `front` (for a bottom-up step) and, if `to_queue`, compacted into the
-// queue and hub items (for a top-down step); `snap` catches up.  `pre` is
-// this lane's first word (index vb * BLOCK + threadIdx.x), already loaded.
+// "expanded already" (bit 1, bfs_narrow_kernel) excepted: written to `front`
+// (for a bottom-up step) and, if `to_queue`, compacted into the queue and hub
+// items (for a top-down step); `snap` catches up.  `pre` is this lane's first
+// word (index vb * BLOCK + threadIdx.x), already loaded.
 template <int BLOCK>
 __device__ void frontier_words(const BfsArgs &a, uint32_t *front, uint32_t nw, bool to_queue, uint32_t *qcount,
                                uint32_t *hcount, uint32_t vb, uint32_t nvb, const WordLoad &pre) {

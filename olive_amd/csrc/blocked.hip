@@ -371,7 +371,7 @@ int build_segmented(const uint32_t *rp, const uint32_t *col, const uint32_t *eid
   bp.ntasks = (uint32_t)task;
   bp.nparts = (uint32_t)part;
   // Tasks to workgroups: consecutive runs of about equal cost, a task
-  // kTaskCost (classes of short pieces store more) and a segment's slice
+  // task_cost (classes of short pieces store more) and a segment's slice
   // kSliceCost (its 128 KB load between two barriers, and the ring's restart).
   std::vector<uint4> first, items;
   {

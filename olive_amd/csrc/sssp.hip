@@ -8,23 +8,23 @@
 // (negative-cycle guard, SSSP.cu:153-157).  Shortest distances are unique,
 // so relaxing straight into dist with atomicMin -- no accumulator array, no
 // per-round O(V) reset -- reaches the same fixed point: a vertex whose
-// distance dropped this round is marked in a bitmap and expanded next round.
+// distance dropped this round is marked and expanded next round.
 //
 // Near-far ordering (Davidson et al., IPDPS'14): with a split distance T, an
 // improved vertex joins the next round's frontier only if its new distance
 // is below T; otherwise it stays marked.  When the near frontier runs dry, T
-// moves to the smallest marked distance + delta (never an empty promotion)
-// and the marked vertices below it form the next frontier.  Vertices are then
-// mostly expanded once with their final distance instead of once per
-// improvement, and the fixed point -- hence every distance -- is the same.
+// moves to the smallest marked distance + delta and the marked vertices below
+// it form the next frontier.  Vertices are then mostly expanded once with
+// their final distance instead of once per improvement, and the fixed point --
+// hence every distance -- is the same.
 // Negative weights turn the ordering off (plain rounds, so the reference's
 // n-round negative-cycle rule applies unchanged).
 //
 // A vertex whose distance dropped is marked with a plain byte store: the
 // bitmap atomics that marked it before cost as much as the distance atomics
 // and serialised on the words of an RMAT graph's hubs, and extracting a
-// frontier from them took a lane per 32 vertices (16-28 us per large round;
-// 5-7 from the bytes).
+// frontier from them took a lane per 32 vertices (RMAT 250K x 4M: 16-28 us per
+// large round; 5-7 from the bytes).
 //
 // k sources run as k instances over one shared CSR: instance s owns virtual
 // vertices s*n .. s*n+n-1 (dist row s), so one launch per round relaxes all
@@ -71,7 +71,7 @@ static bool with_copies(const olv_graph *g, uint64_t nv) {
   return nv <= (g->max_outdeg >= g->tune.hub_thr ? kCopiesHubs : kCopiesNoHubs);
 }
 
-template <bool Multi, bool Copies>
+template <bool Multi>
 struct SsspVisitor {
   using P = typename std::conditional<Multi, unsigned long long, int32_t>::type;
   const uint32_t *col;
@@ -169,8 +169,7 @@ struct ModRow {
 template <bool Multi, bool Copies>
 __device__ __forceinline__ void sssp_round(const SsspParams &p, uint32_t qsize, uint32_t nhubs, uint32_t vb,
                                            uint32_t nvb, unsigned long long &insp) {
-  SsspVisitor<Multi, Copies> vis(p.col, p.w, p.dist, Copies ? p.cand + (size_t)(vb % kCopies) * p.nv : p.dist, p.mark,
-                               p.n);
+  SsspVisitor<Multi> vis(p.col, p.w, p.dist, Copies ? p.cand + (size_t)(vb % kCopies) * p.nv : p.dist, p.mark, p.n);
   push_expand<kSBlock>(p.queue, qsize, p.hubs, nhubs, p.row_ptr, p.wave_thr, p.block_thr, p.hub_thr, vb, nvb, vis,
                        insp);
 }
@@ -364,8 +363,8 @@ __global__ void __launch_bounds__(kSBlock) sssp_persistent_kernel(SsspParams p) 
     }
     sssp_round<Multi, false>(p, qsize, nhubs, vb, nvb, insp);
     if (!grid_barrier(p.bar, gb, kSSpin)) break;
-    sssp_take<kSBlock, 1>(p, kInf, true, &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1], &ctl->minfar[0][vb % kCtrSlots].v, vb,
-                       nvb);
+    sssp_take<kSBlock, 1>(p, kInf, true, &ctl->qfill[(R + 1) & 1], &ctl->hfill[(R + 1) & 1],
+                          &ctl->minfar[0][vb % kCtrSlots].v, vb, nvb);
     if (!grid_barrier(p.bar, gb, kSSpin)) break;
   }
   __shared__ unsigned long long s_red[kSBlock / kWave];
@@ -578,7 +577,8 @@ static int sssp_run(const olv_graph *g, const uint32_t *srcs, uint32_t k, const 
   p.max_rounds = delta ? (uint32_t)std::min<uint64_t>(4ull * g->n + 1024, 0xffffffffull) : g->n;
   Timer t;
   t.start();
-  hipLaunchKernelGGL(sssp_reset_kernel, dim3(sgrid((size_t)nv * (p.cand ? kCopies : 1u), 256)), dim3(256), 0, s, p, srcs[0]);
+  hipLaunchKernelGGL(sssp_reset_kernel, dim3(sgrid((size_t)nv * (p.cand ? kCopies : 1u), 256)), dim3(256), 0, s, p,
+                     srcs[0]);
   if (multi) hipLaunchKernelGGL(sssp_seed_kernel, dim3(1), dim3(256), 0, s, ds.as<uint32_t>(), k, p);
   OLV_HIP(hipGetLastError());
   if (flags & OLV_PERSISTENT) {

@@ -62,7 +62,8 @@ __device__ __forceinline__ int32_t add_clamp(int32_t t, int32_t d) { return t > 
 // CU) up to 16M virtual vertices.  (2^13-vertex slices fit two workgroups per
 // CU by LDS, but the second ones started up to 120 us late on MI355X and a
 // 4M-vertex run took 1.78 ms against 1.30 ms.)
-constexpr uint32_t kFParts = 1024;               // partitions at most (16M virtual vertices)
+constexpr uint32_t kFSb = 14, kFS = 1u << kFSb;  // vertices of a slice
+constexpr uint32_t kFParts = 1024;               // slices at most (16M virtual vertices)
 constexpr int kFB = 1024;                        // workgroup
 
 struct alignas(128) FusedSlot {
@@ -113,9 +114,7 @@ __device__ __forceinline__ uint32_t fused_scan(uint32_t v, uint32_t *wt, uint32_
   return before + inc - v;
 }
 
-template <uint32_t kFSb>
 __global__ void __launch_bounds__(kFB) ssspf_round_kernel(FusedArgs a, uint32_t R) {
-  constexpr uint32_t kFS = 1u << kFSb;
   constexpr uint32_t kFV = kFS / kFB;  // consecutive vertices per lane
   FusedCtl *ctl = a.ctl;
   const uint32_t t = threadIdx.x, lane = lane_id();
@@ -427,17 +426,17 @@ __global__ void __launch_bounds__(kFB) ssspf_round_kernel(FusedArgs a, uint32_t 
 // Edges from slice p to slice q (virtual): cap[q * nparts + p]; one
 // workgroup per source slice.
 __global__ void ssspf_cap_kernel(const uint32_t *rp, const uint32_t *col, uint32_t n, uint32_t k, uint32_t nv,
-                                 uint32_t nparts, uint32_t sb, uint32_t *cap) {
+                                 uint32_t nparts, uint32_t *cap) {
   __shared__ uint32_t s_h[kFParts];
   const uint32_t p = blockIdx.x;
   for (uint32_t i = threadIdx.x; i < nparts; i += blockDim.x) s_h[i] = 0;
   __syncthreads();
-  const uint32_t x0 = p << sb, x1 = min(nv, x0 + (1u << sb));
+  const uint32_t x0 = p << kFSb, x1 = min(nv, x0 + kFS);
   // one wave per source vertex
   const uint32_t lane = lane_id(), wv = threadIdx.x / kWave, nwv = blockDim.x / kWave;
   for (uint32_t x = x0 + wv; x < x1; x += nwv) {
     const uint32_t row = k > 1 ? x % n : x, xb = x - row;
-    for (uint32_t e = rp[row] + lane; e < rp[row + 1]; e += kWave) atomicAdd(&s_h[(xb + col[e]) >> sb], 1u);
+    for (uint32_t e = rp[row] + lane; e < rp[row + 1]; e += kWave) atomicAdd(&s_h[(xb + col[e]) >> kFSb], 1u);
   }
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < nparts; i += blockDim.x)
@@ -467,7 +466,7 @@ __global__ void ssspf_seed_kernel(const uint32_t *srcs, FusedArgs a) {
 
 // --------------------------------------------------------------------- host
 struct SsspBinWork {
-  uint32_t k = 0, sb = 0, nparts = 0, nw = 0, nwp = 0;
+  uint32_t k = 0, nparts = 0, nw = 0, nwp = 0;
   uint64_t nv = 0;
   uint32_t *dirty = nullptr;
   uint2 *pairs[2] = {nullptr, nullptr};
@@ -495,17 +494,16 @@ static unsigned bgrid(size_t items, size_t per) {
 // slices), their offsets, two pair stores and two count matrices.  Published to
 // the graph only once the offsets are on the device: the rounds store pairs by
 // them.
-static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) {
-  if (g->sssp_bin && g->sssp_bin->k == k && g->sssp_bin->sb == sb) {
+static int fused_work(olv_graph *g, uint32_t k, SsspBinWork **out) {
+  if (g->sssp_bin && g->sssp_bin->k == k) {
     *out = g->sssp_bin;
     return OLV_OK;
   }
   free_sssp_bin(g);
   std::unique_ptr<SsspBinWork> w(new SsspBinWork());
   w->k = k;
-  w->sb = sb;
   w->nv = (uint64_t)k * g->n;
-  w->nparts = (uint32_t)((w->nv + (1u << sb) - 1) >> sb);
+  w->nparts = (uint32_t)((w->nv + kFS - 1) >> kFSb);
   w->nw = (uint32_t)((w->nv + 31) / 32);
   w->nwp = (w->nw + 63) / 64 * 64;
   const size_t P2 = (size_t)w->nparts * w->nparts;
@@ -523,7 +521,7 @@ static int fused_work(olv_graph *g, uint32_t k, uint32_t sb, SsspBinWork **out) 
   OLV_TRY(cap.alloc(P2 * 4));
   OLV_HIP(hipMemsetAsync(cap.p, 0, P2 * 4, stream()));
   hipLaunchKernelGGL(ssspf_cap_kernel, dim3(w->nparts), dim3(1024), 0, stream(), g->row_ptr, g->col, g->n, k,
-                     (uint32_t)w->nv, w->nparts, sb, cap.as<uint32_t>());
+                     (uint32_t)w->nv, w->nparts, cap.as<uint32_t>());
   OLV_HIP(hipGetLastError());
   std::vector<uint32_t> hc(P2), hb(P2 + 1);
   OLV_HIP(hipMemcpyAsync(hc.data(), cap.p, P2 * 4, hipMemcpyDeviceToHost, stream()));
@@ -546,10 +544,7 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
                      int32_t delta, unsigned flags, olv_stats *st) {
   olv_graph *gm = const_cast<olv_graph *>(g);
   SsspBinWork *w = nullptr;
-  const uint64_t nv = (uint64_t)k * g->n;
-  const uint32_t sb = 14;
-  (void)nv;
-  OLV_TRY(fused_work(gm, k, sb, &w));
+  OLV_TRY(fused_work(gm, k, &w));
   FusedArgs a;
   a.row_ptr = g->row_ptr;
   a.col = g->col;
@@ -583,7 +578,7 @@ static int fused_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, con
   uint64_t enq = 0;
   for (;;) {
     for (uint32_t i = 0; i < chunk; ++i)
-      hipLaunchKernelGGL(ssspf_round_kernel<14>, dim3(w->nparts), dim3(kFB), 0, s, a, (uint32_t)(enq + i));
+      hipLaunchKernelGGL(ssspf_round_kernel, dim3(w->nparts), dim3(kFB), 0, s, a, (uint32_t)(enq + i));
     OLV_HIP(hipGetLastError());
     t.stop();
     enq += chunk;
@@ -632,7 +627,7 @@ constexpr uint64_t kBinMinVertices = 1250000, kBinMinSparse = 900000, kBinSparse
 bool sssp_bin_fits(const olv_graph *g, uint32_t k) {
   const uint64_t nv = (uint64_t)k * g->n;
   if (!g->m || (uint64_t)k * g->m >= (1ull << 32) || nv >= (1ull << 32)) return false;
-  if (g->max_outdeg >= g->tune.hub_thr || g->n > ((uint64_t)kFParts << 14)) return false;
+  if (g->max_outdeg >= g->tune.hub_thr || g->n > ((uint64_t)kFParts << kFSb)) return false;
   return nv >= kBinMinVertices || (nv >= kBinMinSparse && g->m <= kBinSparse * g->n);
 }
 
@@ -641,7 +636,7 @@ bool sssp_bin_fits(const olv_graph *g, uint32_t k) {
 // vertices run in groups of as many as fit.
 int sssp_bin_run(const olv_graph *g, const uint32_t *d_srcs, uint32_t k, const int32_t *weights, int32_t *dist,
                  int32_t delta, unsigned flags, olv_stats *st) {
-  const uint32_t gk = (uint32_t)std::min<uint64_t>(k, ((uint64_t)kFParts << 14) / g->n);
+  const uint32_t gk = (uint32_t)std::min<uint64_t>(k, ((uint64_t)kFParts << kFSb) / g->n);
   if (gk == k) return fused_run(g, d_srcs, k, weights, dist, delta, flags, st);
   olv_stats tot;
   std::memset(&tot, 0, sizeof(tot));
