@@ -339,6 +339,7 @@ __device__ __forceinline__ void mbfs_pull_finish8(const MbfsParams &p, bool vali
 }
 
 constexpr uint32_t kCoopRows = 1u << 16;  // one-lane rows from which a wave records them together
+constexpr int kCoopLanes = 16;            // and rows of the wave with something to record
 
 // Pull level: every vertex not yet holding every source ORs the frontier
 // masks of its active in-neighbours, with 1, 8, 64 or 256 lanes per vertex by
@@ -408,6 +409,7 @@ __global__ void __launch_bounds__(kMB) mbfs_pull_kernel(MbfsParams p, SegDev d) 
       const bool ok = idx < d.off[1];
       const uint32_t v = ok ? d.list[idx] : 0u;
       const bool todo = ok && !bm_test(p.D, v);
+      bool got = false;  // a source that v does not hold yet
       if (todo) {
         uint32_t vv[kMW];
 #pragma unroll
@@ -434,15 +436,20 @@ __global__ void __launch_bounds__(kMB) mbfs_pull_kernel(MbfsParams p, SegDev d) 
           if (full) break;
         }
         insp += k;
+#pragma unroll
+        for (int j = 0; j < kMW; ++j) got = got || (acc[j] & ~vv[j]);
       }
       // The wave goes through its vertices' state eight vertices at a time
       // (word j of vertex 8 r + q to lane 8 q + j): whole lines, but eight
-      // rounds one after another, which only a chip full of waves hides.  By
-      // lanes and so: 256 sources on RMAT-20 1.50 and 1.36 ms, 64 sources 0.88
-      // and 0.84, 256 on 2^18 vertices with 2^20 uniform edges 1.12 and 0.91;
-      // on a 200 x 150 grid, 64 sources, 6.8 and 7.9 ms.
-      if (p.sstride < 64 || d.off[1] - d.off[0] < kCoopRows) {
-        if (todo) mbfs_pull_finish(p, v, acc, An, Fn, nlevel, nf, mf);
+      // rounds one after another, which only a chip full of waves hides and
+      // only a wave with much to record repays.  By lanes and so: 256 sources
+      // on RMAT-20 1.50 and 1.36 ms, 64 sources 0.88 and 0.84, 256 on 2^18
+      // vertices with 2^20 uniform edges 1.12 and 0.91; levels of small
+      // frontiers, 40 sources on a 1000 x 1000 grid, 77 and 85 (8 to 48 rows:
+      // 78).
+      const uint64_t gots = ballot(got);
+      if (p.sstride < 64 || d.off[1] - d.off[0] < kCoopRows || __popcll(gots) < kCoopLanes) {
+        if (got) mbfs_pull_finish(p, v, acc, An, Fn, nlevel, nf, mf);
         continue;
       }
       const uint32_t lane = lane_id(), w0 = threadIdx.x - lane;
@@ -451,11 +458,10 @@ __global__ void __launch_bounds__(kMB) mbfs_pull_kernel(MbfsParams p, SegDev d) 
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      const uint64_t todos = ballot(todo);
       for (uint32_t r = 0; r < 8; ++r) {
-        if (!((todos >> (8 * r)) & 0xffu)) continue;
+        if (!((gots >> (8 * r)) & 0xffu)) continue;
         const uint32_t from = 8 * r + lane / 8;
-        mbfs_pull_finish8(p, (todos >> from) & 1u, __shfl(v, (int)from, kWave), s_acc[w0 + from][lane & 7u], An, Fn,
+        mbfs_pull_finish8(p, (gots >> from) & 1u, __shfl(v, (int)from, kWave), s_acc[w0 + from][lane & 7u], An, Fn,
                           nlevel, nf, mf);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
