@@ -363,7 +363,9 @@ __global__ void __launch_bounds__(kBlkThreads) blk_segment_kernel(BlkDev d, cons
 // both ping-pong buffers, later iterations skip them.
 // kSolo: there is no segment pass, so this launch applies the stop rule
 // (every workgroup reads the residual of iteration k - 1).
-template <class Fin, bool kW, bool kSolo>
+// kMany: a lane has four rows and more (a kernel of its own: with their code in
+// it a weighted forward on RMAT-20 took 1.142 ms, without 1.132).
+template <class Fin, bool kW, bool kSolo, bool kMany>
 __global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, const float *__restrict__ src,
                                                           IterCtl *ctl, uint32_t k, uint32_t huge_blocks,
                                                           uint32_t big_blocks, uint32_t mid_blocks) {
@@ -510,19 +512,21 @@ __global__ void __launch_bounds__(256) blk_combine_kernel(BlkDev d, Fin fin, con
     using R2 = std::integral_constant<uint32_t, 2>;
     using R4 = std::integral_constant<uint32_t, 4>;
     uint32_t v = blk * 256 + threadIdx.x;
-    for (; nv > 3 * step && v < nv - 3 * step; v += 4 * step) {
-      uint32_t a[4], b[4], most = 0;
+    if constexpr (kMany) {
+      for (; nv > 3 * step && v < nv - 3 * step; v += 4 * step) {
+        uint32_t a[4], b[4], most = 0;
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) a[i] = d.cmb_rp[v + i * step], b[i] = d.cmb_rp[v + i * step + 1];
+        for (uint32_t i = 0; i < 4; ++i) a[i] = d.cmb_rp[v + i * step], b[i] = d.cmb_rp[v + i * step + 1];
 #pragma unroll
-      for (uint32_t i = 0; i < 4; ++i) most = max(most, b[i] - a[i]);
-      if (!ballot(most > 2)) {
-        rows(R4{}, R2{}, v, a, b);
-      } else if (!ballot(most > 4)) {
-        rows(R2{}, R4{}, v, a, b);
-        rows(R2{}, R4{}, v + 2 * step, a + 2, b + 2);
-      } else {
-        for (uint32_t i = 0; i < 4; ++i) one(v + i * step);
+        for (uint32_t i = 0; i < 4; ++i) most = max(most, b[i] - a[i]);
+        if (!ballot(most > 2)) {
+          rows(R4{}, R2{}, v, a, b);
+        } else if (!ballot(most > 4)) {
+          rows(R2{}, R4{}, v, a, b);
+          rows(R2{}, R4{}, v + 2 * step, a + 2, b + 2);
+        } else {
+          for (uint32_t i = 0; i < 4; ++i) one(v + i * step);
+        }
       }
     }
     for (; v < nv; v += step) one(v);

@@ -608,16 +608,18 @@ static int enqueue_blocked(const BlockedPlan &bp, const float *weights, const fl
   const unsigned gh = std::min<unsigned>(bp.n_huge, cu * 4);
   const unsigned gb = std::min<unsigned>((bp.n_big + 3) / 4, cu * 8);
   const unsigned gm = std::min<unsigned>((bp.n_mid + 256 / kCmbMidLanes - 1) / (256 / kCmbMidLanes), cu * 16);
-  const dim3 gc(gh + gb + gm + ew_grid(bp.n));
+  const unsigned gl = ew_grid(bp.n);
+  const dim3 gc(gh + gb + gm + gl);
+  const bool many = bp.n > (size_t)gl * 256 * 3;
   hipEvent_t a = prof ? prof->next() : nullptr, b = prof ? prof->next() : nullptr;
   if (a) OLV_HIP(hipEventRecord(a, stream()));
   if (bp.ngroups) {
     hipLaunchKernelGGL(blk_segment_kernel<kW>, dim3(bp.ngroups), dim3(kBlkThreads), 0, stream(), bd, src, w->ctl, k);
-    hipLaunchKernelGGL((blk_combine_kernel<Fin, kW, false>), gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh,
-                       gb, gm);
+    auto *combine = many ? blk_combine_kernel<Fin, kW, false, true> : blk_combine_kernel<Fin, kW, false, false>;
+    hipLaunchKernelGGL(combine, gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh, gb, gm);
   } else {
-    hipLaunchKernelGGL((blk_combine_kernel<Fin, kW, true>), gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh, gb,
-                       gm);
+    auto *combine = many ? blk_combine_kernel<Fin, kW, true, true> : blk_combine_kernel<Fin, kW, true, false>;
+    hipLaunchKernelGGL(combine, gc, dim3(256), 0, stream(), bd, fin, src, w->ctl, k, gh, gb, gm);
   }
   if (b) OLV_HIP(hipEventRecord(b, stream()));
   OLV_HIP(hipGetLastError());
