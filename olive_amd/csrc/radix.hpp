@@ -95,17 +95,18 @@ __device__ __forceinline__ uint32_t tile_rows(const uint32_t *__restrict__ rp, u
     __syncthreads();
     return first;
   }
-  for (uint32_t q = first + 1 + t; q <= last; q += kIWalk * kIB) {
+  const uint32_t span = last - first;  // counted from `first`: ids of rows reach 2^32 - 2
+  for (uint32_t q = 1 + t; q <= span; q += kIWalk * kIB) {
     uint32_t at[kIWalk], end[kIWalk];
 #pragma unroll
     for (uint32_t i = 0; i < kIWalk; ++i) {
-      const uint32_t r = min(q + i * kIB, last);
+      const uint32_t r = first + min(q + i * kIB, span);
       at[i] = rp[r];
-      end[i] = rp[r + 1];
+      end[i] = rp[(size_t)r + 1];
     }
 #pragma unroll
     for (uint32_t i = 0; i < kIWalk; ++i)
-      if (end[i] > at[i] && q + i * kIB <= last) s_row[at[i] - base] = q + i * kIB - first;
+      if (end[i] > at[i] && q + i * kIB <= span) s_row[at[i] - base] = q + i * kIB;
   }
   __syncthreads();
   uint32_t v[kIItems], run = 0;
