@@ -83,7 +83,7 @@ def run(tmp_path_factory):
 BINNED = """
 n, m = 1_300_000, 40
 def caps(args):   # ssspf_cap_kernel: all edges go from the first slice to itself
-    u32(u64(args[7]).value).value = u32(args[3]).value * m
+    u32(u64(args[6]).value).value = u32(args[3]).value * m
 bases = []
 def round_(args):
     a = args[0]
@@ -272,7 +272,7 @@ def test_sssp_route(run, n, m, k, binned):
 groups = []
 def caps(args):   # (k at 3)
     groups.append(u32(args[3]).value)
-    u32(u64(args[7]).value).value = u32(args[3]).value * m
+    u32(u64(args[6]).value).value = u32(args[3]).value * m
 def round_(args):
     u32(u64(args[0] + 80).value).value = 1
 def done(args):
