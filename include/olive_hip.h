@@ -76,11 +76,14 @@ enum {
                                         device-scope atomics per edge instead of
                                         binning the candidates by destination
                                         partition, also where the bins would be
-                                        used: from 1.25 M virtual vertices up,
-                                        on graphs without hubs (the direct
-                                        rounds also run what the bins cannot:
-                                        more than 2^25 virtual vertices or 2^32
-                                        bin entries) */
+                                        used: from 1.25 M virtual vertices up
+                                        (900 K where a vertex has at most five
+                                        edges), on graphs without hubs.  The
+                                        direct rounds also run what the bins
+                                        cannot: graphs of more than 2^24
+                                        vertices, 2^32 bin entries; a batch of
+                                        more than 2^24 virtual vertices is
+                                        binned in groups of sources */
 
 /* weight dtypes for olv_graph_create */
 enum { OLV_W_NONE = 0, OLV_W_I32 = 1, OLV_W_F32 = 2 };
@@ -281,7 +284,8 @@ int olv_bfs_noalloc(const olv_graph *g, uint32_t src, int32_t *levels,
  * bin their candidates by destination partition and min-reduce them in LDS,
  * the others relax with atomics (OLV_SSSP_DIRECT: all do).  The first binned
  * call on a graph keeps its bins (k x m pairs of 8 bytes) on the graph until
- * olv_graph_destroy, a direct call its queue, marks and candidate copies. */
+ * olv_graph_destroy, a direct call its queue, marks and candidate copies (up to
+ * 4 GiB; larger ones are freed when the call ends). */
 int olv_sssp(const olv_graph *g, uint32_t src, const int32_t *weights,
              int32_t *dist, unsigned flags, olv_stats *st);
 

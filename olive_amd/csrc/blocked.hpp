@@ -42,7 +42,7 @@
 // imbalance -- and the combine 9.7 us, 4 of them its launch and the others
 // its gathered partials; 24.5 us per iteration against 32.4 when every unit
 // of entries was staged in LDS with 16K-source slices.  Weighted, the pass
-// reads 110 MB in 22 us (28 before) at the rate of the caches behind L2.
+// reads 118 MB in 22.5 us (28 before), 5.2 TB/s: the rate of the caches behind L2.
 //
 // A piece's terms are summed in a fixed order and the terms of a row in
 // segment order, so an iteration is bit-reproducible from run to run.

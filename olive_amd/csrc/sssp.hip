@@ -179,11 +179,12 @@ __device__ __forceinline__ void sssp_round(const SsspParams &p, uint32_t qsize, 
 // split has not moved (`all` false) vertices marked far stay so, and only those
 // lowered since are looked at.  A lane takes W consecutive words of four mark
 // bytes.  W = 1 with candidate copies, where a vertex costs five loads and lanes
-// are few; else W = kWideWords, and a workgroup collects its vertices in LDS: its place in the queue comes from an atomic, and one for every 1024
-// vertices, 12 ns each after another, made a compaction of 16.7M vertices 195
-// us whatever it found (85 to 110 with W = 4, 25 to 50 collected and without the
-// far ones).  Relaxed directly, 16.7M vertices with 67M edges 8.4 -> 4.8 ms a
-// call, 5M with 40M 3.33 -> 2.46.
+// are few; else W = kWideWords, and a workgroup collects its vertices in LDS:
+// its place in the queue comes from an atomic, and one for every 1024 vertices,
+// 12 ns each after another, made a compaction of 16.7M vertices 195 us whatever
+// it found (85 to 110 with W = 4, 25 to 50 collected and without the far ones).
+// Relaxed directly, 16.7M vertices with 67M edges 8.4 -> 4.8 ms a call, 5M with
+// 40M 3.33 -> 2.46.
 template <int BLOCK, uint32_t W>
 __device__ void sssp_take(const SsspParams &p, int32_t split, bool all, uint32_t *qcount, uint32_t *hcount,
                           int32_t *minfar, uint32_t vb, uint32_t nvb) {

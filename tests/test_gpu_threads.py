@@ -1,4 +1,6 @@
-"""Calls from several threads on one graph: each has work buffers of its own."""
+"""Buffers that a graph lends to its calls: two calls in flight at once, as from
+several threads on a graph whose plans are already built, never hold the same ones.
+Building those plans is left to one thread."""
 import threading
 
 import numpy as np
